@@ -56,9 +56,13 @@ __global__ void k_contract_keys(const uint32_t *__restrict__ sk, int S, int K, i
     if (val < -(int64_t)(q / 2)) val += q;
     if (j < K) kd[((size_t)s * S + v) * K + j] = (double)val;
     unsigned int a = (unsigned int)(val < 0 ? -val : val);
-    // wave-level max then one atomic per wave
+    // wave-level max, then an atomic only where the wave's maximum beats the
+    // value read before it (a stale read is at most too small): with one
+    // atomic per wave the 400,000 waves of 2,000 keys queued on three
+    // addresses and the kernel took 4.63 ms instead of 0.23 ms
     for (int d = 32; d >= 1; d >>= 1) a = max(a, (unsigned int)__shfl_xor((int)a, d, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(maxabs + s, a);
+    if ((threadIdx.x & 63) == 0 && a > __hip_atomic_load(maxabs + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(maxabs + s, a);
 }
 
 
