@@ -10,9 +10,8 @@
 //   1. candidates: every chunk of a speculative window, in parallel: AES (LDS
 //      T-tables), uniform/CDT/Bernoulli per candidate, wave ballot -> per-chunk
 //      accept count and the accepted values compacted in order;
-//   2. walk: one wave per stream turns counts into call boundaries with
-//      1024-chunk windows and a wave prefix scan, and labels every chunk with
-//      (call, first output position);
+//   2. walk (k_gauss_walk.hip): counts into call boundaries; every chunk
+//      labelled with (call, first output position);
 //   3. scatter: every accepted candidate of a used chunk writes its three
 //      residues to its call's polynomial.
 #include <stdlib.h>
@@ -417,92 +416,6 @@ __global__ __launch_bounds__(CAND_THREADS) void k_gauss_firsts(const GaussStream
     }
 }
 
-// One wave per stream.  Window of 64 lanes x 16 chunks.  Full streams label
-// every used chunk with (call << 13 | first output position); compact streams
-// record only the first non-empty chunk of each call in firsts.
-__global__ __launch_bounds__(64) void k_gauss_walk(const GaussStream *__restrict__ streams, const uint8_t *__restrict__ cnt,
-                                                    int *__restrict__ pos, long long *__restrict__ firsts,
-                                                    int *__restrict__ status)
-{
-    const GaussStream *S = streams + blockIdx.x;
-    const int lane = threadIdx.x;
-    const long long base = S->chunk_base;
-    const int nchunks = S->nchunks, ncalls = S->ncalls;
-    const bool compact = S->coef0_only != 0;
-    int c = 0, call = 0, filled = 0;
-    bool first_done = false;
-    while (call < ncalls) {
-        if (c >= nchunks) {
-            if (lane == 0) status[blockIdx.x] = 1;
-            return;
-        }
-        uint32_t v[16];
-        uint32_t lsum = 0;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int ci = c + 16 * lane + r;
-            v[r] = (ci < nchunks) ? cnt[base + ci] : 0u;
-            lsum += v[r];
-        }
-        // inclusive wave scan of lsum
-        uint32_t incl = lsum;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            uint32_t o = __shfl_up(incl, d, 64);
-            if (lane >= d) incl += o;
-        }
-        const uint32_t excl = incl - lsum;
-        const uint32_t total = __shfl(incl, 63, 64);
-        if (compact && !first_done) {
-            const uint64_t nz = __ballot(lsum > 0);
-            if (nz) {
-                const int fl = __ffsll((unsigned long long)nz) - 1;
-                if (lane == fl) {
-                    int rr = 0;
-                    while (rr < 15 && v[rr] == 0) ++rr;
-                    firsts[S->first_base + call] = base + c + 16 * lane + rr;
-                }
-                first_done = true;
-            }
-        }
-        const uint32_t need = (uint32_t)S->slen - (uint32_t)filled;
-        const uint64_t hit = __ballot(incl >= need);
-        int e_chunk = -1;  // last chunk of this call, relative to c
-        if (hit) {
-            const int hl = __ffsll((unsigned long long)hit) - 1;
-            if (lane == hl) {
-                uint32_t run = excl;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    run += v[r];
-                    if (run >= need && e_chunk < 0) e_chunk = 16 * lane + r;
-                }
-            }
-            e_chunk = __shfl(e_chunk, hl, 64);
-        }
-        if (!compact) {
-            const int last = (e_chunk >= 0) ? e_chunk : 1023;
-            uint32_t run = excl;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int rel = 16 * lane + r;
-                const int ci = c + rel;
-                if (rel <= last && ci < nchunks) pos[base + ci] = (call << 13) | (int)((uint32_t)filled + run);
-                run += v[r];
-            }
-        }
-        if (e_chunk >= 0) {
-            ++call;
-            filled = 0;
-            first_done = false;
-            c += e_chunk + 1;
-        } else {
-            filled += (int)total;
-            c += 1024;
-        }
-    }
-}
-
 __global__ void k_gauss_scatter(const GaussStream *__restrict__ streams, int nstreams,
                                 const long long *__restrict__ chunk_prefix, long long nchunks_total,
                                 const uint8_t *__restrict__ cnt, const uint64_t *__restrict__ vals,
@@ -622,15 +535,6 @@ int launch_gauss_candidates(const GaussStream *d_streams, int nstreams, const lo
         hipLaunchKernelGGL((k_gauss_candidates<0, CAND_THREADS>), dim3(grid), dim3(CAND_THREADS), 0, st,
                            d_streams, nstreams, d_tile_prefix, ntiles, g_aes_te, cnt, vals, status, full,
                            scan_limit());
-    HIP_OK(hipGetLastError());
-    return 0;
-}
-
-int launch_gauss_walk(const GaussStream *d_streams, int nstreams, const uint8_t *cnt, int *pos, long long *firsts,
-                      int *status, hipStream_t st)
-{
-    if (nstreams <= 0) return 0;
-    hipLaunchKernelGGL(k_gauss_walk, dim3(nstreams), dim3(64), 0, st, d_streams, cnt, pos, firsts, status);
     HIP_OK(hipGetLastError());
     return 0;
 }

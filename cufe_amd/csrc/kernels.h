@@ -65,7 +65,8 @@ struct GaussStream {
     uint32_t q[4];           // output moduli, limbs 0 .. nmod-1
     uint32_t fold[4];        // mod_prime fold shifts per limb: a | b << 8 (q = 2^a - 2^b + 1)
     int nmod;                // output limbs
-    int pad;
+    int span;                // chunks a call may span (a longer one counts as a short window)
+    long long map_base;      // compact streams: first word of the stream's maps in the walk's map array
 };
 
 // Chunks per tile of the candidate pass (the host's tile_prefix counts tiles of
@@ -80,10 +81,15 @@ constexpr int GAUSS_TILE_CHUNKS = 63;
 // read unless a chunk's uniform scan runs long, which sets status bit 4)
 int launch_gauss_candidates(const GaussStream *d_streams, int nstreams, const long long *d_tile_prefix,
                             long long ntiles, uint8_t *cnt, uint64_t *vals, int *status, int full, hipStream_t st);
-// Walk: per stream, the call boundaries from the counts; writes per chunk
-// (call << 13 | offset) or -1.  status[stream] = 1 when the window was short.
-int launch_gauss_walk(const GaussStream *d_streams, int nstreams, const uint8_t *cnt, int *pos, long long *firsts,
-                      int *status, hipStream_t st);
+// Walk (k_gauss_walk.hip): per stream, the call boundaries from the counts;
+// writes per chunk of the full streams (call << 13 | offset) or -1, padding
+// included.  status[stream] = 1 when the window was short (else it stays).
+// Streams start on a multiple of 16 chunks and pad their last to one; map
+// holds span words per window of GAUSS_WALK_WIN chunks of the compact
+// streams (full streams keep theirs in pos); max_chunks: the longest window.
+constexpr int GAUSS_WALK_WIN = 16384;
+int launch_gauss_walk(const GaussStream *d_streams, int nstreams, int max_chunks, const uint8_t *cnt, int *pos,
+                      uint32_t *map, long long *firsts, int *status, hipStream_t st);
 // Compact streams: recompute the first non-empty chunk of every call and write sample 0.
 int launch_gauss_firsts(const GaussStream *d_streams, int nstreams, const long long *d_first_prefix,
                         const long long *firsts, long long nitems, int *status, int full, hipStream_t st);

@@ -133,15 +133,26 @@ StreamReq make_stream_ps(const PsetSpec &ps, const uint8_t key[32], uint16_t non
 // root).  The window takes the mean plus 1.5% plus 8 standard deviations;
 // level m doubles the margin m times (a short window is detected and retried,
 // never wrong).
+static const double kChunkMean[6] = {0.0, 751.6, 951.8, 1323.4, 752.8, 753.4};
+static const double kChunkSd[6] = {0.0, 6.6, 10.1, 16.2, 6.6, 6.8};
+
 long long gauss_window(int which, int slen, int ncalls, int m)
 {
-    static const double mean[6] = {0.0, 751.6, 951.8, 1323.4, 752.8, 753.4};
-    static const double sd[6] = {0.0, 6.6, 10.1, 16.2, 6.6, 6.8};
     const int w = (which >= 1 && which <= 5) ? which : 3;
     const double n = (double)ncalls * (double)slen / 4096.0;
-    double margin = 0.015 * mean[w] * n + 8.0 * sd[w] * sqrt(n) + 64.0;
+    double margin = 0.015 * kChunkMean[w] * n + 8.0 * kChunkSd[w] * sqrt(n) + 64.0;
     for (int i = 0; i < m; ++i) margin *= 2.0;
-    return (long long)ceil(mean[w] * n + margin);
+    return (long long)ceil(kChunkMean[w] * n + margin);
+}
+
+// Chunks one call of slen samples may span in the walk: the mean plus 20
+// standard deviations plus 1.5% (never exceeded; a longer call would be
+// reported as a short window).  At most slen / 2, for the walk's halo.
+static int gauss_span(int which, int slen)
+{
+    const int w = (which >= 1 && which <= 5) ? which : 3;
+    const double n = (double)slen / 4096.0;
+    return std::min(slen / 2, (int)ceil(1.015 * kChunkMean[w] * n + 20.0 * kChunkSd[w] * sqrt(n)));
 }
 
 long long gauss_window(int which, int ncalls, int m) { return gauss_window(which, IPFE_N, ncalls, m); }
@@ -149,7 +160,10 @@ long long gauss_window(int which, int ncalls, int m) { return gauss_window(which
 size_t gauss_bytes(int which, int slen, int ncalls, int coef0_only)
 {
     const long long ch = gauss_window(which, slen, ncalls, 0);
-    return coef0_only ? (size_t)ch * 1 + (size_t)ncalls * 8 : (size_t)ch * (1 + 64 + 4);
+    // compact streams: a count per chunk, a first chunk per call, the walk's maps
+    return coef0_only ? (size_t)ch * 1 + (size_t)ncalls * 8 +
+                            (size_t)((ch + GAUSS_WALK_WIN - 1) / GAUSS_WALK_WIN) * gauss_span(which, slen) * 4
+                      : (size_t)ch * (1 + 64 + 4);
 }
 
 size_t gauss_bytes(int which, int ncalls, int coef0_only) { return gauss_bytes(which, IPFE_N, ncalls, coef0_only); }
@@ -163,7 +177,8 @@ int GaussPlan::build(const StreamReq *reqs, int count, int lvl, bool alloc_meta)
     tile_prefix.assign(n, 0);
     chunk_prefix.assign(n, 0);
     first_prefix.assign(n, 0);
-    tiles = chunks = full_chunks = nfirst = 0;
+    tiles = chunks = full_chunks = nfirst = map_words = 0;
+    max_chunks = 0;
     // full streams first, so per-chunk values and labels cover only their chunks
     std::vector<int> order;
     for (int i = 0; i < n; ++i)
@@ -190,14 +205,22 @@ int GaussPlan::build(const StreamReq *reqs, int count, int lvl, bool alloc_meta)
             g.fold[t] = rq.fold[t];
         }
         g.nmod = rq.nmod;
-        g.pad = 0;
+        g.span = gauss_span(rq.which, rq.slen);
+        g.map_base = map_words;
         tile_prefix[i] = tiles;
         chunk_prefix[i] = chunks;
         first_prefix[i] = nfirst;
         tiles += (g.nchunks + kTile - 1) / kTile;
-        chunks += g.nchunks;
-        if (g.coef0_only) nfirst += g.ncalls;
-        else full_chunks = chunks;
+        // whole groups of 16 chunks, so that the walk reads and writes several
+        // chunks at a time
+        chunks += (g.nchunks + 15) / 16 * 16;
+        max_chunks = std::max(max_chunks, g.nchunks);
+        if (g.coef0_only) {
+            nfirst += g.ncalls;
+            map_words += (long long)((g.nchunks + GAUSS_WALK_WIN - 1) / GAUSS_WALK_WIN) * g.span;
+        } else {
+            full_chunks = chunks;
+        }
     }
     if (!alloc_meta) return 0;
     if (d_streams.alloc(n) || d_tp.alloc(n) || d_cp.alloc(n) || d_fp.alloc(n) || d_status.alloc(n + 1) ||
@@ -262,9 +285,12 @@ int GaussPlan::bind_scratch(uint8_t *cnt, uint64_t *vals, int *pos)
 
 int GaussPlan::alloc_scratch()
 {
-    if (own_cnt.alloc((size_t)chunks) || own_vals.alloc((size_t)full_chunks * 8 + 1) ||
+    // the counts, then (compact streams) the walk's maps
+    const size_t counts = align256((size_t)chunks);
+    if (own_cnt.alloc(counts + (size_t)map_words * 4) || own_vals.alloc((size_t)full_chunks * 8 + 1) ||
         own_pos.alloc((size_t)full_chunks + 1))
         return -1;
+    s_map = (uint32_t *)(own_cnt.get() + counts);
     return bind_scratch(own_cnt.get(), own_vals.get(), own_pos.get());
 }
 
@@ -291,12 +317,12 @@ int GaussPlan::upload(hipStream_t st)
     return 0;
 }
 
-// Kernels only (fills, candidates, walk, scatter, firsts): capturable.
+// Kernels only (fill, candidates, walk, scatter, firsts): capturable.
 int GaussPlan::launch(hipStream_t st)
 {
-    if (launch_fill_i32(s_pos, -1, (size_t)full_chunks, st) || launch_fill_i32(m_status, 0, n + 1, st)) return -1;
+    if (launch_fill_i32(m_status, 0, n + 1, st)) return -1;
     if (launch_gauss_candidates(m_streams, n, m_tp, tiles, s_cnt, s_vals, m_status + n, full, st)) return -1;
-    if (launch_gauss_walk(m_streams, n, s_cnt, s_pos, m_first, m_status, st)) return -1;
+    if (launch_gauss_walk(m_streams, n, max_chunks, s_cnt, s_pos, s_map, m_first, m_status, st)) return -1;
     if (launch_gauss_scatter(m_streams, n, m_cp, full_chunks, s_cnt, s_vals, s_pos, st)) return -1;
     if (launch_gauss_firsts(m_streams, n, m_fp, m_first, nfirst, m_status + n, full, st)) return -1;
     return 0;

@@ -92,6 +92,8 @@ struct GaussPlan {
     int n = 0, level = 0;
     int full = 0;  // all 24 AES blocks per chunk (set after a chunk needed them)
     long long tiles = 0, chunks = 0, full_chunks = 0, nfirst = 0;
+    long long map_words = 0;  // of the walk's maps of the compact streams
+    int max_chunks = 0;
     std::vector<GaussStream> hs;
     std::vector<long long> tile_prefix, chunk_prefix, first_prefix;
     DevBuf<GaussStream> d_streams;
@@ -108,9 +110,12 @@ struct GaussPlan {
     uint8_t *s_cnt = nullptr;
     uint64_t *s_vals = nullptr;
     int *s_pos = nullptr;
+    uint32_t *s_map = nullptr;  // the walk's maps of the compact streams
 
     // alloc_meta false: plan only; the caller binds the device metadata
     // (bind_meta) and the chunk scratch (bind_scratch_region) to its memory
+    // (plans of full streams only: the walk's maps of compact streams come
+    // with alloc_scratch)
     int build(const StreamReq *reqs, int n, int level, bool alloc_meta = true);
     size_t meta_bytes() const;
     int bind_meta(uint8_t *base);

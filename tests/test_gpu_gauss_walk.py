@@ -1,0 +1,47 @@
+"""The sampler's call boundaries across the walk's windows of 16,384 chunks:
+streams that end inside the first window, near its edge and several windows
+on, the calls that lie across an edge, two streams of different lengths in one
+plan, and compact streams (sample 0 of each call).  Every word equals the
+oracle's sequential stream."""
+import hashlib
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def h(t: bytes) -> bytes:
+    return hashlib.sha256(t).digest()
+
+
+# a call takes about 752 (S1), 952 (S2) and 1323 (S3) chunks: the edge lies in
+# call 21, 17 and 12
+@pytest.mark.parametrize("which,ncalls", [(1, 21), (1, 22), (1, 66), (2, 17), (2, 18), (3, 12), (3, 13), (3, 27)])
+def test_calls_across_windows(gpu, po, which, ncalls):
+    print(f"[gpu-walk] S{which} x {ncalls}", flush=True)
+    key = h(b"w%d-%d" % (which, ncalls))
+    want = po.gauss_calls(key, 3, which, ncalls)
+    assert np.array_equal(gpu.gauss_sample([key], [3], which, ncalls)[0], want)
+    assert np.array_equal(gpu.gauss_sample_first([key], [3], which, ncalls)[0], want[:, :, 0])
+
+
+@pytest.mark.parametrize("pid,ncalls", [(0, 45), (2, 14)])
+def test_other_call_lengths_across_windows(gpu, po, pid, ncalls):
+    """2,048 and 8,192 samples a call: shorter and longer spans than 4,096."""
+    print(f"[gpu-walk] set {pid} x {ncalls}", flush=True)
+    key = h(b"wp%d" % pid)
+    for which in (1, 3):
+        got = gpu.PSet(pid).gauss_sample([key], [9], which, ncalls)[0]
+        assert np.array_equal(got, po.ps_gauss_calls(pid, key, 9, which, ncalls))
+
+
+def test_streams_of_uneven_lengths_in_one_plan(gpu, po):
+    """One message a plan: r and f_0 (two S2 calls, one window) beside l calls of S3."""
+    l = 30
+    a = po.sample_polya(h(b"wa"))
+    mpk, _ = po.setup_from_a(a, h(b"ws"), h(b"we"), l)
+    x = np.arange(2 * l, dtype=np.uint32).reshape(2, l) % 5
+    got = gpu.encrypt(x, mpk, h(b"w2"), h(b"w3"), nonce0=4)
+    for b in range(2):
+        assert np.array_equal(got[b], po.encrypt(x[b], mpk, h(b"w2"), h(b"w3"), 4 + b))
