@@ -107,7 +107,7 @@ __global__ __launch_bounds__(512) void k_mb_aes_rep2(const uint32_t *__restrict_
     const uint32_t base = (blockIdx.x * blockDim.x + threadIdx.x) * nblocks_per_thread;
     for (uint32_t i = 0; i < nblocks_per_thread; ++i) {
         uint32_t o[4];
-        aes256_ctr_block_t(tb, rk, 7u, base + i, o);
+        aes256_ctr_block_t(tb, rk, rk + 60, 7u, base + i, o);
         x ^= o[0] ^ o[1] ^ o[2] ^ o[3];
     }
     out[blockIdx.x * blockDim.x + threadIdx.x] = x;
@@ -209,14 +209,14 @@ __global__ void k_mb_aes_check(const uint32_t *__restrict__ rk, const uint32_t *
     aes256_ctr_block(rk, te, 9u, ctr, o1);
     if (rep2) {
         const AesTabRep2 tb(rep);
-        aes256_ctr_block_t(tb, rk, 9u, ctr, o2);
+        aes256_ctr_block_t(tb, rk, rk + 60, 9u, ctr, o2);
         aes256_ctr_window(tb, rk, 9u, ctr >> 8, w);
-        aes256_ctr_block_win(tb, rk, w, ctr, o3);
+        aes256_ctr_block_win(tb, rk, rk + 60, w, ctr, o3);
     } else {
         const AesTabRep tb(rep);
         aes256_ctr_block_rep(rk, rep, 9u, ctr, o2);
         aes256_ctr_window(tb, rk, 9u, ctr >> 8, w);
-        aes256_ctr_block_win(tb, rk, w, ctr, o3);
+        aes256_ctr_block_win(tb, rk, rk + 60, w, ctr, o3);
     }
     bool ok = true;
 #pragma unroll
@@ -312,11 +312,12 @@ extern "C" int cufe_microbench(int kind, double *result)
         if (out.alloc((size_t)blocks * 256 * 2)) return -1;
         const int iters = 4096;
         DevBuf<uint32_t> rk;
-        uint32_t hrk[60];
+        uint32_t hrk[64];  // round keys, then the last four byte-swapped
         uint8_t key[32];
         for (int i = 0; i < 32; ++i) key[i] = (uint8_t)i;
         aes256_expand_key(key, hrk);
-        if (rk.alloc(60)) return -1;
+        for (int i = 0; i < 4; ++i) hrk[60 + i] = __builtin_bswap32(hrk[56 + i]);
+        if (rk.alloc(64)) return -1;
         HIP_OK(hipMemcpy(rk.get(), hrk, sizeof hrk, hipMemcpyHostToDevice));
         for (int rep = 0; rep < 2; ++rep) {
             HIP_OK(hipEventRecord(a, st));

@@ -17,7 +17,6 @@
 #include <stdlib.h>
 
 #include <algorithm>
-#include <type_traits>
 
 #include "aes_dev.h"
 #include "kernels.h"
@@ -55,15 +54,19 @@ __device__ __forceinline__ uint32_t stream_residue(const GaussStream *S, int s, 
 }
 
 // CDT rows (low word, high word), src/gauss.c:62-72.
-__constant__ uint64_t c_CDT[9][2] = {{2200310400551559144ull, 3327841033070651387ull},
-                                     {7912151619254726620ull, 380075531178589176ull},
-                                     {5167367257772081627ull, 11604843442081400ull},
-                                     {5081592746475748971ull, 90134450315532ull},
-                                     {6522074513864805092ull, 175786317361ull},
-                                     {2579734681240182346ull, 85801740ull},
-                                     {8175784047440310133ull, 10472ull},
-                                     {2947787991558061753ull, 0ull},
-                                     {22489665999543ull, 0ull}};
+#define IPFE_CDT                                                                                            \
+    {{2200310400551559144ull, 3327841033070651387ull}, {7912151619254726620ull, 380075531178589176ull},     \
+     {5167367257772081627ull, 11604843442081400ull},   {5081592746475748971ull, 90134450315532ull},         \
+     {6522074513864805092ull, 175786317361ull},        {2579734681240182346ull, 85801740ull},               \
+     {8175784047440310133ull, 10472ull},               {2947787991558061753ull, 0ull},                      \
+     {22489665999543ull, 0ull}}
+constexpr uint64_t kCdt[9][2] = IPFE_CDT;
+__constant__ uint64_t c_CDT[9][2] = IPFE_CDT;
+// the upper halves of the high words that are not zero
+constexpr uint32_t kCdtHigh[5] = {(uint32_t)(kCdt[0][1] >> 32), (uint32_t)(kCdt[1][1] >> 32),
+                                  (uint32_t)(kCdt[2][1] >> 32), (uint32_t)(kCdt[3][1] >> 32),
+                                  (uint32_t)(kCdt[4][1] >> 32)};
+static_assert(kCdtHigh[4] > 0 && kCdt[5][1] >> 32 == 0, "five entries have an upper half");
 
 // Coefficients of the 2^a polynomial, src/gauss.c:82-103 (IEEE-754 bit patterns).
 __constant__ uint64_t c_EXP[10] = {0x3e833b70ffa2c5d4ull, 0x3eb4a480fda7e6e1ull, 0x3ef01b254493363full,
@@ -74,7 +77,6 @@ __constant__ uint64_t c_EXP[10] = {0x3e833b70ffa2c5d4ull, 0x3eb4a480fda7e6e1ull,
 extern const uint32_t *g_aes_te;  // device T-tables, set by the context
 
 constexpr int CAND_THREADS = 256;
-constexpr int TILE_CHUNKS = GAUSS_TILE_CHUNKS;
 constexpr int CHUNK_WORDS = 96;
 
 __device__ __forceinline__ int find_stream(const long long *prefix, int n, long long key)
@@ -90,7 +92,8 @@ __device__ __forceinline__ int find_stream(const long long *prefix, int n, long 
 // Bernoulli decision (src/gauss.c:204-264 and the S2/S3 copies): the
 // reference's exact sequence of IEEE double operations and integer bit tricks.
 // rb points at the 36 Bernoulli bytes of the candidate's group.
-__device__ __forceinline__ bool bernoulli_bit(uint64_t b, double k2inv, const uint32_t *rb, int ln)
+// bernoulli_exp: the bits the uniform word is compared with.
+__device__ __forceinline__ uint64_t bernoulli_exp(uint64_t b, double k2inv)
 {
     double vx = __longlong_as_double((long long)(b | 0x4330000000000000ull)) - 4503599627370496.0;
     vx = __dmul_rn(vx, k2inv);
@@ -101,7 +104,12 @@ __device__ __forceinline__ bool bernoulli_bit(uint64_t b, double k2inv, const ui
     double s = __fma_rn(__longlong_as_double((long long)c_EXP[0]), a, __longlong_as_double((long long)c_EXP[1]));
 #pragma unroll
     for (int i = 2; i < 10; ++i) s = __fma_rn(s, a, __longlong_as_double((long long)c_EXP[i]));
-    uint64_t res = t + (uint64_t)__double_as_longlong(s);
+    return t + (uint64_t)__double_as_longlong(s);
+}
+
+__device__ __forceinline__ bool bernoulli_bit(uint64_t b, double k2inv, const uint32_t *rb, int ln)
+{
+    const uint64_t res = bernoulli_exp(b, k2inv);
     uint64_t res_mant = (res & ((1ull << 52) - 1)) | (1ull << 52);
     uint64_t e = (res >> 52) + (uint64_t)(long long)-1003;
     uint64_t res_exp = (e < 64) ? (1ull << e) : 0ull;
@@ -121,7 +129,7 @@ struct Cand {
     bool acc;
 };
 
-// AES blocks of a chunk computed by default: 0..15 (bytes 0..255) and 17
+// AES blocks of a chunk k_gauss_firsts computes by default: 0..15 (bytes 0..255) and 17
 // (bytes 272..287, holding the sign byte 280).  Candidates read bytes 0..199
 // (CDT and Bernoulli words), the uniform words from byte 200 and byte 280; the
 // uniform scan stays below byte 256 unless it needs more than 14 words (seven
@@ -130,20 +138,10 @@ struct Cand {
 constexpr int PART_BLOCKS = 17;
 __device__ __forceinline__ int chunk_block(int j, int full) { return (full || j < 16) ? j : 17; }
 
-// Sign word (bytes 280..283) read from the chunk in LDS.
-struct SignInLds {
-    __device__ uint32_t operator()(const uint32_t *ch) const { return ch[70]; }
-};
-
 // ulim: uniform words a partial chunk may scan (14 covers its blocks; lower
-// values exist to exercise the rerun).  sign_word(ch) returns bytes 280..283
-// of the chunk, which hold the candidate's sign bit; with sign_if_zero it is
-// asked only for a zero candidate (the only one whose acceptance depends on
-// its sign), and the sign of every other candidate is reported as 0.
-template <typename SignWord = SignInLds>
+// values exist to exercise the rerun).
 __device__ __forceinline__ Cand eval_candidate(const uint32_t *ch, int c, int which, bool valid, int *status,
-                                               int full, int ulim, SignWord sign_word = SignWord(),
-                                               bool sign_if_zero = false)
+                                               int full, int ulim)
 {
     const uint64_t K = c_K[which], BF = c_BF[which];
     const uint32_t UQ = (uint32_t)c_UQ[which];
@@ -193,167 +191,318 @@ __device__ __forceinline__ Cand eval_candidate(const uint32_t *ch, int c, int wh
     out.z = xk + y;
     const uint64_t bin = (uint64_t)(uint32_t)(out.z + xk) * (uint64_t)(uint32_t)y;
     const bool bit = bernoulli_bit(bin, K2INV, gb + 16, ln);
-    out.sgn = (!sign_if_zero || out.z == 0) ? (sign_word(ch) >> c) & 1u : 0u;
+    out.sgn = (ch[70] >> c) & 1u;  // sign byte 280
     out.acc = bit && (out.z != 0 || out.sgn != 0);
     return out;
 }
 
-// AES of nch chunks of one stream into LDS: chunk k at ks + 96 k uses
-// counters 24 (chunk_of(k)) .. +23.
-// nb: blocks per chunk -- 24 (all), PART_BLOCKS (0..15 and 17) or 16 (0..15,
-// for streams whose values are not stored: the sign byte then matters only for
-// a zero candidate, and that block is computed where it is needed).
-// TM: the T-table layout in te -- 0: four 1 KiB tables; 1: T0 replicated per
-// bank (AesTabRep); 2: T0 and T2 replicated per bank (AesTabRep2).
-// win (TM 1 and 2; may be null): the counter windows w0, w0 + 1, ... of
-// aes256_ctr_window, 8 words each, covering every counter.
+// ---------------------------------------------------------------------------
+// Candidate pass.
+//
+// What a chunk's eight candidates read (byte offsets in the 384-byte chunk;
+// candidate c = 4 g + ln): the CDT words r1, r2 at 100 g + 8 ln and 32 beyond,
+// the Bernoulli words at 100 g + 64 + 8 ln and the byte 100 g + 96 + ln, the
+// uniform words from byte 200, the sign byte 280.  r1 decides only where r2
+// equals a CDT entry's high word, so blocks 0, 1 and 7 (r1 alone) and block 15
+// (the uniform words past the tenth) are not computed; nor is more than the
+// high 32 bits of r2 and of the Bernoulli word looked at, whose low halves
+// decide only where the high halves tie.  A candidate that such a tie (6 in
+// 2^31, 1 in 2^21) or a third rejected uniform word (7e-5 of chunks) leaves
+// open is recomputed by its lane from whole words.  That leaves the 12 blocks
+// 2..6, 8..14 of 24 a chunk -- and block 17, the sign, for streams whose
+// values are stored; without them only a zero candidate's acceptance depends
+// on its sign -- where all words of blocks 0..15 took 16 (17).
+//
+// Each wave works alone: 16 chunks are 192 blocks, three full rounds of the
+// wave (blocks 2-5, 8-11 and 6, 12-14, so that a round's lanes need the same
+// output words: two of four in the first two), then 128 candidates, two full
+// rounds.  No workgroup barriers, so the lookups of some waves run under the
+// arithmetic of others.  The 28 words a chunk leaves for its candidates fit 16
+// waves' buffers beside 128 KiB of tables.
+//
+// Bound by the LDS lookups (197 a block, 64 lanes in 2 CU cycles) and the VALU,
+// about equally: 5.8 G chunks/s on the
+// streams of 2,048 rows of 124 slots (58 ms; 114 ms for all words of blocks 0..15
+// in 512-thread workgroups with T0 and T2 alone, encryption and evaluation
+// alternating across barriers).
+//
+// Words of a chunk in the wave's buffer (28, 112 bytes):
+//    0..3  r2 high of candidates 0..3       4..7  their Bernoulli high words
+//    8     bytes of candidates 0..3         9..12 r2 high of 4..7
+//   13..16 Bernoulli high words of 4..7    17     their bytes
+//   18..27 uniform words 0..9
+// ---------------------------------------------------------------------------
+typedef const __attribute__((address_space(4))) uint32_t *RoundKeys;  // scalar loads
+
+// TM: the T-table layout in LDS -- 0: four 1 KiB tables; 1: T0 replicated per
+// bank (AesTabRep); 2: T0 and T2 (AesTabRep2); 3: all four (AesTabRep4).
 template <int TM>
-__device__ __forceinline__ void aes_block(const GaussStream *S, const uint32_t *te, const uint32_t *win, uint32_t w0,
-                                          uint32_t ctr, uint32_t (&o)[4])
-{
-    if constexpr (TM == 0) {
-        aes256_ctr_block(S->rk, te, S->nonce, ctr, o);
-    } else {
-        using Tab = std::conditional_t<TM == 2, AesTabRep2, AesTabRep>;
-        const Tab tb(te);
-        if (win)
-            aes256_ctr_block_win(tb, S->rk, win + 8 * ((ctr >> 8) - w0), ctr, o);
-        else
-            aes256_ctr_block_t(tb, S->rk, S->nonce, ctr, o);
+struct AesLayout;
+template <>
+struct AesLayout<0> {
+    using Tab = AesTab4;
+    static constexpr int words = AES_TABLE_WORDS;
+    static __device__ void stage(uint32_t *te, const uint32_t *g) { aes_stage_tables(te, g); }
+};
+template <>
+struct AesLayout<1> {
+    using Tab = AesTabRep;
+    static constexpr int words = AES_REP_WORDS;
+    static __device__ void stage(uint32_t *te, const uint32_t *g) { aes_stage_tables_rep(te, g); }
+};
+template <>
+struct AesLayout<2> {
+    using Tab = AesTabRep2;
+    static constexpr int words = AES_REP2_WORDS;
+    static __device__ void stage(uint32_t *te, const uint32_t *g) { aes_stage_tables_rep2(te, g); }
+};
+template <>
+struct AesLayout<3> {
+    using Tab = AesTabRep4;
+    static constexpr int words = AES_REP4_WORDS;
+    static __device__ void stage(uint32_t *te, const uint32_t *g) { aes_stage_tables_rep4(te, g); }
+};
+
+constexpr int CAND_NT = 1024, CAND_WAVES = CAND_NT / 64;
+constexpr int SUB_CHUNKS = 16, SUB_WORDS = 28;
+constexpr int CAND_WINDOWS = 8;  // of 256 counters: a 64-chunk tile's 1,536 touch at most seven
+static_assert(SUB_CHUNKS * SUB_WORDS + 8 * CAND_WINDOWS == 512, "the wave's buffer");
+
+// The parameters of a sampler width and the arithmetic all candidates share.
+struct WidthConsts {
+    uint32_t K, BF, UQ;
+    double k2inv;
+    __device__ explicit WidthConsts(int which)
+        : K((uint32_t)c_K[which]), BF((uint32_t)c_BF[which]), UQ((uint32_t)c_UQ[which]), k2inv(c_K2INV[which])
+    {
     }
+};
+
+// uniform word -> y (src/gauss.c:609-703): y = w - (floor(w BF / 2^32) + 1) K,
+// plus K when that is negative.
+__device__ __forceinline__ uint32_t uniform_y(uint32_t w, const WidthConsts &wc)
+{
+    const uint32_t r = w - __umulhi(w, wc.BF) * wc.K;
+    return r >= wc.K ? r - wc.K : r;
 }
 
-// cw: words per chunk in ks (CHUNK_WORDS, or fewer when only the first blocks
-// are stored).
-template <int TM, int NT, typename ChunkOf>
-__device__ __forceinline__ void aes_chunks(const GaussStream *S, const uint32_t *te, int nch, ChunkOf chunk_of,
-                                           uint32_t *ks, int cw, int full, int nb, const uint32_t *win, uint32_t w0)
+// z = xs K + y and the bits of 2^a that the Bernoulli step compares with
+// (bernoulli_bit above, the reference's IEEE double sequence).
+__device__ __forceinline__ uint64_t cand_exp(uint32_t xs, uint32_t y, const WidthConsts &wc, uint64_t &z)
 {
-    for (int g = threadIdx.x; g < nch * nb; g += NT) {
-        const int k = g / nb, blk = chunk_block(g - nb * k, full);
-        const uint32_t ctr = (uint32_t)(chunk_of(k) * 24 + blk);
-        uint32_t o[4];
-        aes_block<TM>(S, te, win, w0, ctr, o);
-        uint32_t *d = ks + k * cw + blk * 4;
-        d[0] = o[0]; d[1] = o[1]; d[2] = o[2]; d[3] = o[3];
-    }
+    const uint64_t xk = (uint64_t)xs * wc.K;
+    z = xk + y;
+    const uint64_t b = (uint64_t)(uint32_t)(z + xk) * y;
+    return bernoulli_exp(b, wc.k2inv);
 }
 
-// TM (aes_block): the four 1 KiB T-tables, T0 replicated per bank (32 KiB of
-// LDS; NT = 512, so that two workgroups per CU hold 16 waves) or T0 and T2
-// replicated (64 KiB).  With the 64 KiB tables two workgroups fit a CU's LDS
-// when the keystream buffer holds 64 words per chunk: streams that need only
-// blocks 0..15 run a tile in one pass; the others run two passes of 32 chunks
-// (72 words per chunk for blocks 0..15 and the sign word, 96 for all 24
-// blocks).
-template <int TM, int NT>
-__global__ __launch_bounds__(NT) void k_gauss_candidates(const GaussStream *__restrict__ streams, int nstreams,
-                                                                    const long long *__restrict__ tile_prefix,
-                                                                    long long ntiles,
-                                                                    const uint32_t *__restrict__ te_global,
-                                                                    uint8_t *__restrict__ cnt, uint64_t *__restrict__ vals,
-                                                                    int *__restrict__ status, int full, int ulim)
+// r_exp < res_exp: r_exp the 19 bits above the Bernoulli word's 53, res_exp =
+// 2^e with e from the exponent field (0 past 63)
+__device__ __forceinline__ bool bernoulli_exp_less(uint32_t res_hi, uint32_t rm_hi, uint32_t byte)
 {
-    // windows of 256 counters one tile spans (its 24 TILE_CHUNKS counters)
-    constexpr int WINDOWS = TILE_CHUNKS * 24 / 256 + 2;
-    constexpr int KS_WORDS = TM == 2 ? TILE_CHUNKS * 64 : TILE_CHUNKS * CHUNK_WORDS;
-    constexpr int HALF = 32;  // chunks per pass of the two-pass tiles
-    static_assert(TM != 2 || (HALF * CHUNK_WORDS <= KS_WORDS && 2 * HALF >= TILE_CHUNKS && NT >= HALF * 9 &&
-                              TILE_CHUNKS * 8 <= NT),
-                  "pass sizes of the two-table kernel");
-    __shared__ uint32_t te[TM == 2 ? AES_REP2_WORDS : TM == 1 ? AES_REP_WORDS : AES_TABLE_WORDS];
-    __shared__ uint32_t ks[KS_WORDS];
-    __shared__ uint32_t win[TM ? WINDOWS * 8 : 8];
-    if (TM == 2)
-        aes_stage_tables_rep2(te, te_global);
-    else if (TM == 1)
-        aes_stage_tables_rep(te, te_global);
-    else
-        aes_stage_tables(te, te_global);
-    const int sh = (threadIdx.x & 63) & 56;
-    for (long long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int si = __builtin_amdgcn_readfirstlane(find_stream(tile_prefix, nstreams, tile));
-        const GaussStream *S = streams + si;
-        const long long chunk0 = (tile - tile_prefix[si]) * TILE_CHUNKS;
-        const int nch = (int)min((long long)TILE_CHUNKS, (long long)S->nchunks - chunk0);
-        const int which = S->which;
-        const bool store_vals = !S->coef0_only;
-        // without stored values only a zero candidate needs its sign (a zero
-        // with sign 0 is rejected, src/gauss.c:1086-1163)
-        const bool lazy_sign = !store_vals && !full;
-        __syncthreads();  // tables staged / previous tile's reads of ks and win done
-        // counter windows of the tile (unless its counters wrap at 2^32)
-        const uint32_t c_lo = (uint32_t)(chunk0 * 24), w0 = c_lo >> 8;
-        const bool use_win = TM && chunk0 * 24 + (long long)nch * 24 <= (1ll << 32);
-        const int nw = (int)((c_lo + (uint32_t)(nch * 24 - 1)) >> 8) - (int)w0 + 1;
-        if constexpr (TM != 0) {
-            using Tab = std::conditional_t<TM == 2, AesTabRep2, AesTabRep>;
-            if (use_win && (int)threadIdx.x < nw)
-                aes256_ctr_window(Tab(te), S->rk, S->nonce, w0 + threadIdx.x, win + 8 * threadIdx.x);
+    const uint32_t e = (res_hi >> 20) - 1003u, r_exp = (rm_hi >> 21) | byte << 11;
+    return e < 64u && (r_exp >> min(e, 31u)) == 0;
+}
+
+// One candidate from whole words of its chunk, AES block by AES block, for the
+// lanes whose candidate the high words leave open.  status: as eval_candidate.
+template <class Tab>
+__device__ Cand cand_whole(const Tab &tb, const GaussStream *S, long long chunk, int c, const WidthConsts &wc,
+                           int *status, int full, int ulim, bool lazy_sign)
+{
+    uint32_t o[4] = {0, 0, 0, 0};
+    int cur = -1;
+    auto word = [&](int i) -> uint32_t {
+        if (cur != i >> 2) {
+            cur = i >> 2;
+            aes256_ctr_block_t(tb, &S->rk[0], &S->rkf[0], S->nonce, (uint32_t)(chunk * 24 + cur), o);
         }
-        // The two-table kernel's partial chunks of stored streams: a pass of
-        // HALF chunks computes blocks 0..15 only (HALF 16 = 512 blocks); the
-        // HALF 8 evaluating lanes take every sign as 1 while the next HALF
-        // threads, otherwise idle, compute block 17 -- the sign word -- of each
-        // chunk, and after a barrier the evaluating lanes settle sign and
-        // acceptance.
-        const bool split_sign = TM == 2 && !full && store_vals;
-        // chunks per pass and words per chunk in ks
-        const int sub = (TM == 2 && (full || store_vals)) ? HALF : TILE_CHUNKS;
-        const int cw = TM != 2 ? CHUNK_WORDS : full ? CHUNK_WORDS : store_vals ? 72 : 64;
-        for (int h = 0; h < nch; h += sub) {
-            __syncthreads();  // windows written / the previous pass's reads of ks done
-            const long long c0 = chunk0 + h;
-            const int nsub = min(sub, nch - h);
-            aes_chunks<TM, NT>(S, te, nsub, [c0](int k) { return c0 + k; }, ks, cw, full,
-                               full ? 24 : (lazy_sign || split_sign) ? 16 : PART_BLOCKS, use_win ? win : nullptr, w0);
-            __syncthreads();
-            // ballot of the accept bits and the chunk's count and values
-            auto commit = [&](const Cand &cd, int k, int c, bool valid) {
+        const uint32_t lo = (i & 1) ? o[1] : o[0], hi = (i & 1) ? o[3] : o[2];
+        return (i & 2) ? hi : lo;
+    };
+    const int g = c >> 2, ln = c & 3;
+    uint32_t w[9];  // uniform, r1, r2, Bernoulli (low, high each), byte word, sign
+    int need = -1, seen = 0;
+#pragma unroll 1
+    for (int u = 0; u < 46 && need < 0; ++u) {
+        if (!full && u >= ulim) break;
+        const uint32_t t = word(50 + u);
+        if (t < wc.UQ && seen++ == c) {
+            w[0] = t;
+            need = u;
+        }
+    }
+    if (need < 0) {
+        atomicOr(status, full ? 2 : 4);
+        w[0] = 0;
+    }
+    const int at[8] = {25 * g + 2 * ln,      25 * g + 2 * ln + 1,  25 * g + 8 + 2 * ln, 25 * g + 9 + 2 * ln,
+                       25 * g + 16 + 2 * ln, 25 * g + 17 + 2 * ln, 25 * g + 24,         70};
+#pragma unroll 1
+    for (int j = 0; j < 8; ++j) {
+        int i = at[0];
+        uint32_t t;
+#pragma unroll
+        for (int v = 1; v < 8; ++v) i = j == v ? at[v] : i;
+        t = word(i);
+#pragma unroll
+        for (int v = 0; v < 8; ++v) w[1 + v] = j == v ? t : w[1 + v];
+    }
+    const uint64_t r1 = (((uint64_t)w[2] << 32) | w[1]) & 0x7fffffffffffffffull;
+    const uint64_t r2 = (((uint64_t)w[4] << 32) | w[3]) & 0x7fffffffffffffffull;
+    uint32_t xs = 0;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) xs += (r2 < c_CDT[i][1]) | ((r2 == c_CDT[i][1]) & (r1 < c_CDT[i][0]));
+    Cand out;
+    const uint64_t res = cand_exp(xs, uniform_y(w[0], wc), wc, out.z);
+    const uint64_t rm = ((uint64_t)w[6] << 32) | w[5];
+    const uint64_t res_mant = (res & ((1ull << 52) - 1)) | (1ull << 52), r_mant = rm & ((1ull << 53) - 1);
+    const bool bit = (r_mant < res_mant && bernoulli_exp_less((uint32_t)(res >> 32), w[6], (w[7] >> (8 * ln)) & 255u)) ||
+                     res == 0x3FF0000000000000ull;
+    out.sgn = (!lazy_sign || out.z == 0) ? (w[8] >> c) & 1u : 0u;
+    out.acc = bit && (out.z != 0 || out.sgn != 0);
+    return out;
+}
+
+template <int TM>
+__global__ __launch_bounds__(CAND_NT) void k_gauss_candidates(const GaussStream *__restrict__ streams, int nstreams,
+                                                               const long long *__restrict__ tile_prefix,
+                                                               long long ntiles, int tile_chunks,
+                                                               const uint32_t *__restrict__ te_global,
+                                                               uint8_t *__restrict__ cnt, uint64_t *__restrict__ vals,
+                                                               int *__restrict__ status, int full, int ulim, int whole)
+{
+    using Tab = typename AesLayout<TM>::Tab;
+    __shared__ __align__(16) uint32_t te[AesLayout<TM>::words];
+    __shared__ __align__(16) uint32_t bufs[CAND_WAVES][512];
+    AesLayout<TM>::stage(te, te_global);
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // this wave's run of consecutive tiles; the first waves of all workgroups
+    // come first, so that a short plan spreads over the CUs
+    const long long waves = (long long)gridDim.x * CAND_WAVES, me = (long long)wv * gridDim.x + blockIdx.x;
+    const long long t0 = me * ntiles / waves, t1 = (me + 1) * ntiles / waves;
+    if (t0 >= t1) return;
+    const Tab tb(te);
+    uint32_t *buf = bufs[wv], *win = buf + SUB_CHUNKS * SUB_WORDS;
+    int si = __builtin_amdgcn_readfirstlane(find_stream(tile_prefix, nstreams, t0));
+    auto wave_sync = [] {  // the wave's LDS accesses stay in order across this point
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+    };
+    for (long long tile = t0; tile < t1; ++tile) {
+        while (si + 1 < nstreams && tile_prefix[si + 1] <= tile) ++si;
+        const GaussStream *S = streams + si;
+        const long long chunk0 = (tile - tile_prefix[si]) * tile_chunks;
+        const int nch = (int)min((long long)tile_chunks, (long long)S->nchunks - chunk0);
+        const WidthConsts wc(S->which);
+        const bool store_vals = !S->coef0_only;
+        const uint32_t nonce = S->nonce;
+        const uint64_t rk_addr = reinterpret_cast<uint64_t>(&S->rk[0]);
+        // The round keys are read anew for every round of blocks (the empty
+        // asm keeps the loads there): 64 scalar registers held across the
+        // evaluation would be spilled to vector lanes.
+        auto keys = [rk_addr]() {
+            uint64_t a = rk_addr;
+            asm volatile("" : "+s"(a));
+            return (RoundKeys)a;
+        };
+        // windows of 256 counters the tile touches (counters wrap at 2^32)
+        const uint32_t c_lo = (uint32_t)(chunk0 * 24), w0 = c_lo >> 8;
+        const int nw = (int)(((c_lo & 255u) + (uint32_t)(nch * 24 - 1)) >> 8) + 1;
+        wave_sync();
+        if (lane < nw) aes256_ctr_window(tb, keys(), nonce, (w0 + lane) & 0xffffffu, win + 8 * lane);
+        wave_sync();
+        auto window = [&](uint32_t ctr) { return win + 8 * (((ctr >> 8) - w0) & (CAND_WINDOWS - 1)); };
+        uint32_t sign = 0;  // lane l: the sign word of the tile's chunk l
+        if (store_vals) {
+            const uint32_t ctr = (uint32_t)((chunk0 + min(lane, nch - 1)) * 24 + 17);
+            uint32_t o[4];
+            const RoundKeys rk = keys();
+            aes256_ctr_block_win<4>(tb, rk, rk + 60, window(ctr), ctr, o);
+            sign = o[2];
+        }
+        for (int s = 0; s < nch; s += SUB_CHUNKS) {
+            const int nsub = min(SUB_CHUNKS, nch - s);
+            {
+                const int k = lane >> 2, j = lane & 3;
+                const uint32_t base = (uint32_t)((chunk0 + s + min(k, nsub - 1)) * 24);
+                uint32_t *d = buf + SUB_WORDS * k;
+                uint32_t o[4];
+                {
+                    const uint32_t ctr = base + 2 + j;
+                    const RoundKeys rk = keys();
+                    aes256_ctr_block_win<2 | 8>(tb, rk, rk + 60, window(ctr), ctr, o);
+                    *reinterpret_cast<uint2 *>(d + 2 * j) = make_uint2(o[1], o[3]);
+                }
+                {
+                    const uint32_t ctr = base + 8 + j;
+                    const RoundKeys rk = keys();
+                    aes256_ctr_block_win<1 | 4>(tb, rk, rk + 60, window(ctr), ctr, o);
+                    *reinterpret_cast<uint2 *>(d + 8 + 2 * j) = make_uint2(o[0], o[2]);
+                }
+                {
+                    const uint32_t ctr = base + (j == 0 ? 6 : 11 + j);
+                    const RoundKeys rk = keys();
+                    aes256_ctr_block_win(tb, rk, rk + 60, window(ctr), ctr, o);
+                    if (j == 0)
+                        d[8] = o[0];  // over block 8's first word, which no candidate reads
+                    else
+                        *reinterpret_cast<uint4 *>(d + 12 + 4 * j) = make_uint4(o[0], o[1], o[2], o[3]);
+                }
+            }
+            wave_sync();
+#pragma unroll 1
+            for (int e = 0; e < 2; ++e) {
+                const int k = 8 * e + (lane >> 3), c = lane & 7, sh = lane & 56;
+                const bool valid = k < nsub;
+                const uint32_t *q = buf + SUB_WORDS * k;
+                // the c-th uniform word below UQ
+                uint32_t w = q[18 + c];
+                bool open = false;
+                const uint64_t kept = __ballot(w < wc.UQ);
+                if (kept != ~0ull) {
+                    const uint32_t bad = ~((uint32_t)((kept >> sh) & 0xffu) | (q[26] < wc.UQ ? 256u : 0u) |
+                                           (q[27] < wc.UQ ? 512u : 0u));
+                    // its position: c plus the rejected words up to it
+                    int pos = c;
+#pragma unroll
+                    for (int it = 0; it < 3; ++it) pos = c + __popc(bad & ((2u << min(pos, 15)) - 1u));
+                    open = pos >= min(ulim, 10) || pos != c + __popc(bad & ((2u << min(pos, 15)) - 1u));
+                    w = q[18 + min(pos, 9)];
+                }
+                const uint32_t y = uniform_y(w, wc);
+                // CDT rank by the high word
+                const uint32_t r2h = q[c < 4 ? c : c + 5] & 0x7fffffffu;
+                uint32_t xs = 0;
+                bool tie = r2h == 0;  // the entries from the sixth on have a zero high word
+#pragma unroll
+                for (int i = 0; i < 5; ++i) {
+                    xs += r2h < kCdtHigh[i];
+                    tie = tie || r2h == kCdtHigh[i];
+                }
+                Cand cd;
+                const uint64_t res = cand_exp(xs, y, wc, cd.z);
+                const uint32_t rm_hi = q[c < 4 ? 4 + c : 9 + c], bytes = q[c < 4 ? 8 : 17];
+                const uint32_t res_hi = (uint32_t)(res >> 32);
+                const uint32_t mant = (res_hi & 0xfffffu) | 0x100000u, rmant = rm_hi & 0x1fffffu;
+                const bool bit = (rmant < mant && bernoulli_exp_less(res_hi, rm_hi, (bytes >> (8 * (c & 3))) & 255u)) ||
+                                 res == 0x3FF0000000000000ull;
+                open = valid && (whole || open || tie || rmant == mant || (!store_vals && cd.z == 0));
+                cd.sgn = store_vals ? (__shfl(sign, s + k, 64) >> c) & 1u : 0u;
+                cd.acc = valid && bit && (store_vals ? (cd.z != 0 || cd.sgn != 0) : true);
+                if (open) cd = cand_whole(tb, S, chunk0 + s + k, c, wc, status, full, ulim, !store_vals);
                 const uint64_t am = __ballot(cd.acc);
                 const uint32_t gm = (uint32_t)((am >> sh) & 0xffu);
                 if (valid) {
-                    const long long gc = S->chunk_base + c0 + k;
+                    const long long gc = S->chunk_base + chunk0 + s + k;
                     if (c == 0) cnt[gc] = (uint8_t)__popc(gm);
                     if (store_vals && cd.acc)
                         vals[gc * 8 + __popc(gm & ((1u << c) - 1u))] = cd.z | ((uint64_t)cd.sgn << 63);
                 }
-            };
-            if (split_sign) {
-                const int t = threadIdx.x, k = t >> 3, c = t & 7;
-                const bool eval = t < HALF * 8;
-                Cand cd{};
-                if (eval) {
-                    cd = eval_candidate(ks + k * cw, c, which, k < nsub, status, full, ulim,
-                                        [](const uint32_t *) { return ~0u; });
-                } else if (t < HALF * 8 + nsub) {
-                    const int kb = t - HALF * 8;
-                    uint32_t o[4];
-                    aes_block<TM>(S, te, use_win ? win : nullptr, w0, (uint32_t)((c0 + kb) * 24 + 17), o);
-                    ks[kb * cw + 70] = o[2];
-                }
-                __syncthreads();
-                if (eval) {
-                    // with every sign 1, cd.acc was the Bernoulli bit alone
-                    cd.sgn = (ks[k * cw + 70] >> c) & 1u;
-                    cd.acc = cd.acc && (cd.z != 0 || cd.sgn != 0);
-                    commit(cd, k, c, k < nsub);
-                }
-                continue;
             }
-            for (int slot = threadIdx.x; slot < sub * 8; slot += NT) {
-                const int k = slot >> 3, c = slot & 7;
-                // with lazy_sign, block 17 of chunk k is computed by the asking
-                // lane alone (a zero candidate: about 1e-9 of S2/S3 candidates)
-                auto sign_word = [&](const uint32_t *ch) -> uint32_t {
-                    if (!lazy_sign) return ch[70];
-                    uint32_t o[4];
-                    aes_block<TM>(S, te, nullptr, 0, (uint32_t)((c0 + k) * 24 + 17), o);
-                    return o[2];
-                };
-                commit(eval_candidate(ks + k * cw, c, which, k < nsub, status, full, ulim, sign_word, lazy_sign),
-                       k, c, k < nsub);
-            }
+            wave_sync();
         }
     }
 }
@@ -497,13 +646,12 @@ __global__ void k_aes_ctr(const uint32_t *__restrict__ rk, const uint32_t *__res
 }
 
 // ---------------------------------------------------------------------------
-// 0: four T-tables, 256 threads; 1: T0 replicated, 512 threads; 2: T0
-// replicated, 256 threads; 3 (default): T0 and T2 replicated, 512 threads,
-// keystream in half-tile passes (CUFE_AES_REP)
+// CUFE_AES_REP: the table layout of the candidate pass -- 0: the four 1 KiB
+// T-tables; 1, 2: T0 replicated; 3: T0 and T2; else (default) all four.
 static int aes_rep_mode()
 {
     const char *e = getenv("CUFE_AES_REP");
-    return e && *e ? atoi(e) : 3;
+    return e && *e ? atoi(e) : 4;
 }
 
 // Uniform words a partial chunk may scan before it asks for all 24 blocks:
@@ -516,25 +664,46 @@ static int scan_limit()
     return v < 8 ? 8 : (v > 14 ? 14 : v);
 }
 
+// One workgroup per CU: its tables and buffers take the whole LDS.
+static int candidate_blocks()
+{
+    static const int cus = [] {
+        hipDeviceProp_t prop;
+        int d = 0;
+        if (hipGetDevice(&d) != hipSuccess || hipGetDeviceProperties(&prop, d) != hipSuccess) return 256;
+        return prop.multiProcessorCount;
+    }();
+    return cus;
+}
+
+int gauss_candidate_waves() { return candidate_blocks() * CAND_WAVES; }
+
 int launch_gauss_candidates(const GaussStream *d_streams, int nstreams, const long long *d_tile_prefix,
-                            long long ntiles, uint8_t *cnt, uint64_t *vals, int *status, int full, hipStream_t st)
+                            long long ntiles, int tile, uint8_t *cnt, uint64_t *vals, int *status, int full,
+                            hipStream_t st)
 {
     if (ntiles <= 0) return 0;
-    const unsigned grid = (unsigned)std::min<long long>(ntiles, 1ll << 20);
+    if (tile != 16 && tile != 32 && tile != 64) {
+        ipfe_set_error("Gaussian candidates: tiles of %d chunks", tile);
+        return -1;
+    }
+    const unsigned grid = (unsigned)std::min<long long>(ntiles, candidate_blocks());
     const int rep = aes_rep_mode();
-    if (rep >= 3)
-        hipLaunchKernelGGL((k_gauss_candidates<2, 512>), dim3(grid), dim3(512), 0, st, d_streams, nstreams,
-                           d_tile_prefix, ntiles, g_aes_te, cnt, vals, status, full, scan_limit());
-    else if (rep == 2)
-        hipLaunchKernelGGL((k_gauss_candidates<1, 256>), dim3(grid), dim3(256), 0, st, d_streams, nstreams,
-                           d_tile_prefix, ntiles, g_aes_te, cnt, vals, status, full, scan_limit());
-    else if (rep == 1)
-        hipLaunchKernelGGL((k_gauss_candidates<1, 512>), dim3(grid), dim3(512), 0, st, d_streams, nstreams,
-                           d_tile_prefix, ntiles, g_aes_te, cnt, vals, status, full, scan_limit());
+    // CUFE_GAUSS_WHOLE=1 (tests): every candidate from whole words
+    const char *w = getenv("CUFE_GAUSS_WHOLE");
+    const int whole = w && atoi(w) != 0;
+#define CAND(TM)                                                                                                   \
+    hipLaunchKernelGGL(k_gauss_candidates<TM>, dim3(grid), dim3(CAND_NT), 0, st, d_streams, nstreams, d_tile_prefix, \
+                       ntiles, tile, g_aes_te, cnt, vals, status, full, scan_limit(), whole)
+    if (rep >= 4)
+        CAND(3);
+    else if (rep == 3)
+        CAND(2);
+    else if (rep >= 1)
+        CAND(1);
     else
-        hipLaunchKernelGGL((k_gauss_candidates<0, CAND_THREADS>), dim3(grid), dim3(CAND_THREADS), 0, st,
-                           d_streams, nstreams, d_tile_prefix, ntiles, g_aes_te, cnt, vals, status, full,
-                           scan_limit());
+        CAND(0);
+#undef CAND
     HIP_OK(hipGetLastError());
     return 0;
 }

@@ -50,6 +50,7 @@ int launch_point_mul(const uint32_t *a, const uint32_t *b, uint32_t *out, size_t
 // candidates each; call 0 writes to out0, call k >= 1 to out1 + (k-1)*out_stride.
 struct GaussStream {
     uint32_t rk[60];         // expanded AES-256 key
+    uint32_t rkf[4];         // its last four words, byte-swapped
     uint32_t nonce;          // 16-bit nonce
     int which;               // sampler width index into the device tables: 1, 2, 3 (S1, S2, S3 of the
                              // reference set), 4, 5 (the S2 / S3 widths of the N = 2048 set)
@@ -69,18 +70,16 @@ struct GaussStream {
     long long map_base;      // compact streams: first word of the stream's maps in the walk's map array
 };
 
-// Chunks per tile of the candidate pass (the host's tile_prefix counts tiles of
-// this size): 63, so that a tile's 16 AES blocks per chunk take two rounds of
-// 512 threads and its keystream (64 words per chunk) fits the LDS left beside
-// the 64 KiB T-tables of two workgroups.
-constexpr int GAUSS_TILE_CHUNKS = 63;
-
 // Candidate pass: for every chunk of every stream, AES + CDT + Bernoulli;
 // writes the accepted count and the accepted (z | sign << 63) values in order.
-// full: compute all 24 AES blocks of each chunk (else the 17 that candidates
-// read unless a chunk's uniform scan runs long, which sets status bit 4)
+// tile_prefix counts tiles of `tile` chunks per stream (16, 32 or 64).
+// full: a chunk whose uniform scan runs past the words the default AES blocks
+// hold is scanned on (else it sets status bit 4)
 int launch_gauss_candidates(const GaussStream *d_streams, int nstreams, const long long *d_tile_prefix,
-                            long long ntiles, uint8_t *cnt, uint64_t *vals, int *status, int full, hipStream_t st);
+                            long long ntiles, int tile, uint8_t *cnt, uint64_t *vals, int *status, int full,
+                            hipStream_t st);
+// Waves the candidate pass runs at once (tiles are dealt to them).
+int gauss_candidate_waves();
 // Walk (k_gauss_walk.hip): per stream, the call boundaries from the counts;
 // writes per chunk of the full streams (call << 13 | offset) or -1, padding
 // included.  status[stream] = 1 when the window was short (else it stays).

@@ -168,9 +168,14 @@ size_t gauss_bytes(int which, int slen, int ncalls, int coef0_only)
 
 size_t gauss_bytes(int which, int ncalls, int coef0_only) { return gauss_bytes(which, IPFE_N, ncalls, coef0_only); }
 
+static void set_round_keys(GaussStream &g, const StreamReq &rq)
+{
+    memcpy(g.rk, rq.rk, sizeof g.rk);
+    for (int i = 0; i < 4; ++i) g.rkf[i] = __builtin_bswap32(rq.rk[56 + i]);
+}
+
 int GaussPlan::build(const StreamReq *reqs, int count, int lvl, bool alloc_meta)
 {
-    constexpr int kTile = GAUSS_TILE_CHUNKS;
     n = count;
     level = lvl;
     hs.assign(n, GaussStream{});
@@ -188,7 +193,7 @@ int GaussPlan::build(const StreamReq *reqs, int count, int lvl, bool alloc_meta)
     for (int i = 0; i < n; ++i) {
         const StreamReq &rq = reqs[order[i]];
         GaussStream &g = hs[i];
-        memcpy(g.rk, rq.rk, sizeof g.rk);
+        set_round_keys(g, rq);
         g.nonce = rq.nonce;
         g.which = rq.which;
         g.ncalls = rq.ncalls;
@@ -207,10 +212,8 @@ int GaussPlan::build(const StreamReq *reqs, int count, int lvl, bool alloc_meta)
         g.nmod = rq.nmod;
         g.span = gauss_span(rq.which, rq.slen);
         g.map_base = map_words;
-        tile_prefix[i] = tiles;
         chunk_prefix[i] = chunks;
         first_prefix[i] = nfirst;
-        tiles += (g.nchunks + kTile - 1) / kTile;
         // whole groups of 16 chunks, so that the walk reads and writes several
         // chunks at a time
         chunks += (g.nchunks + 15) / 16 * 16;
@@ -221,6 +224,26 @@ int GaussPlan::build(const StreamReq *reqs, int count, int lvl, bool alloc_meta)
         } else {
             full_chunks = chunks;
         }
+    }
+    // Chunks per tile of the candidate pass.  A wave's tile takes three rounds
+    // of AES per 16 chunks, and for full streams one more for the tile's sign
+    // blocks, of which a 64-chunk tile fills every lane; smaller tiles spread a
+    // short plan over more waves.  The size whose busiest wave has the fewest
+    // rounds, larger on a tie.
+    const long long waves = gauss_candidate_waves();
+    long long best = 0;
+    for (int t : {64, 32, 16}) {
+        long long nt = 0;
+        for (const GaussStream &g : hs) nt += (g.nchunks + t - 1) / t;
+        const long long rounds = (nt + waves - 1) / waves * (3 * t / 16 + (full_chunks > 0));
+        if (best == 0 || rounds < best) {
+            best = rounds;
+            tile = t;
+        }
+    }
+    for (int i = 0; i < n; ++i) {
+        tile_prefix[i] = tiles;
+        tiles += (hs[i].nchunks + tile - 1) / tile;
     }
     if (!alloc_meta) return 0;
     if (d_streams.alloc(n) || d_tp.alloc(n) || d_cp.alloc(n) || d_fp.alloc(n) || d_status.alloc(n + 1) ||
@@ -303,7 +326,7 @@ void GaussPlan::rekey(const StreamReq *reqs)
     for (int i = 0; i < n; ++i)
         if (reqs[i].coef0_only) order.push_back(i);
     for (int i = 0; i < n; ++i) {
-        memcpy(hs[i].rk, reqs[order[i]].rk, sizeof hs[i].rk);
+        set_round_keys(hs[i], reqs[order[i]]);
         hs[i].nonce = reqs[order[i]].nonce;
     }
 }
@@ -321,7 +344,7 @@ int GaussPlan::upload(hipStream_t st)
 int GaussPlan::launch(hipStream_t st)
 {
     if (launch_fill_i32(m_status, 0, n + 1, st)) return -1;
-    if (launch_gauss_candidates(m_streams, n, m_tp, tiles, s_cnt, s_vals, m_status + n, full, st)) return -1;
+    if (launch_gauss_candidates(m_streams, n, m_tp, tiles, tile, s_cnt, s_vals, m_status + n, full, st)) return -1;
     if (launch_gauss_walk(m_streams, n, max_chunks, s_cnt, s_pos, s_map, m_first, m_status, st)) return -1;
     if (launch_gauss_scatter(m_streams, n, m_cp, full_chunks, s_cnt, s_vals, s_pos, st)) return -1;
     if (launch_gauss_firsts(m_streams, n, m_fp, m_first, nfirst, m_status + n, full, st)) return -1;

@@ -90,10 +90,11 @@ int run_gauss(const std::vector<StreamReq> &reqs, hipStream_t st, size_t scratch
 // status check that reports a speculative window that was too short.
 struct GaussPlan {
     int n = 0, level = 0;
-    int full = 0;  // all 24 AES blocks per chunk (set after a chunk needed them)
+    int full = 0;  // scan a chunk past its default AES blocks (set after one needed it)
     long long tiles = 0, chunks = 0, full_chunks = 0, nfirst = 0;
     long long map_words = 0;  // of the walk's maps of the compact streams
     int max_chunks = 0;
+    int tile = 16;  // chunks per tile of the candidate pass
     std::vector<GaussStream> hs;
     std::vector<long long> tile_prefix, chunk_prefix, first_prefix;
     DevBuf<GaussStream> d_streams;

@@ -45,3 +45,22 @@ def test_streams_of_uneven_lengths_in_one_plan(gpu, po):
     got = gpu.encrypt(x, mpk, h(b"w2"), h(b"w3"), nonce0=4)
     for b in range(2):
         assert np.array_equal(got[b], po.encrypt(x[b], mpk, h(b"w2"), h(b"w3"), 4 + b))
+
+
+@pytest.mark.parametrize("variant", [{}, {"CUFE_AES_REP": "3"}, {"CUFE_GAUSS_WHOLE": "1"}])
+@pytest.mark.parametrize("nstreams,which,ncalls", [(1, 1, 1), (1, 2, 2), (3, 3, 5), (40, 2, 2), (5, 3, 90)])
+def test_tile_sizes_and_whole_words(gpu, po, monkeypatch, nstreams, which, ncalls, variant):
+    """From a few tiles of 16 chunks to several tiles of 64 a wave, with the
+    high words deciding and with every candidate from whole words (what a tie
+    of the high words takes), and the two-table layout."""
+    for k, v in variant.items():
+        monkeypatch.setenv(k, v)
+    print(f"[gpu-candidates] {nstreams} x S{which} x {ncalls} {variant}", flush=True)
+    keys = [h(b"t%d" % t) for t in range(nstreams)]
+    nonces = list(range(nstreams))
+    got = gpu.gauss_sample(keys, nonces, which, ncalls)
+    first = gpu.gauss_sample_first(keys, nonces, which, ncalls)
+    for t in {0, nstreams - 1}:
+        want = po.gauss_calls(keys[t], nonces[t], which, ncalls)
+        assert np.array_equal(got[t], want)
+        assert np.array_equal(first[t], want[:, :, 0])
