@@ -20,8 +20,9 @@ constexpr size_t kPoly = (size_t)3 * IPFE_N;  // words per [3][N] polynomial
 struct EventTimer {
     hipEvent_t a = nullptr, b = nullptr;
     hipStream_t st;
-    explicit EventTimer(hipStream_t s) : st(s)
+    explicit EventTimer(hipStream_t s, bool on = true) : st(s)
     {
+        if (!on) return;
         (void)hipEventCreate(&a);
         (void)hipEventCreate(&b);
         (void)hipEventRecord(a, st);
@@ -29,6 +30,7 @@ struct EventTimer {
     float stop()
     {
         float ms = 0;
+        if (!a) return ms;
         (void)hipEventRecord(b, st);
         (void)hipEventSynchronize(b);
         (void)hipEventElapsedTime(&ms, a, b);
@@ -95,11 +97,11 @@ int do_setup(uint32_t *mpk, uint32_t *msk, const unsigned char *seed2, const uns
     Device *dev = device();
     if (!dev) return -1;
     hipStream_t st = dev->stream;
-    EventTimer tm(st);
+    EventTimer tm(st, ms != nullptr);
     DevBuf<uint32_t> d_mpk, d_msk, d_e, d_ap;
     if (d_mpk.alloc((l + 1) * kPoly) || d_msk.alloc(l * kPoly) || d_e.alloc(l * kPoly) || d_ap.alloc(kPoly)) return -1;
     uint32_t *d_ahat = d_mpk.get() + (size_t)l * kPoly;
-    HIP_OK(hipMemcpyAsync(d_ahat, mpk + (size_t)l * kPoly, kPoly * 4, hipMemcpyHostToDevice, st));
+    if (copy_to_device(d_ahat, mpk + (size_t)l * kPoly, kPoly * 4, st)) return -1;
     if (launch_ntt_fwd(d_ahat, d_ahat, 3, dev->tw_all, st)) return -1;
     if (launch_shoup_prep(d_ahat, d_ap.get(), kPoly, st)) return -1;
     std::vector<StreamReq> reqs;
@@ -107,8 +109,8 @@ int do_setup(uint32_t *mpk, uint32_t *msk, const unsigned char *seed2, const uns
     reqs.push_back(make_stream(seed3, 0, 1, l, d_e.get(), d_e.get() + kPoly, (long long)kPoly));
     if (run_gauss(reqs, st)) return -1;
     if (launch_setup_pk(d_msk.get(), d_e.get(), d_ahat, d_ap.get(), d_mpk.get(), l, dev->tw_all, st)) return -1;
-    HIP_OK(hipMemcpyAsync(mpk, d_mpk.get(), (l + 1) * kPoly * 4, hipMemcpyDeviceToHost, st));
-    HIP_OK(hipMemcpyAsync(msk, d_msk.get(), l * kPoly * 4, hipMemcpyDeviceToHost, st));
+    if (copy_to_host(mpk, d_mpk.get(), (l + 1) * kPoly * 4, st)) return -1;
+    if (copy_to_host(msk, d_msk.get(), l * kPoly * 4, st)) return -1;
     float e = tm.stop();
     if (ms) *ms += e;
     return sync_stream(st);
@@ -126,10 +128,10 @@ int do_encrypt(const uint32_t *m, const uint32_t *mpk, uint32_t *c, const unsign
         return -1;
     }
     hipStream_t st = dev->stream;
-    EventTimer tm(st);
+    EventTimer tm(st, ms != nullptr);
     DevBuf<uint32_t> d_mpk;
     if (d_mpk.alloc((l + 1) * kPoly)) return -1;
-    HIP_OK(hipMemcpyAsync(d_mpk.get(), mpk, (l + 1) * kPoly * 4, hipMemcpyHostToDevice, st));
+    if (copy_to_device(d_mpk.get(), mpk, (l + 1) * kPoly * 4, st)) return -1;
     const size_t ct_words = (size_t)(l + 1) * kPoly;
     // messages per group: bound ciphertext + sampler scratch to ~16 GiB
     const size_t per_msg = ct_words * 4 + gauss_bytes(3, l, 0) + gauss_bytes(2, 2, 0) + 2 * kPoly * 4;
@@ -143,7 +145,7 @@ int do_encrypt(const uint32_t *m, const uint32_t *mpk, uint32_t *c, const unsign
             d_rp.alloc((size_t)g * kPoly) || d_msgs.alloc(g) || d_items.alloc((size_t)g * (l + 1)))
             return -1;
         if (l > 0)
-            HIP_OK(hipMemcpyAsync(d_x.get(), m + (size_t)b0 * l, (size_t)g * l * 4, hipMemcpyHostToDevice, st));
+            if (copy_to_device(d_x.get(), m + (size_t)b0 * l, (size_t)g * l * 4, st)) return -1;
         std::vector<StreamReq> reqs;
         std::vector<EncMsg> msgs(g);
         std::vector<EncItem> items;
@@ -169,7 +171,7 @@ int do_encrypt(const uint32_t *m, const uint32_t *mpk, uint32_t *c, const unsign
         if (launch_enc_poly(d_items.get(), (int)items.size(), d_msgs.get(), d_mpk.get(), l, dev->tw_all, dev->ninv,
                             dev->scale, st))
             return -1;
-        HIP_OK(hipMemcpyAsync(c + (size_t)b0 * ct_words, d_c.get(), (size_t)g * ct_words * 4, hipMemcpyDeviceToHost, st));
+        if (copy_to_host(c + (size_t)b0 * ct_words, d_c.get(), (size_t)g * ct_words * 4, st)) return -1;
         if (sync_stream(st)) return -1;
     }
     float e = tm.stop();
@@ -182,17 +184,35 @@ int do_keygen(const uint32_t *y, const uint32_t *msk, uint32_t *sk, int repeat, 
     Device *dev = device();
     if (!dev) return -1;
     hipStream_t st = dev->stream;
-    EventTimer tm(st);
+    EventTimer tm(st, ms != nullptr);
     HostSparse hsp = to_sparse(y, repeat, l);
     DevSparse dsp;
     DevBuf<uint32_t> d_msk, d_sk;
     if (dsp.upload(hsp, l, st) || d_msk.alloc((size_t)l * kPoly + 1) || d_sk.alloc((size_t)repeat * kPoly)) return -1;
-    if (l > 0) HIP_OK(hipMemcpyAsync(d_msk.get(), msk, (size_t)l * kPoly * 4, hipMemcpyHostToDevice, st));
+    if (l > 0 && copy_to_device(d_msk.get(), msk, (size_t)l * kPoly * 4, st)) return -1;
     if (launch_keygen(dsp.view, repeat, d_msk.get(), d_sk.get(), st)) return -1;
-    HIP_OK(hipMemcpyAsync(sk, d_sk.get(), (size_t)repeat * kPoly * 4, hipMemcpyDeviceToHost, st));
+    if (copy_to_host(sk, d_sk.get(), (size_t)repeat * kPoly * 4, st)) return -1;
     float e = tm.stop();
     if (ms) *ms += e;
     return sync_stream(st);
+}
+
+// Decryption of c [l+1][3][N] under `repeat` keys, on the device: d [repeat][3][N].
+// c's last polynomial and sk are transformed in place.
+int decrypt_dev(const SparseY &y, uint32_t *c, uint32_t *sk, uint32_t *d, int repeat, int l, Device *dev,
+                hipStream_t st)
+{
+    DevBuf<uint32_t> d_chat;
+    if (d_chat.alloc((size_t)repeat * kPoly)) return -1;
+    if (launch_dec_sum(y, repeat, c, d, st)) return -1;
+    // poly_mul_ntt(c_L, sk) (src/ntt.c:10-26): NTT both, pointwise, INTT
+    if (launch_ntt_fwd(c + (size_t)l * kPoly, d_chat.get(), 3, dev->tw_all, st)) return -1;
+    if (launch_ntt_fwd(sk, sk, repeat * 3, dev->tw_all, st)) return -1;
+    for (int v = 1; v < repeat; ++v)
+        HIP_OK(hipMemcpyAsync(d_chat.get() + (size_t)v * kPoly, d_chat.get(), kPoly * 4, hipMemcpyDeviceToDevice, st));
+    if (launch_point_mul(d_chat.get(), sk, sk, (size_t)repeat * kPoly, dev->barrett, st)) return -1;
+    if (launch_ntt_inv(sk, sk, repeat * 3, dev->tw_all, dev->ninv, st)) return -1;
+    return launch_poly_sub(d, sk, (size_t)repeat * kPoly, st);
 }
 
 // One ciphertext c [l+1][3][N] against `repeat` keys -> d_y [repeat][3][N].
@@ -201,28 +221,42 @@ int do_decrypt(const uint32_t *c, const uint32_t *y, const uint32_t *sk, uint32_
     Device *dev = device();
     if (!dev) return -1;
     hipStream_t st = dev->stream;
-    EventTimer tm(st);
+    EventTimer tm(st, ms != nullptr);
     HostSparse hsp = to_sparse(y, repeat, l);
     DevSparse dsp;
-    DevBuf<uint32_t> d_c, d_sk, d_d, d_chat, d_prod;
+    DevBuf<uint32_t> d_c, d_sk, d_d;
     if (dsp.upload(hsp, l, st) || d_c.alloc((size_t)(l + 1) * kPoly) || d_sk.alloc((size_t)repeat * kPoly) ||
-        d_d.alloc((size_t)repeat * kPoly) || d_chat.alloc((size_t)repeat * kPoly) ||
-        d_prod.alloc((size_t)repeat * kPoly))
+        d_d.alloc((size_t)repeat * kPoly))
         return -1;
-    HIP_OK(hipMemcpyAsync(d_c.get(), c, (size_t)(l + 1) * kPoly * 4, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(d_sk.get(), sk, (size_t)repeat * kPoly * 4, hipMemcpyHostToDevice, st));
-    if (launch_dec_sum(dsp.view, repeat, d_c.get(), d_d.get(), st)) return -1;
-    // poly_mul_ntt(c_L, sk) (src/ntt.c:10-26): NTT both, pointwise, INTT
-    if (launch_ntt_fwd(d_c.get() + (size_t)l * kPoly, d_chat.get(), 3, dev->tw_all, st)) return -1;
-    if (launch_ntt_fwd(d_sk.get(), d_prod.get(), repeat * 3, dev->tw_all, st)) return -1;
-    for (int v = 1; v < repeat; ++v)
-        HIP_OK(hipMemcpyAsync(d_chat.get() + (size_t)v * kPoly, d_chat.get(), kPoly * 4, hipMemcpyDeviceToDevice, st));
-    if (launch_point_mul(d_chat.get(), d_prod.get(), d_prod.get(), (size_t)repeat * kPoly, dev->barrett, st)) return -1;
-    if (launch_ntt_inv(d_prod.get(), d_prod.get(), repeat * 3, dev->tw_all, dev->ninv, st)) return -1;
-    if (launch_poly_sub(d_d.get(), d_prod.get(), (size_t)repeat * kPoly, st)) return -1;
-    HIP_OK(hipMemcpyAsync(d, d_d.get(), (size_t)repeat * kPoly * 4, hipMemcpyDeviceToHost, st));
+    if (copy_to_device(d_c.get(), c, (size_t)(l + 1) * kPoly * 4, st)) return -1;
+    if (copy_to_device(d_sk.get(), sk, (size_t)repeat * kPoly * 4, st)) return -1;
+    if (decrypt_dev(dsp.view, d_c.get(), d_sk.get(), d_d.get(), repeat, l, dev, st)) return -1;
+    if (copy_to_host(d, d_d.get(), (size_t)repeat * kPoly * 4, st)) return -1;
     float e = tm.stop();
     if (ms) *ms += e;
+    return sync_stream(st);
+}
+
+// Key values of one ciphertext c [L+1][3][N] under the keys of `n` vectors y
+// [n][L]: key generation, decryption and the rounding of coefficient 0, with
+// the keys and the decryptions kept on the device.
+int do_kvalues(const uint32_t *c, const uint32_t *y, const uint32_t *msk, uint32_t *kv, int n)
+{
+    Device *dev = device();
+    if (!dev) return -1;
+    hipStream_t st = dev->stream;
+    HostSparse hsp = to_sparse(y, n, IPFE_L);
+    DevSparse dsp;
+    DevBuf<uint32_t> d_msk, d_c, d_sk, d_d, d_kv;
+    if (dsp.upload(hsp, IPFE_L, st) || d_msk.alloc(IPFE_L * kPoly) || d_c.alloc((IPFE_L + 1) * kPoly) ||
+        d_sk.alloc((size_t)n * kPoly) || d_d.alloc((size_t)n * kPoly) || d_kv.alloc(n))
+        return -1;
+    if (copy_to_device(d_msk.get(), msk, IPFE_L * kPoly * 4, st)) return -1;
+    if (launch_keygen(dsp.view, n, d_msk.get(), d_sk.get(), st)) return -1;
+    if (copy_to_device(d_c.get(), c, (IPFE_L + 1) * kPoly * 4, st)) return -1;
+    if (decrypt_dev(dsp.view, d_c.get(), d_sk.get(), d_d.get(), n, IPFE_L, dev, st)) return -1;
+    if (launch_crt_round(d_d.get(), n, 0, d_kv.get(), st)) return -1;
+    HIP_OK(hipMemcpyAsync(kv, d_kv.get(), (size_t)n * 4, hipMemcpyDeviceToHost, st));
     return sync_stream(st);
 }
 
@@ -271,7 +305,7 @@ extern "C" int cufe_sample_polya(const unsigned char seed[32], uint32_t *a)
     if (d_rk.alloc(60) || d_a.alloc(kPoly)) return -1;
     HIP_OK(hipMemcpyAsync(d_rk.get(), rk, sizeof rk, hipMemcpyHostToDevice, st));
     if (launch_sample_polya(d_rk.get(), d_a.get(), st)) return -1;
-    HIP_OK(hipMemcpyAsync(a, d_a.get(), kPoly * 4, hipMemcpyDeviceToHost, st));
+    if (copy_to_host(a, d_a.get(), kPoly * 4, st)) return -1;
     return sync_stream(st);
 }
 
@@ -290,26 +324,18 @@ extern "C" double cufe_svm_predict_gpu(const cufe_svm_model *model,
         return std::nan("");
     }
     const int l = model->l;
-    std::vector<uint32_t> sk((size_t)l * kPoly), dy((size_t)l * kPoly);
-    // the steps of rlwe_sife_keygen_gpu and rlwe_sife_decrypt_gmp_gpu, with
-    // their status checked: a failed device call yields NaN, never a label
-    // voted from unwritten key values
-    if (do_keygen(model->sv, &msk[0][0][0], sk.data(), l, IPFE_L, nullptr) ||
-        do_decrypt(&c[0][0][0], model->sv, sk.data(), dy.data(), l, IPFE_L, nullptr)) {
+    // the steps of rlwe_sife_keygen_gpu and rlwe_sife_decrypt_gmp_gpu and the
+    // rounding of the one coefficient that round_extract_gmp2 keeps, with their
+    // status checked: a failed device call yields NaN, never a label voted from
+    // unwritten key values
+    std::vector<uint32_t> rounded(l);
+    if (do_kvalues(&c[0][0][0], model->sv, &msk[0][0][0], rounded.data(), l)) {
         report("cufe_svm_predict_gpu");
         if (kvalue)
             for (int i = 0; i < l; ++i) kvalue[i] = std::nan("");
         return std::nan("");
     }
-    std::vector<double> kv(l);
-    for (int i = 0; i < l; ++i) {
-        // round_extract_gmp2 reconstructs every coefficient and keeps only the first
-        for (int k = 0; k < IPFE_N; ++k) {
-            const uint32_t *dk = dy.data() + (size_t)i * kPoly + k;
-            uint32_t r = crt_decode(dk[0], dk[IPFE_N], dk[2 * IPFE_N]);
-            if (k == 0) kv[i] = (double)r;
-        }
-    }
+    std::vector<double> kv(rounded.begin(), rounded.end());
     if (kvalue) memcpy(kvalue, kv.data(), sizeof(double) * l);
     // one-vs-one vote (main.c:338-389)
     const int nr = model->nr_class;
@@ -356,10 +382,10 @@ extern "C" int cufe_ntt_forward(uint32_t *polys, int npoly)
     hipStream_t st = dev->stream;
     DevBuf<uint32_t> d;
     if (d.alloc((size_t)npoly * kPoly)) return -1;
-    HIP_OK(hipMemcpyAsync(d.get(), polys, (size_t)npoly * kPoly * 4, hipMemcpyHostToDevice, st));
+    if (copy_to_device(d.get(), polys, (size_t)npoly * kPoly * 4, st)) return -1;
     const PsetState *ps = pset_state(1);  // the reference set, tuned transform shape
     if (!ps || ps_ntt(*ps, false, d.get(), d.get(), npoly * 3, st)) return -1;
-    HIP_OK(hipMemcpyAsync(polys, d.get(), (size_t)npoly * kPoly * 4, hipMemcpyDeviceToHost, st));
+    if (copy_to_host(polys, d.get(), (size_t)npoly * kPoly * 4, st)) return -1;
     return sync_stream(st);
 }
 
@@ -370,10 +396,10 @@ extern "C" int cufe_ntt_inverse(uint32_t *polys, int npoly)
     hipStream_t st = dev->stream;
     DevBuf<uint32_t> d;
     if (d.alloc((size_t)npoly * kPoly)) return -1;
-    HIP_OK(hipMemcpyAsync(d.get(), polys, (size_t)npoly * kPoly * 4, hipMemcpyHostToDevice, st));
+    if (copy_to_device(d.get(), polys, (size_t)npoly * kPoly * 4, st)) return -1;
     const PsetState *ps = pset_state(1);
     if (!ps || ps_ntt(*ps, true, d.get(), d.get(), npoly * 3, st)) return -1;
-    HIP_OK(hipMemcpyAsync(polys, d.get(), (size_t)npoly * kPoly * 4, hipMemcpyDeviceToHost, st));
+    if (copy_to_host(polys, d.get(), (size_t)npoly * kPoly * 4, st)) return -1;
     return sync_stream(st);
 }
 
@@ -397,7 +423,7 @@ extern "C" int cufe_gauss_sample(const unsigned char *keys, const uint16_t *nonc
         reqs.push_back(make_stream(keys + 32 * (size_t)t, nonces[t], which, ncalls, o, o + kPoly, (long long)kPoly));
     }
     if (run_gauss(reqs, st)) return -1;
-    HIP_OK(hipMemcpyAsync(out, d.get(), (size_t)nstreams * per_stream * 4, hipMemcpyDeviceToHost, st));
+    if (copy_to_host(out, d.get(), (size_t)nstreams * per_stream * 4, st)) return -1;
     return sync_stream(st);
 }
 
@@ -421,7 +447,7 @@ extern "C" int cufe_gauss_sample_first(const unsigned char *keys, const uint16_t
         reqs.push_back(make_stream(keys + 32 * (size_t)t, nonces[t], which, ncalls, d.get() + (size_t)t * per_stream,
                                    nullptr, 0, 1));
     if (run_gauss(reqs, st)) return -1;
-    HIP_OK(hipMemcpyAsync(out, d.get(), (size_t)nstreams * per_stream * 4, hipMemcpyDeviceToHost, st));
+    if (copy_to_host(out, d.get(), (size_t)nstreams * per_stream * 4, st)) return -1;
     return sync_stream(st);
 }
 
@@ -453,7 +479,7 @@ extern "C" int cufe_crt_round(const uint32_t *d, int nvec, int coef, uint32_t *r
     hipStream_t st = dev->stream;
     DevBuf<uint32_t> d_d, d_r;
     if (d_d.alloc((size_t)nvec * kPoly) || d_r.alloc((size_t)nvec + 1)) return -1;
-    HIP_OK(hipMemcpyAsync(d_d.get(), d, (size_t)nvec * kPoly * 4, hipMemcpyHostToDevice, st));
+    if (copy_to_device(d_d.get(), d, (size_t)nvec * kPoly * 4, st)) return -1;
     if (launch_crt_round(d_d.get(), nvec, coef, d_r.get(), st)) return -1;
     HIP_OK(hipMemcpyAsync(r, d_r.get(), (size_t)nvec * 4, hipMemcpyDeviceToHost, st));
     return sync_stream(st);

@@ -283,8 +283,8 @@ extern "C" int cufe_encbatch_export(const cufe_encbatch *eb, int b0, int nb, uin
     }
     if (nb == 0) return 0;
     const size_t end = (b0 + nb < eb->n) ? eb->coff[b0 + nb] : eb->c_words;
-    HIP_OK(hipMemcpy(c, eb->d_c.get() + eb->coff[b0], (end - eb->coff[b0]) * 4, hipMemcpyDeviceToHost));
-    return 0;
+    if (copy_to_host(c, eb->d_c.get() + eb->coff[b0], (end - eb->coff[b0]) * 4, eb->st)) return -1;
+    return sync_stream(eb->st);
 }
 
 // Position-weighted 64-bit checksum of every ciphertext word of the batch,

@@ -622,6 +622,29 @@ int launch_contract_sgpr(const double *A, const double *B, int R, int S, int K, 
     return 0;
 }
 
+// c_L of rows [r0, r0 + n) of the balanced store [3][cap][ldr] as canonical
+// words [n][3][N], four columns a thread (ldr is a multiple of 16).
+__global__ void k_rows_export(const int32_t *__restrict__ a, int cap, int ldr, int r0, int n,
+                              uint32_t *__restrict__ cl)
+{
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (size_t)n * 3 * (IPFE_N / 4)) return;
+    const int j = 4 * (int)(i % (IPFE_N / 4)), s = (int)(i / (IPFE_N / 4) % 3), r = (int)(i / (3 * (IPFE_N / 4)));
+    const int4 v = *reinterpret_cast<const int4 *>(a + ((size_t)s * cap + r0 + r) * ldr + j);
+    const uint32_t q = qmod(s);
+    auto canon = [q](int x) { return (uint32_t)x + (x < 0 ? q : 0u); };
+    *reinterpret_cast<uint4 *>(cl + 4 * i) = make_uint4(canon(v.x), canon(v.y), canon(v.z), canon(v.w));
+}
+
+int launch_rows_export(const int32_t *a, int cap, int ldr, int r0, int n, uint32_t *cl, hipStream_t st)
+{
+    const size_t quads = (size_t)n * 3 * (IPFE_N / 4);
+    if (quads == 0) return 0;
+    hipLaunchKernelGGL(k_rows_export, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, a, cap, ldr, r0, n, cl);
+    HIP_OK(hipGetLastError());
+    return 0;
+}
+
 int launch_rows_blocked(const int32_t *a32, int cap, int cap64, int ldr, int r0, int R, double *a64, hipStream_t st)
 {
     const size_t n = (size_t)3 * R * ldr;

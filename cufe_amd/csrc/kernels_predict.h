@@ -98,6 +98,7 @@ int launch_frac_exact(const int32_t *A, size_t limb_stride, int ldr, const int16
 int frac_variant_count();
 void frac_shape(int variant, int *wr, int *wk);
 const char *frac_variant_label(int variant);
+int launch_rows_export(const int32_t *a, int cap, int ldr, int r0, int n, uint32_t *cl, hipStream_t st);
 int launch_rows_blocked(const int32_t *a32, int cap, int cap64, int ldr, int r0, int R, double *a64, hipStream_t st);
 int launch_crt_kvalue(const uint32_t *D, size_t n, uint32_t *kval, hipStream_t st);
 int launch_kvalue(const uint32_t *D, const uint32_t *c0, int l, const SparseY &y, int R, int S, uint32_t *kval,

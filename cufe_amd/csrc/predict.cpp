@@ -573,9 +573,9 @@ int predict_rows(const Model &m, const RowStore &rs, int row0, int nrows, Scratc
         if (labels_host)
             HIP_OK(hipMemcpyAsync(labels_host + (r0 - row0), sc.labels.get(), sizeof(double) * R,
                                   hipMemcpyDeviceToHost, st));
-        if (kval_host)
-            HIP_OK(hipMemcpyAsync(kval_host + (size_t)(r0 - row0) * S, sc.kval.get(), sizeof(uint32_t) * R * S,
-                                  hipMemcpyDeviceToHost, st));
+        if (kval_host &&
+            copy_to_host(kval_host + (size_t)(r0 - row0) * S, sc.kval.get(), sizeof(uint32_t) * R * S, st))
+            return -1;
         if (r0 + chunk < row0 + nrows) {
             // the scratch is reused by the next chunk: wait for this one
             HIP_OK(hipStreamSynchronize(st));
@@ -735,8 +735,10 @@ extern "C" int cufe_ctx_load_keys(cufe_ctx *c, const uint32_t *mpk, const uint32
     }
     if (!device()) return -1;
     if (c->mpk.alloc((size_t)(l + 1) * kPoly) || c->msk.alloc((size_t)l * kPoly)) return -1;
-    HIP_OK(hipMemcpy(c->mpk.get(), mpk, (size_t)(l + 1) * kPoly * 4, hipMemcpyHostToDevice));
-    HIP_OK(hipMemcpy(c->msk.get(), msk, (size_t)l * kPoly * 4, hipMemcpyHostToDevice));
+    hipStream_t st = device()->stream;
+    if (copy_to_device(c->mpk.get(), mpk, (size_t)(l + 1) * kPoly * 4, st) ||
+        copy_to_device(c->msk.get(), msk, (size_t)l * kPoly * 4, st) || sync_stream(st))
+        return -1;
     c->l_key = l;
     c->model.S = 0;
     return 0;
@@ -780,9 +782,10 @@ extern "C" int cufe_ctx_get_keys(cufe_ctx *c, uint32_t *mpk, uint32_t *msk)
         ipfe_set_error("cufe_ctx_get_keys: no keys in context");
         return -1;
     }
-    if (mpk) HIP_OK(hipMemcpy(mpk, c->mpk.get(), (size_t)(c->l_key + 1) * kPoly * 4, hipMemcpyDeviceToHost));
-    if (msk) HIP_OK(hipMemcpy(msk, c->msk.get(), (size_t)c->l_key * kPoly * 4, hipMemcpyDeviceToHost));
-    return 0;
+    hipStream_t st = device()->stream;
+    if (mpk && copy_to_host(mpk, c->mpk.get(), (size_t)(c->l_key + 1) * kPoly * 4, st)) return -1;
+    if (msk && copy_to_host(msk, c->msk.get(), (size_t)c->l_key * kPoly * 4, st)) return -1;
+    return sync_stream(st);
 }
 
 // Functional keys of every support vector, generated on the device and kept.
@@ -981,8 +984,9 @@ extern "C" int cufe_ctx_get_model_keys(const cufe_ctx *c, uint32_t *sk)
         ipfe_set_error("cufe_ctx_get_model_keys: no model");
         return -1;
     }
-    HIP_OK(hipMemcpy(sk, c->model.sk.get(), (size_t)c->model.S * kPoly * 4, hipMemcpyDeviceToHost));
-    return 0;
+    hipStream_t st = device()->stream;
+    if (copy_to_host(sk, c->model.sk.get(), (size_t)c->model.S * kPoly * 4, st)) return -1;
+    return sync_stream(st);
 }
 
 // Stored compact ciphertexts of rows [row0, row0+n): c_L [n][3][N] canonical
@@ -994,18 +998,19 @@ extern "C" int cufe_ctx_export_rows(const cufe_ctx *c, int row0, int n, uint32_t
         return -1;
     }
     const RowStore &rs = c->rows;
-    std::vector<int32_t> a((size_t)n * rs.ldr);
-    for (int s = 0; s < 3; ++s) {
-        HIP_OK(hipMemcpy(a.data(), rs.A.get() + ((size_t)s * rs.cap + row0) * rs.ldr, (size_t)n * rs.ldr * 4,
-                         hipMemcpyDeviceToHost));
-        for (int r = 0; r < n; ++r) {
-            uint32_t *dst = cl + ((size_t)r * 3 + s) * IPFE_N;
-            const int32_t *src = a.data() + (size_t)r * rs.ldr;
-            for (int j = 0; j < IPFE_N; ++j) dst[j] = (uint32_t)(src[j] < 0 ? (int64_t)src[j] + qmod(s) : src[j]);
-        }
+    hipStream_t st = device()->stream;
+    // canonical words in blocks of rows, so that the copy out is one
+    constexpr int kBlock = 4096;
+    DevBuf<uint32_t> out;
+    if (out.alloc((size_t)std::min(n, kBlock) * kPoly)) return -1;
+    for (int r = 0; r < n; r += kBlock) {
+        const int k = std::min(kBlock, n - r);
+        if (launch_rows_export(rs.A.get(), rs.cap, rs.ldr, row0 + r, k, out.get(), st) ||
+            copy_to_host(cl + (size_t)r * kPoly, out.get(), (size_t)k * kPoly * 4, st) || sync_stream(st))
+            return -1;
     }
-    HIP_OK(hipMemcpy(c0, rs.c0.get() + (size_t)row0 * rs.l * 3, (size_t)n * rs.l * 3 * 4, hipMemcpyDeviceToHost));
-    return 0;
+    if (copy_to_host(c0, rs.c0.get() + (size_t)row0 * rs.l * 3, (size_t)n * rs.l * 3 * 4, st)) return -1;
+    return sync_stream(st);
 }
 
 extern "C" int cufe_ctx_get_row(const cufe_ctx *c, int row, uint32_t *cl, uint32_t *c0)

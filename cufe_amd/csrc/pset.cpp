@@ -230,7 +230,7 @@ static int ps_ntt_host(int pset, int inverse, int variant, uint32_t *polys, int 
     const size_t words = (size_t)npoly * poly_words(*st);
     DevBuf<uint32_t> d;
     if (d.alloc(words)) return -1;
-    HIP_OK(hipMemcpyAsync(d.get(), polys, words * 4, hipMemcpyHostToDevice, s));
+    if (copy_to_device(d.get(), polys, words * 4, s)) return -1;
     const int ntrans = npoly * st->dev.nmod;
     if (variant < 0) {
         if (ps_ntt(*st, inverse != 0, d.get(), d.get(), ntrans, s)) return -1;
@@ -238,7 +238,7 @@ static int ps_ntt_host(int pset, int inverse, int variant, uint32_t *polys, int 
                                pset == 1, s)) {
         return -1;
     }
-    HIP_OK(hipMemcpyAsync(polys, d.get(), words * 4, hipMemcpyDeviceToHost, s));
+    if (copy_to_host(polys, d.get(), words * 4, s)) return -1;
     return sync_stream(s);
 }
 
@@ -292,7 +292,7 @@ extern "C" int cufe_ps_sample_polya(int pset, const unsigned char seed[32], uint
     if (d_rk.alloc(60) || d_a.alloc(poly_words(*st))) return -1;
     HIP_OK(hipMemcpyAsync(d_rk.get(), rk, sizeof rk, hipMemcpyHostToDevice, s));
     if (launch_sample_polya_ps(d_rk.get(), d_a.get(), st->dev.N, st->dev.nmod, st->dev.q, s)) return -1;
-    HIP_OK(hipMemcpyAsync(a, d_a.get(), poly_words(*st) * 4, hipMemcpyDeviceToHost, s));
+    if (copy_to_host(a, d_a.get(), poly_words(*st) * 4, s)) return -1;
     return sync_stream(s);
 }
 
@@ -327,7 +327,7 @@ extern "C" int cufe_ps_gauss_sample(int pset, const unsigned char *keys, const u
     DevBuf<uint32_t> d;
     if (d.alloc(words)) return -1;
     if (ps_gauss_dev(*st, keys, nonces, nstreams, which, ncalls, d.get(), s)) return -1;
-    HIP_OK(hipMemcpyAsync(out, d.get(), words * 4, hipMemcpyDeviceToHost, s));
+    if (copy_to_host(out, d.get(), words * 4, s)) return -1;
     return sync_stream(s);
 }
 
@@ -349,7 +349,7 @@ extern "C" int cufe_ps_setup(int pset, uint32_t *mpk, uint32_t *msk, const unsig
         d_ap.alloc(pw))
         return -1;
     uint32_t *ahat = d_mpk.get() + (size_t)l * pw;
-    HIP_OK(hipMemcpyAsync(ahat, mpk + (size_t)l * pw, pw * 4, hipMemcpyHostToDevice, s));
+    if (copy_to_device(ahat, mpk + (size_t)l * pw, pw * 4, s)) return -1;
     if (ps_ntt(*st, false, ahat, ahat, st->dev.nmod, s) || ps_launch_shoup(*st, ahat, d_ap.get(), pw, s)) return -1;
     const uint16_t zero = 0;
     const PsetSpec &sp = *pset_spec(pset);
@@ -358,8 +358,8 @@ extern "C" int cufe_ps_setup(int pset, uint32_t *mpk, uint32_t *msk, const unsig
     reqs.push_back(make_stream_ps(sp, seed3, zero, 1, l, d_e.get(), d_e.get() + pw, (long long)pw));
     if (run_gauss(reqs, s)) return -1;
     if (ps_launch_setup_pk(*st, d_msk.get(), d_e.get(), ahat, d_ap.get(), d_mpk.get(), l, s)) return -1;
-    HIP_OK(hipMemcpyAsync(mpk, d_mpk.get(), (size_t)(l + 1) * pw * 4, hipMemcpyDeviceToHost, s));
-    HIP_OK(hipMemcpyAsync(msk, d_msk.get(), (size_t)l * pw * 4, hipMemcpyDeviceToHost, s));
+    if (copy_to_host(mpk, d_mpk.get(), (size_t)(l + 1) * pw * 4, s)) return -1;
+    if (copy_to_host(msk, d_msk.get(), (size_t)l * pw * 4, s)) return -1;
     return sync_stream(s);
 }
 
@@ -382,8 +382,8 @@ extern "C" int cufe_ps_encrypt(int pset, const uint32_t *m, const uint32_t *mpk,
     if (d_mpk.alloc((size_t)(l + 1) * pw) || d_c.alloc((size_t)repeat * ct) || d_r.alloc((size_t)repeat * pw) ||
         d_rp.alloc((size_t)repeat * pw) || d_x.alloc((size_t)repeat * l + 1))
         return -1;
-    HIP_OK(hipMemcpyAsync(d_mpk.get(), mpk, (size_t)(l + 1) * pw * 4, hipMemcpyHostToDevice, s));
-    if (l > 0) HIP_OK(hipMemcpyAsync(d_x.get(), m, (size_t)repeat * l * 4, hipMemcpyHostToDevice, s));
+    if (copy_to_device(d_mpk.get(), mpk, (size_t)(l + 1) * pw * 4, s)) return -1;
+    if (l > 0 && copy_to_device(d_x.get(), m, (size_t)repeat * l * 4, s)) return -1;
     const PsetSpec &sp = *pset_spec(pset);
     std::vector<StreamReq> reqs;
     for (int b = 0; b < repeat; ++b) {
@@ -398,7 +398,7 @@ extern "C" int cufe_ps_encrypt(int pset, const uint32_t *m, const uint32_t *mpk,
         ps_launch_shoup(*st, d_r.get(), d_rp.get(), (size_t)repeat * pw, s) ||
         ps_launch_enc_poly(*st, d_mpk.get(), d_r.get(), d_rp.get(), d_x.get(), d_c.get(), repeat, l, s))
         return -1;
-    HIP_OK(hipMemcpyAsync(c, d_c.get(), (size_t)repeat * ct * 4, hipMemcpyDeviceToHost, s));
+    if (copy_to_host(c, d_c.get(), (size_t)repeat * ct * 4, s)) return -1;
     return sync_stream(s);
 }
 
@@ -416,10 +416,10 @@ extern "C" int cufe_ps_keygen(int pset, const uint32_t *y, const uint32_t *msk, 
     const size_t pw = poly_words(*st);
     DevBuf<uint32_t> d_y, d_msk, d_sk;
     if (d_y.alloc((size_t)repeat * l) || d_msk.alloc((size_t)l * pw) || d_sk.alloc((size_t)repeat * pw)) return -1;
-    HIP_OK(hipMemcpyAsync(d_y.get(), y, (size_t)repeat * l * 4, hipMemcpyHostToDevice, s));
-    HIP_OK(hipMemcpyAsync(d_msk.get(), msk, (size_t)l * pw * 4, hipMemcpyHostToDevice, s));
+    if (copy_to_device(d_y.get(), y, (size_t)repeat * l * 4, s)) return -1;
+    if (copy_to_device(d_msk.get(), msk, (size_t)l * pw * 4, s)) return -1;
     if (ps_launch_fold(*st, d_y.get(), repeat, l, d_msk.get(), d_sk.get(), s)) return -1;
-    HIP_OK(hipMemcpyAsync(sk, d_sk.get(), (size_t)repeat * pw * 4, hipMemcpyDeviceToHost, s));
+    if (copy_to_host(sk, d_sk.get(), (size_t)repeat * pw * 4, s)) return -1;
     return sync_stream(s);
 }
 
@@ -441,9 +441,9 @@ extern "C" int cufe_ps_decrypt(int pset, const uint32_t *c, const uint32_t *y, c
     if (d_c.alloc((size_t)(l + 1) * pw) || d_y.alloc((size_t)repeat * l) || d_sk.alloc(nk) || d_d.alloc(nk) ||
         d_cl.alloc(nk))
         return -1;
-    HIP_OK(hipMemcpyAsync(d_c.get(), c, (size_t)(l + 1) * pw * 4, hipMemcpyHostToDevice, s));
-    HIP_OK(hipMemcpyAsync(d_y.get(), y, (size_t)repeat * l * 4, hipMemcpyHostToDevice, s));
-    HIP_OK(hipMemcpyAsync(d_sk.get(), sk, nk * 4, hipMemcpyHostToDevice, s));
+    if (copy_to_device(d_c.get(), c, (size_t)(l + 1) * pw * 4, s)) return -1;
+    if (copy_to_device(d_y.get(), y, (size_t)repeat * l * 4, s)) return -1;
+    if (copy_to_device(d_sk.get(), sk, nk * 4, s)) return -1;
     // sum part: fold over the l slots
     if (ps_launch_fold(*st, d_y.get(), repeat, l, d_c.get(), d_d.get(), s)) return -1;
     // poly_mul_ntt(c_L, sk_v) (src/ntt.c:10-26): NTT(c_L) once, copied per key
@@ -456,7 +456,7 @@ extern "C" int cufe_ps_decrypt(int pset, const uint32_t *c, const uint32_t *y, c
         ps_ntt(*st, true, d_cl.get(), d_cl.get(), repeat * st->dev.nmod, s) ||
         ps_launch_sub(*st, d_d.get(), d_cl.get(), nk, s))
         return -1;
-    HIP_OK(hipMemcpyAsync(d, d_d.get(), nk * 4, hipMemcpyDeviceToHost, s));
+    if (copy_to_host(d, d_d.get(), nk * 4, s)) return -1;
     return sync_stream(s);
 }
 
@@ -475,9 +475,9 @@ extern "C" int cufe_ps_crt_round(int pset, const uint32_t *d, int nvec, int coef
     const size_t nin = (size_t)nvec * poly_words(*st), nout = (size_t)nvec * (coef < 0 ? st->dev.N : 1);
     DevBuf<uint32_t> d_d, d_r;
     if (d_d.alloc(nin) || d_r.alloc(nout)) return -1;
-    HIP_OK(hipMemcpyAsync(d_d.get(), d, nin * 4, hipMemcpyHostToDevice, s));
+    if (copy_to_device(d_d.get(), d, nin * 4, s)) return -1;
     if (ps_launch_crt_round(*st, d_d.get(), nvec, coef, d_r.get(), s)) return -1;
-    HIP_OK(hipMemcpyAsync(r, d_r.get(), nout * 4, hipMemcpyDeviceToHost, s));
+    if (copy_to_host(r, d_r.get(), nout * 4, s)) return -1;
     return sync_stream(s);
 }
 

@@ -28,6 +28,20 @@ struct Device {
 // Initialises on first use; returns nullptr (error set) on failure.
 Device *device();
 
+// A device block of at least `bytes` bytes, uninitialised, and its release.
+// Released blocks are kept for the next allocation (xfer.cpp): bounded, from
+// any thread; a block is not handed out again before the device has finished
+// the work issued before its release.
+int dev_alloc(void **out, size_t bytes);
+void dev_free(void *p);
+
+// Copies between device memory and the caller's, after the work st holds; what
+// st is given later follows a copy_to_device.  Large copies to or from
+// pageable memory are done when they return; the others when st is (as
+// hipMemcpyAsync).  Not for a stream that is being captured.
+int copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t st);
+int copy_to_device(void *dst, const void *src, size_t bytes, hipStream_t st);
+
 template <typename T>
 struct DevBuf {
     T *p = nullptr;
@@ -38,7 +52,7 @@ struct DevBuf {
     ~DevBuf() { reset(); }
     void reset()
     {
-        if (p) (void)hipFree(p);
+        dev_free(p);
         p = nullptr;
         n = 0;
     }
@@ -46,12 +60,7 @@ struct DevBuf {
     {
         reset();
         if (count == 0) return 0;
-        hipError_t e = hipMalloc((void **)&p, count * sizeof(T));
-        if (e != hipSuccess) {
-            p = nullptr;
-            ipfe_set_error("hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
-            return -1;
-        }
+        if (dev_alloc((void **)&p, count * sizeof(T))) return -1;
         n = count;
         return 0;
     }
