@@ -52,6 +52,7 @@ void report(const char *fn)
 struct HostSparse {
     std::vector<int> off, idx;
     std::vector<uint32_t> val;
+    bool dense = false;
 };
 HostSparse to_sparse(const uint32_t *y, int n, int len)
 {
@@ -66,6 +67,9 @@ HostSparse to_sparse(const uint32_t *y, int n, int len)
             }
     }
     h.off[n] = (int)h.idx.size();
+    uint32_t max_y = 0;
+    for (uint32_t v : h.val) max_y = std::max(max_y, v);
+    h.dense = fold_dense((size_t)n, (size_t)len, h.idx.size(), max_y);
     if (h.idx.empty()) {  // keep device pointers valid
         h.idx.push_back(0);
         h.val.push_back(0);
@@ -77,8 +81,17 @@ struct DevSparse {
     DevBuf<int> off, idx;
     DevBuf<uint32_t> val;
     SparseY view{};
-    int upload(const HostSparse &h, int len, hipStream_t st)
+    // y [n][len]: the vectors h was made from
+    int upload(const HostSparse &h, const uint32_t *y, int n, int len, hipStream_t st)
     {
+        view.len = len;
+        if (h.dense) {
+            if (val.alloc((size_t)n * len + fold_packed_words(n, len))) return -1;
+            if (copy_to_device(val.get(), y, (size_t)n * len * 4, st)) return -1;
+            view.dense = val.get();
+            view.dense_packed = val.get() + (size_t)n * len;
+            return 0;
+        }
         if (off.alloc(h.off.size()) || idx.alloc(h.idx.size()) || val.alloc(h.val.size())) return -1;
         HIP_OK(hipMemcpyAsync(off.get(), h.off.data(), h.off.size() * 4, hipMemcpyHostToDevice, st));
         HIP_OK(hipMemcpyAsync(idx.get(), h.idx.data(), h.idx.size() * 4, hipMemcpyHostToDevice, st));
@@ -86,7 +99,6 @@ struct DevSparse {
         view.off = off.get();
         view.idx = idx.get();
         view.val = val.get();
-        view.len = len;
         return 0;
     }
 };
@@ -188,9 +200,9 @@ int do_keygen(const uint32_t *y, const uint32_t *msk, uint32_t *sk, int repeat, 
     HostSparse hsp = to_sparse(y, repeat, l);
     DevSparse dsp;
     DevBuf<uint32_t> d_msk, d_sk;
-    if (dsp.upload(hsp, l, st) || d_msk.alloc((size_t)l * kPoly + 1) || d_sk.alloc((size_t)repeat * kPoly)) return -1;
+    if (dsp.upload(hsp, y, repeat, l, st) || d_msk.alloc((size_t)l * kPoly + 1) || d_sk.alloc((size_t)repeat * kPoly)) return -1;
     if (l > 0 && copy_to_device(d_msk.get(), msk, (size_t)l * kPoly * 4, st)) return -1;
-    if (launch_keygen(dsp.view, repeat, d_msk.get(), d_sk.get(), st)) return -1;
+    if (launch_fold(dsp.view, repeat, d_msk.get(), d_sk.get(), dev->barrett, st)) return -1;
     if (copy_to_host(sk, d_sk.get(), (size_t)repeat * kPoly * 4, st)) return -1;
     float e = tm.stop();
     if (ms) *ms += e;
@@ -204,7 +216,7 @@ int decrypt_dev(const SparseY &y, uint32_t *c, uint32_t *sk, uint32_t *d, int re
 {
     DevBuf<uint32_t> d_chat;
     if (d_chat.alloc((size_t)repeat * kPoly)) return -1;
-    if (launch_dec_sum(y, repeat, c, d, st)) return -1;
+    if (launch_fold(y, repeat, c, d, dev->barrett, st)) return -1;
     // poly_mul_ntt(c_L, sk) (src/ntt.c:10-26): NTT both, pointwise, INTT
     if (launch_ntt_fwd(c + (size_t)l * kPoly, d_chat.get(), 3, dev->tw_all, st)) return -1;
     if (launch_ntt_fwd(sk, sk, repeat * 3, dev->tw_all, st)) return -1;
@@ -225,7 +237,7 @@ int do_decrypt(const uint32_t *c, const uint32_t *y, const uint32_t *sk, uint32_
     HostSparse hsp = to_sparse(y, repeat, l);
     DevSparse dsp;
     DevBuf<uint32_t> d_c, d_sk, d_d;
-    if (dsp.upload(hsp, l, st) || d_c.alloc((size_t)(l + 1) * kPoly) || d_sk.alloc((size_t)repeat * kPoly) ||
+    if (dsp.upload(hsp, y, repeat, l, st) || d_c.alloc((size_t)(l + 1) * kPoly) || d_sk.alloc((size_t)repeat * kPoly) ||
         d_d.alloc((size_t)repeat * kPoly))
         return -1;
     if (copy_to_device(d_c.get(), c, (size_t)(l + 1) * kPoly * 4, st)) return -1;
@@ -248,11 +260,11 @@ int do_kvalues(const uint32_t *c, const uint32_t *y, const uint32_t *msk, uint32
     HostSparse hsp = to_sparse(y, n, IPFE_L);
     DevSparse dsp;
     DevBuf<uint32_t> d_msk, d_c, d_sk, d_d, d_kv;
-    if (dsp.upload(hsp, IPFE_L, st) || d_msk.alloc(IPFE_L * kPoly) || d_c.alloc((IPFE_L + 1) * kPoly) ||
+    if (dsp.upload(hsp, y, n, IPFE_L, st) || d_msk.alloc(IPFE_L * kPoly) || d_c.alloc((IPFE_L + 1) * kPoly) ||
         d_sk.alloc((size_t)n * kPoly) || d_d.alloc((size_t)n * kPoly) || d_kv.alloc(n))
         return -1;
     if (copy_to_device(d_msk.get(), msk, IPFE_L * kPoly * 4, st)) return -1;
-    if (launch_keygen(dsp.view, n, d_msk.get(), d_sk.get(), st)) return -1;
+    if (launch_fold(dsp.view, n, d_msk.get(), d_sk.get(), dev->barrett, st)) return -1;
     if (copy_to_device(d_c.get(), c, (IPFE_L + 1) * kPoly * 4, st)) return -1;
     if (decrypt_dev(dsp.view, d_c.get(), d_sk.get(), d_d.get(), n, IPFE_L, dev, st)) return -1;
     if (launch_crt_round(d_d.get(), n, 0, d_kv.get(), st)) return -1;

@@ -2,10 +2,14 @@
 // CRT + rounding, bit-exact with src/rlwe_sife.c:215-393 and src/crt.c:46-82.
 //
 // Keygen and the first half of decryption fold  acc <- mod_prime(y_i v_i + acc)
-// over every slot i < L in order (src/rlwe_sife.c:232-240, :265-273).  A slot
-// with y_i = 0 only maps acc = q to 0, so the kernels visit the non-zero y_i of
-// a sparse list and canonicalise acc wherever zero slots were skipped; the
-// result is identical to the dense loop.
+// over every slot i < L in order (src/rlwe_sife.c:232-240, :265-273).  Here it
+// is computed as a plain sum: mod_prime returns the canonical residue unless
+// its argument is a multiple of the modulus, so the fold's result is the
+// canonical sum wherever that is not zero.  Where it is zero the result is 0 or
+// q by the fold's last steps (fold_zero).  The sum takes one 64-bit multiply-add
+// a term (two for y of 16 bits and more: the halves of y apart; 785 terms stay
+// below 2^57) and one reduction at the end, in any order, where the fold is a
+// chain of data-dependent loops -- 65 us for one vector of 123 terms.
 #include <algorithm>
 
 #include "crt_dev.h"
@@ -13,42 +17,181 @@
 
 namespace ipfe {
 
-__device__ __forceinline__ uint32_t sparse_fold(const int *__restrict__ idx, const uint32_t *__restrict__ val, int e0,
-                                                int e1, int len, const uint32_t *__restrict__ base, size_t slot_stride,
-                                                int s)
+// y_v[i] mod q_s as the fold takes it; below 2^16 it is y itself
+__device__ __forceinline__ uint32_t fold_y(uint32_t y, int s) { return y >> 16 ? mod_prime_exact(y, s) : y; }
+
+// The fold's result where its sum is 0 mod q: entries 0 .. n-1 with term(e, y,
+// v, i) giving y mod q, v and the slot i of entry e (ascending; slots between
+// entries hold y = 0, which only map acc = q to 0), len slots.  Before the last
+// entry whose product is not 0 mod q, acc is the canonical residue that cancels
+// it, whatever came before; from there on the fold is run literally.  (Sums of
+// small keys are 0 often enough, 10 coefficients of 128 keys over 785 slots,
+// that running the whole fold there took that kernel 205 us instead of 62.)
+template <class Term>
+__device__ uint32_t fold_zero(int n, int len, int s, Term term)
 {
     const uint32_t q = qmod(s);
-    uint32_t acc = 0;
+    uint32_t y, v;
+    int i, e = n - 1;
+    uint64_t t = 0;
+    for (; e >= 0; --e) {
+        term(e, y, v, i);
+        t = (uint64_t)y * v % q;
+        if (t) break;
+    }
+    uint32_t acc = e >= 0 ? q - (uint32_t)t : 0u;
     int last = -1;
-    for (int e = e0; e < e1; ++e) {
-        const int i = idx[e];
+    if (e >= 0) {
+        acc = mod_prime_exact((uint64_t)y * v + acc, s);
+        last = i;
+    }
+    for (++e; e < n; ++e) {
+        term(e, y, v, i);
         if (i > last + 1 && acc == q) acc = 0;
-        const uint64_t ys = mod_prime_exact(val[e], s);
-        acc = mod_prime_exact(ys * base[(size_t)i * slot_stride] + acc, s);
+        acc = mod_prime_exact((uint64_t)y * v + acc, s);
         last = i;
     }
     if (last < len - 1 && acc == q) acc = 0;
     return acc;
 }
 
-// sk[v][s][k]; grid (N/256 * 3, nvec)
-__global__ void k_keygen(SparseY y, const uint32_t *__restrict__ msk, uint32_t *__restrict__ sk)
+struct FoldSum {
+    uint64_t lo = 0, hi = 0;
+    __device__ __forceinline__ void add(uint32_t y, uint32_t v)
+    {
+        lo += (uint64_t)(y & 0xffffu) * v;
+        if (y >> 16) hi += (uint64_t)(y >> 16) * v;
+    }
+    __device__ __forceinline__ uint32_t value(int s, const BarrettConsts &bc) const
+    {
+        const uint64_t h = hi ? reduce64(hi, qmod(s), bc.mu_hi[s], bc.mu_lo[s]) : 0u;
+        return reduce64(lo + (h << 16), qmod(s), bc.mu_hi[s], bc.mu_lo[s]);
+    }
+};
+
+// fold_zero of vector v at the coefficient base points at
+__device__ uint32_t fold_zero_sparse(const SparseY &y, int v, int s, const uint32_t *base)
 {
-    const int v = blockIdx.y;
-    const int s = blockIdx.x / (IPFE_N / 256);
-    const int k = (blockIdx.x % (IPFE_N / 256)) * 256 + threadIdx.x;
-    const uint32_t *base = msk + (size_t)s * IPFE_N + k;
-    sk[((size_t)v * 3 + s) * IPFE_N + k] = sparse_fold(y.idx, y.val, y.off[v], y.off[v + 1], y.len, base, 3 * IPFE_N, s);
+    const int e0 = y.off[v];
+    return fold_zero(y.off[v + 1] - e0, y.len, s, [&](int e, uint32_t &yy, uint32_t &vv, int &i) {
+        i = y.idx[e0 + e];
+        yy = fold_y(y.val[e0 + e], s);
+        vv = base[(size_t)i * 3 * IPFE_N];
+    });
 }
 
-// d[v][s][k] = fold_i y_v[i] c_i[s][k] for one ciphertext c [len+1][3][N].
-__global__ void k_dec_sum(SparseY y, const uint32_t *__restrict__ c, uint32_t *__restrict__ d)
+constexpr int FOLD_WAVES = 4;  // waves of a workgroup, each with its share of the terms
+
+// Few sparse vectors: 64 coefficients a workgroup, the entries dealt to four
+// waves, so that one vector's 12,288 chains are 768 waves of a quarter of the
+// terms (65 us -> 10.5 for one of 123).  Grid (3 N / 64, nvec).
+__global__ __launch_bounds__(64 * FOLD_WAVES) void k_fold_few(SparseY y, const uint32_t *__restrict__ P,
+                                                             uint32_t *__restrict__ out, BarrettConsts bc)
 {
-    const int v = blockIdx.y;
-    const int s = blockIdx.x / (IPFE_N / 256);
-    const int k = (blockIdx.x % (IPFE_N / 256)) * 256 + threadIdx.x;
-    const uint32_t *base = c + (size_t)s * IPFE_N + k;
-    d[((size_t)v * 3 + s) * IPFE_N + k] = sparse_fold(y.idx, y.val, y.off[v], y.off[v + 1], y.len, base, 3 * IPFE_N, s);
+    __shared__ uint32_t part[FOLD_WAVES][64];
+    const int v = blockIdx.y, s = blockIdx.x / (IPFE_N / 64), lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int k = (int)(blockIdx.x % (IPFE_N / 64)) * 64 + lane;
+    const uint32_t *base = P + (size_t)s * IPFE_N + k;
+    const int e0 = y.off[v], e1 = y.off[v + 1];
+    FoldSum acc;
+#pragma unroll 8
+    for (int e = e0 + w; e < e1; e += FOLD_WAVES)
+        acc.add(fold_y(y.val[e], s), base[(size_t)y.idx[e] * 3 * IPFE_N]);
+    part[w][lane] = acc.value(s, bc);
+    __syncthreads();
+    if (w) return;
+    uint64_t t = 0;
+#pragma unroll
+    for (int j = 0; j < FOLD_WAVES; ++j) t += part[j][lane];
+    uint32_t r = (uint32_t)(t % qmod(s));
+    if (r == 0) r = fold_zero_sparse(y, v, s, base);
+    out[((size_t)v * 3 + s) * IPFE_N + k] = r;
+}
+
+// Many sparse vectors: four consecutive coefficients a thread, 16-byte loads
+// (2,000 vectors of 14 entries: 267 -> 80 us, 98 MB written).
+// Grid (3 N / 1024, nvec).
+__global__ __launch_bounds__(256) void k_fold_many(SparseY y, const uint32_t *__restrict__ P,
+                                                   uint32_t *__restrict__ out, BarrettConsts bc)
+{
+    const int v = blockIdx.y, s = blockIdx.x / (IPFE_N / 1024);
+    const int k = (int)(blockIdx.x % (IPFE_N / 1024)) * 1024 + 4 * threadIdx.x;
+    const uint32_t *base = P + (size_t)s * IPFE_N + k;
+    const int e0 = y.off[v], e1 = y.off[v + 1];
+    FoldSum acc[4];
+#pragma unroll 4
+    for (int e = e0; e < e1; ++e) {
+        const uint4 p = *reinterpret_cast<const uint4 *>(base + (size_t)y.idx[e] * 3 * IPFE_N);
+        const uint32_t t = fold_y(y.val[e], s);
+        acc[0].add(t, p.x);
+        acc[1].add(t, p.y);
+        acc[2].add(t, p.z);
+        acc[3].add(t, p.w);
+    }
+    uint32_t r[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        r[u] = acc[u].value(s, bc);
+        if (r[u] == 0) r[u] = fold_zero_sparse(y, v, s, base + u);
+    }
+    *reinterpret_cast<uint4 *>(out + ((size_t)v * 3 + s) * IPFE_N + k) = make_uint4(r[0], r[1], r[2], r[3]);
+}
+
+// Dense vectors with every y below 2^16: FOLD_VECS vectors share each word of
+// P; their y come from scalar loads, a slot's 16 side by side (k_fold_pack; from
+// 16 rows of y apart it took 87 us).  64 coefficients a workgroup, the slots
+// dealt to four waves: 128 vectors of 785 slots in 62 us + 5 for the packing
+// (1,131 for the literal fold).  Grid (3 N / 64, nvec / FOLD_VECS).
+constexpr int FOLD_VECS = 16;
+
+// y [nvec][len] -> [nvec / 16][len][16], zeros past nvec
+__global__ void k_fold_pack(const uint32_t *__restrict__ y, int nvec, int len, uint32_t *__restrict__ packed)
+{
+    const int v = blockIdx.y * FOLD_VECS + (threadIdx.x & (FOLD_VECS - 1));
+    const int i = blockIdx.x * (256 / FOLD_VECS) + threadIdx.x / FOLD_VECS;
+    if (i < len) packed[((size_t)blockIdx.y * len + i) * FOLD_VECS + (threadIdx.x & (FOLD_VECS - 1))] =
+        v < nvec ? y[(size_t)v * len + i] : 0u;
+}
+
+__global__ __launch_bounds__(64 * FOLD_WAVES) void k_fold_dense(const uint32_t *__restrict__ y,
+                                                               const uint32_t *__restrict__ packed, int nvec,
+                                                               int len, const uint32_t *__restrict__ P,
+                                                               uint32_t *__restrict__ out, BarrettConsts bc)
+{
+    __shared__ uint32_t part[FOLD_WAVES][FOLD_VECS][64];
+    const int v0 = blockIdx.y * FOLD_VECS, s = blockIdx.x / (IPFE_N / 64), lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int k = (int)(blockIdx.x % (IPFE_N / 64)) * 64 + lane;
+    const uint32_t *base = P + (size_t)s * IPFE_N + k;
+    const int i0 = len * w / FOLD_WAVES, i1 = len * (w + 1) / FOLD_WAVES;
+    uint64_t acc[FOLD_VECS] = {};
+    const uint32_t *yp = packed + (size_t)blockIdx.y * len * FOLD_VECS;
+#pragma unroll 4
+    for (int i = i0; i < i1; ++i) {
+        const uint32_t p = base[(size_t)i * 3 * IPFE_N];
+#pragma unroll
+        for (int j = 0; j < FOLD_VECS; ++j) acc[j] += (uint64_t)yp[(size_t)i * FOLD_VECS + j] * p;
+    }
+#pragma unroll
+    for (int j = 0; j < FOLD_VECS; ++j)
+        part[w][j][lane] = reduce64(acc[j], qmod(s), bc.mu_hi[s], bc.mu_lo[s]);
+    __syncthreads();
+    for (int j = w; j < FOLD_VECS && v0 + j < nvec; j += FOLD_WAVES) {
+        uint64_t t = 0;
+#pragma unroll
+        for (int u = 0; u < FOLD_WAVES; ++u) t += part[u][j][lane];
+        uint32_t r = (uint32_t)(t % qmod(s));
+        if (r == 0) {
+            const uint32_t *yv = y + (size_t)(v0 + j) * len;
+            r = fold_zero(len, len, s, [&](int e, uint32_t &yy, uint32_t &vv, int &i) {
+                i = e;
+                yy = yv[e];
+                vv = base[(size_t)e * 3 * IPFE_N];
+            });
+        }
+        out[((size_t)(v0 + j) * 3 + s) * IPFE_N + k] = r;
+    }
 }
 
 __global__ void k_poly_sub(uint32_t *__restrict__ d, const uint32_t *__restrict__ prod, size_t n_total)
@@ -67,20 +210,33 @@ __global__ void k_crt_round(const uint32_t *__restrict__ d, int nvec, int coef, 
     r[v] = crt_decode(dv[0], dv[IPFE_N], dv[2 * IPFE_N]);
 }
 
-int launch_keygen(const SparseY &y, int nvec, const uint32_t *msk, uint32_t *sk, hipStream_t st)
+// out[v][3][N] = sum_i y_v[i] P[i] with the reference's sequential fold.
+// Dense form: at least FOLD_VECS vectors with a quarter of their entries set
+// (a vector's own list then costs more than sharing each word of P with 15
+// others).  Sparse form: from 32 vectors on their coefficients alone fill the
+// GPU (96 waves each), below that the entries are split as well.
+int launch_fold(const SparseY &y, int nvec, const uint32_t *P, uint32_t *out, const BarrettConsts &bc, hipStream_t st)
 {
     if (nvec <= 0) return 0;
-    hipLaunchKernelGGL(k_keygen, dim3(3 * IPFE_N / 256, nvec), dim3(256), 0, st, y, msk, sk);
+    if (y.dense) {
+        const unsigned groups = (unsigned)(nvec + FOLD_VECS - 1) / FOLD_VECS;
+        hipLaunchKernelGGL(k_fold_pack, dim3((y.len * FOLD_VECS + 255) / 256, groups), dim3(256), 0, st, y.dense, nvec,
+                           y.len, y.dense_packed);
+        hipLaunchKernelGGL(k_fold_dense, dim3(3 * IPFE_N / 64, groups), dim3(64 * FOLD_WAVES), 0, st, y.dense,
+                           y.dense_packed, nvec, y.len, P, out, bc);
+    } else if (nvec < 32)
+        hipLaunchKernelGGL(k_fold_few, dim3(3 * IPFE_N / 64, nvec), dim3(64 * FOLD_WAVES), 0, st, y, P, out, bc);
+    else
+        hipLaunchKernelGGL(k_fold_many, dim3(3 * IPFE_N / 1024, nvec), dim3(256), 0, st, y, P, out, bc);
     HIP_OK(hipGetLastError());
     return 0;
 }
 
-int launch_dec_sum(const SparseY &y, int nvec, const uint32_t *c, uint32_t *d, hipStream_t st)
+size_t fold_packed_words(size_t nvec, size_t len) { return (nvec + FOLD_VECS - 1) / FOLD_VECS * FOLD_VECS * len; }
+
+bool fold_dense(size_t nvec, size_t len, size_t nnz, uint32_t max_y)
 {
-    if (nvec <= 0) return 0;
-    hipLaunchKernelGGL(k_dec_sum, dim3(3 * IPFE_N / 256, nvec), dim3(256), 0, st, y, c, d);
-    HIP_OK(hipGetLastError());
-    return 0;
+    return nvec >= FOLD_VECS && nnz > 0 && max_y < 65536u && nnz * 4 >= nvec * len;
 }
 
 int launch_poly_sub(uint32_t *d, const uint32_t *prod, size_t n_total, hipStream_t st)

@@ -112,11 +112,18 @@ struct SparseY {
     const int *idx;
     const uint32_t *val;
     int len;
+    // the vectors themselves [nvec][len] where fold_dense holds, and scratch of
+    // fold_packed_words(nvec, len)
+    const uint32_t *dense = nullptr;
+    uint32_t *dense_packed = nullptr;
 };
-// sk[v][3][N] = sum_i y_v[i] msk[i] with the reference's sequential fold.
-int launch_keygen(const SparseY &y, int nvec, const uint32_t *msk, uint32_t *sk, hipStream_t st);
-// d[v][3][N] = sum_i y_v[i] c_i (fold)  (first half of rlwe_sife_decrypt_gmp).
-int launch_dec_sum(const SparseY &y, int nvec, const uint32_t *c, uint32_t *d, hipStream_t st);
+// out[v][3][N] = sum_i y_v[i] P[i] with the reference's sequential fold: keygen
+// (P = msk) and the first half of rlwe_sife_decrypt_gmp (P = c).
+int launch_fold(const SparseY &y, int nvec, const uint32_t *P, uint32_t *out, const BarrettConsts &bc,
+                hipStream_t st);
+// Whether vectors with nnz entries in all, none above max_y, take the dense form.
+bool fold_dense(size_t nvec, size_t len, size_t nnz, uint32_t max_y);
+size_t fold_packed_words(size_t nvec, size_t len);
 // d[v] = sub_mod(d[v], prod[v]) elementwise.
 int launch_poly_sub(uint32_t *d, const uint32_t *prod, size_t n_total, hipStream_t st);
 // CRT + rounding of coefficient k of d[v][3][N] -> r[v]  (k = 0 for kvalues).

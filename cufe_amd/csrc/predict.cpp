@@ -232,7 +232,7 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
     y.idx = y_idx.get();
     y.val = y_val.get();
     y.len = L;
-    if (launch_keygen(y, nS, msk_dev, sk.get(), st)) return -1;
+    if (launch_fold(y, nS, msk_dev, sk.get(), device()->barrett, st)) return -1;
     DevBuf<unsigned int> d_max;
     if (d_max.alloc(3)) return -1;
     if (launch_fill_i32((int *)d_max.get(), 0, 3, st)) return -1;
