@@ -210,21 +210,15 @@ int do_keygen(const uint32_t *y, const uint32_t *msk, uint32_t *sk, int repeat, 
 }
 
 // Decryption of c [l+1][3][N] under `repeat` keys, on the device: d [repeat][3][N].
-// c's last polynomial and sk are transformed in place.
-int decrypt_dev(const SparseY &y, uint32_t *c, uint32_t *sk, uint32_t *d, int repeat, int l, Device *dev,
+// c's last polynomial is transformed in place.
+int decrypt_dev(const SparseY &y, uint32_t *c, const uint32_t *sk, uint32_t *d, int repeat, int l, Device *dev,
                 hipStream_t st)
 {
-    DevBuf<uint32_t> d_chat;
-    if (d_chat.alloc((size_t)repeat * kPoly)) return -1;
+    uint32_t *cl = c + (size_t)l * kPoly;
     if (launch_fold(y, repeat, c, d, dev->barrett, st)) return -1;
     // poly_mul_ntt(c_L, sk) (src/ntt.c:10-26): NTT both, pointwise, INTT
-    if (launch_ntt_fwd(c + (size_t)l * kPoly, d_chat.get(), 3, dev->tw_all, st)) return -1;
-    if (launch_ntt_fwd(sk, sk, repeat * 3, dev->tw_all, st)) return -1;
-    for (int v = 1; v < repeat; ++v)
-        HIP_OK(hipMemcpyAsync(d_chat.get() + (size_t)v * kPoly, d_chat.get(), kPoly * 4, hipMemcpyDeviceToDevice, st));
-    if (launch_point_mul(d_chat.get(), sk, sk, (size_t)repeat * kPoly, dev->barrett, st)) return -1;
-    if (launch_ntt_inv(sk, sk, repeat * 3, dev->tw_all, dev->ninv, st)) return -1;
-    return launch_poly_sub(d, sk, (size_t)repeat * kPoly, st);
+    if (launch_ntt_fwd(cl, cl, 3, dev->tw_all, st)) return -1;
+    return launch_dec_poly(cl, sk, d, repeat, dev->tw_all, dev->ninv, dev->barrett, st);
 }
 
 // One ciphertext c [l+1][3][N] against `repeat` keys -> d_y [repeat][3][N].

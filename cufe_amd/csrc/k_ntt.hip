@@ -190,16 +190,43 @@ __global__ __launch_bounds__(NTT_THREADS) void k_enc_poly(const EncItem *__restr
 }
 
 // ---------------------------------------------------------------------------
-// Pointwise product of two NTT-domain limbs, both read at [z][N] (z = poly*3+s):
-// out = mul_mod(a, b), exact for operands in [0, q].
+// Second half of rlwe_sife_decrypt_gmp (src/rlwe_sife.c:274-284) for one limb of
+// one key: d = sub_mod(d, INTT(chat (.) NTT(sk))), each product mul_mod exact for
+// operands in [0, q].  One workgroup keeps the limb in registers and LDS from
+// sk to d: 48 KiB of HBM a limb, where separate transform, product, inverse and
+// difference kernels moved 192 KiB and needed c_L's transform copied per key
+// (100 keys: 22 us for 31 in four kernels and 99 copies of 2 us each).
 // ---------------------------------------------------------------------------
-__global__ void k_point_mul(const uint32_t *__restrict__ a, const uint32_t *__restrict__ b, uint32_t *__restrict__ out,
-                            size_t n_total, BarrettConsts bc)
+__global__ __launch_bounds__(NTT_THREADS) void k_dec_poly(const uint32_t *__restrict__ chat,
+                                                           const uint32_t *__restrict__ sk, uint32_t *__restrict__ d,
+                                                           const uint32_t *__restrict__ tw_all, NinvConsts nc,
+                                                           BarrettConsts bc)
 {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_total) return;
-    const int s = (int)((i / IPFE_N) % 3);
-    out[i] = mul_exact(a[i], b[i], s, bc.mu_hi[s], bc.mu_lo[s]);
+    __shared__ uint32_t lds[NTT_LDS_WORDS];
+    const int z = blockIdx.x, s = z % 3, tid = threadIdx.x;
+    const uint32_t q = qmod(s);
+    uint32_t x[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) x[r] = sk[(size_t)z * IPFE_N + posA(tid, r)];
+    if (__syncthreads_or(any_eq_q(x, q)))
+        ntt_fwd_block<true>(x, lds, tw_fwd(tw_all, s), twp_fwd(tw_all, s), q);
+    else
+        ntt_fwd_block<false>(x, lds, tw_fwd(tw_all, s), twp_fwd(tw_all, s), q);
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        x[r] = mul_exact(chat[s * IPFE_N + posA(tid, r)], x[r], s, bc.mu_hi[s], bc.mu_lo[s]);
+    uint32_t *dz = d + (size_t)z * IPFE_N;
+    if (__syncthreads_or(any_eq_q(x, q))) {
+        ntt_inv_block<true>(x, lds, tw_inv(tw_all, s), twp_inv(tw_all, s), q);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[r] = scale_ninv<true>(x[r], nc.ninv[s], nc.ninvp[s], nc.flag[s], q);
+    } else {
+        ntt_inv_block<false>(x, lds, tw_inv(tw_all, s), twp_inv(tw_all, s), q);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[r] = scale_ninv<false>(x[r], nc.ninv[s], nc.ninvp[s], nc.flag[s], q);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dz[posA(tid, r)] = sub_q(dz[posA(tid, r)], x[r], q);
 }
 
 // ---------------------------------------------------------------------------
@@ -249,12 +276,11 @@ int launch_enc_poly(const EncItem *items, int nitems, const EncMsg *msgs, const 
     return 0;
 }
 
-int launch_point_mul(const uint32_t *a, const uint32_t *b, uint32_t *out, size_t n_total, const BarrettConsts &bc,
-                     hipStream_t st)
+int launch_dec_poly(const uint32_t *chat, const uint32_t *sk, uint32_t *d, int nvec, const uint32_t *tw_all,
+                    const NinvConsts &nc, const BarrettConsts &bc, hipStream_t st)
 {
-    if (n_total == 0) return 0;
-    const int bs = 256;
-    hipLaunchKernelGGL(k_point_mul, dim3((unsigned)((n_total + bs - 1) / bs)), dim3(bs), 0, st, a, b, out, n_total, bc);
+    if (nvec <= 0) return 0;
+    hipLaunchKernelGGL(k_dec_poly, dim3((unsigned)nvec * 3), dim3(NTT_THREADS), 0, st, chat, sk, d, tw_all, nc, bc);
     HIP_OK(hipGetLastError());
     return 0;
 }

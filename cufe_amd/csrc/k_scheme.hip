@@ -194,14 +194,6 @@ __global__ __launch_bounds__(64 * FOLD_WAVES) void k_fold_dense(const uint32_t *
     }
 }
 
-__global__ void k_poly_sub(uint32_t *__restrict__ d, const uint32_t *__restrict__ prod, size_t n_total)
-{
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_total) return;
-    const uint32_t q = qmod((int)((i / IPFE_N) % 3));
-    d[i] = sub_q(d[i], prod[i], q);
-}
-
 __global__ void k_crt_round(const uint32_t *__restrict__ d, int nvec, int coef, uint32_t *__restrict__ r)
 {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
@@ -237,14 +229,6 @@ size_t fold_packed_words(size_t nvec, size_t len) { return (nvec + FOLD_VECS - 1
 bool fold_dense(size_t nvec, size_t len, size_t nnz, uint32_t max_y)
 {
     return nvec >= FOLD_VECS && nnz > 0 && max_y < 65536u && nnz * 4 >= nvec * len;
-}
-
-int launch_poly_sub(uint32_t *d, const uint32_t *prod, size_t n_total, hipStream_t st)
-{
-    if (n_total == 0) return 0;
-    hipLaunchKernelGGL(k_poly_sub, dim3((unsigned)((n_total + 255) / 256)), dim3(256), 0, st, d, prod, n_total);
-    HIP_OK(hipGetLastError());
-    return 0;
 }
 
 int launch_crt_round(const uint32_t *d, int nvec, int coef, uint32_t *r, hipStream_t st)

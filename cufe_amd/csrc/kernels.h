@@ -41,8 +41,10 @@ int launch_setup_pk(const uint32_t *msk, const uint32_t *e, const uint32_t *ahat
                     int l, const uint32_t *tw_all, hipStream_t st);
 int launch_enc_poly(const EncItem *items, int nitems, const EncMsg *msgs, const uint32_t *mpk, int mpk_l,
                     const uint32_t *tw_all, const NinvConsts &nc, const ScaleConsts &sc, hipStream_t st);
-int launch_point_mul(const uint32_t *a, const uint32_t *b, uint32_t *out, size_t n_total, const BarrettConsts &bc,
-                     hipStream_t st);
+// d[v] = sub_mod(d[v], poly_mul_ntt(c_L, sk[v])) for nvec keys; chat = NTT(c_L)
+// [3][N], sk and d [nvec][3][N].
+int launch_dec_poly(const uint32_t *chat, const uint32_t *sk, uint32_t *d, int nvec, const uint32_t *tw_all,
+                    const NinvConsts &nc, const BarrettConsts &bc, hipStream_t st);
 
 // ----- Sampler (k_sampler.hip) -----
 // One AES-256-CTR Gaussian stream cut into 384-byte chunks (24 AES blocks).
@@ -124,8 +126,6 @@ int launch_fold(const SparseY &y, int nvec, const uint32_t *P, uint32_t *out, co
 // Whether vectors with nnz entries in all, none above max_y, take the dense form.
 bool fold_dense(size_t nvec, size_t len, size_t nnz, uint32_t max_y);
 size_t fold_packed_words(size_t nvec, size_t len);
-// d[v] = sub_mod(d[v], prod[v]) elementwise.
-int launch_poly_sub(uint32_t *d, const uint32_t *prod, size_t n_total, hipStream_t st);
 // CRT + rounding of coefficient k of d[v][3][N] -> r[v]  (k = 0 for kvalues).
 int launch_crt_round(const uint32_t *d, int nvec, int coef, uint32_t *r, hipStream_t st);
 // out += sum over i of (2i+1) * w[i] mod 2^64 (out must be cleared first)
