@@ -153,34 +153,76 @@ __global__ void k_rows_frac(const uint32_t *__restrict__ cl, const uint32_t *__r
     *reinterpret_cast<uint64_t *>(ref + (size_t)row * (ksteps * 32) + k) = dw;
 }
 
-// Keys: whether every key coefficient is the same integer in the three limbs
-// (kd [3][S][K] balanced; *neq set otherwise), the margins M_v = ceil(s / 2) +
-// ceil(s / 2^16) + 1 (72 bits) and M88_v = ceil(s / 2) + ceil(s / 2^7) + 1
-// (88 bits) with s = sum_k |B_v[k]|, each times 2^widen up to 2^62 (widen > 0
-// only to test the exact kernel on many pairs), and limb 0's values as int16
-// k16 [S][K] for the exact kernel (two key digits: |B| <= 32,512).
-__global__ void k_keys_frac(const double *__restrict__ kd, int S, int K, int widen, uint64_t *__restrict__ margin,
-                            uint64_t *__restrict__ margin88, int16_t *__restrict__ k16, int *__restrict__ neq)
+// Keys in contraction order (k_contract_keys with sign -1): column 0 -sk_0,
+// column j < N  sk_{N-j}, then the y slots, balanced.  One workgroup per key,
+// all three limbs at once: largest |value| per limb (maxabs), whether every
+// value is the same integer in the three limbs (*neq set otherwise), the
+// margins M_v = ceil(s / 2) + ceil(s / 2^16) + 1 (72 bits) and M88_v =
+// ceil(s / 2) + ceil(s / 2^7) + 1 (88 bits) with s = sum_k |B_v[k]|, each times
+// 2^widen up to 2^62 (widen > 0 only to test the exact kernel on many pairs),
+// and limb 0's values as int16 k16 [S][K] (meaningful within two key digits,
+// |B| <= 32,512).  Bound by HBM: 98 MB of keys read and 17 MB written for 2,000
+// keys (28 us, and 13 for the digits), where the fp64 operand in between made it 203 MB
+// written and twice read, 306 us in all.
+__global__ __launch_bounds__(256) void k_keys_build(const uint32_t *__restrict__ sk, int S, int K, SparseY y,
+                                                    int widen, uint64_t *__restrict__ margin,
+                                                    uint64_t *__restrict__ margin88, int16_t *__restrict__ k16,
+                                                    unsigned int *__restrict__ maxabs, int *__restrict__ neq)
 {
-    __shared__ unsigned long long part[256];
-    const int v = blockIdx.x;
-    unsigned long long sum = 0;
-    bool bad = false;
-    for (int k = threadIdx.x; k < K; k += blockDim.x) {
-        const double b0 = kd[(size_t)v * K + k], b1 = kd[((size_t)S + v) * K + k], b2 = kd[((size_t)2 * S + v) * K + k];
-        bad = bad || b0 != b1 || b0 != b2 || fabs(b0) > 32767.0;
-        sum += (unsigned long long)fabs(b0);
-        k16[(size_t)v * K + k] = (int16_t)b0;
-    }
-    if (bad) atomicOr(neq, 1);
-    part[threadIdx.x] = sum;
+    __shared__ uint32_t slots[IPFE_L + 15];
+    __shared__ unsigned long long part[4];
+    __shared__ unsigned int pmax[4][3];
+    __shared__ int pbad[4];
+    const int v = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const uint32_t *src = sk + (size_t)v * 3 * IPFE_N;
+    for (int i = tid; i < K - IPFE_N; i += 256) slots[i] = 0;
     __syncthreads();
-    for (int h = blockDim.x / 2; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) part[threadIdx.x] += part[threadIdx.x + h];
-        __syncthreads();
+    for (int e = y.off[v] + tid; e < y.off[v + 1]; e += 256) slots[y.idx[e]] = y.val[e];
+    __syncthreads();
+    unsigned long long sum = 0;
+    unsigned int mx[3] = {0, 0, 0};
+    bool bad = false;
+#pragma unroll 4
+    for (int j = tid; j < K; j += 256) {
+        int b[3];
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+            const uint32_t q = qmod(s);
+            uint32_t t;
+            if (j < IPFE_N)
+                t = src[s * IPFE_N + (j == 0 ? 0 : IPFE_N - j)];
+            else
+                t = mod_prime_exact(slots[j - IPFE_N], s);
+            if (t >= q) t -= q;
+            b[s] = t > q / 2 ? (int)((int64_t)t - q) : (int)t;
+            if (j == 0) b[s] = -b[s];  // |b| <= (q - 1) / 2: still balanced
+            mx[s] = max(mx[s], (unsigned int)abs(b[s]));
+        }
+        bad = bad || b[0] != b[1] || b[0] != b[2];
+        sum += (unsigned int)abs(b[0]);
+        k16[(size_t)v * K + j] = (int16_t)b[0];
     }
-    if (threadIdx.x == 0) {
-        const unsigned long long s = part[0], cap = 1ull << 62;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        sum += __shfl_xor(sum, d, 64);
+#pragma unroll
+        for (int s = 0; s < 3; ++s) mx[s] = max(mx[s], (unsigned int)__shfl_xor((int)mx[s], d, 64));
+    }
+    const bool wbad = __ballot(bad) != 0;
+    if (lane == 0) {
+        part[w] = sum;
+        pbad[w] = wbad;
+#pragma unroll
+        for (int s = 0; s < 3; ++s) pmax[w][s] = mx[s];
+    }
+    __syncthreads();
+    if (tid < 3) {
+        const unsigned int m = max(max(pmax[0][tid], pmax[1][tid]), max(pmax[2][tid], pmax[3][tid]));
+        if (m > __hip_atomic_load(maxabs + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(maxabs + tid, m);
+    }
+    if (tid == 0) {
+        if (pbad[0] || pbad[1] || pbad[2] || pbad[3]) atomicOr(neq, 1);
+        const unsigned long long s = part[0] + part[1] + part[2] + part[3], cap = 1ull << 62;
         const unsigned long long m = (s + 1) / 2 + (s + (1ull << 16) - 1) / (1ull << 16) + 1;
         const unsigned long long m88 = (s + 1) / 2 + (s + 127) / 128 + 1;
         margin[v] = m > (cap >> widen) ? cap : m << widen;
@@ -587,16 +629,16 @@ int launch_rows_frac(const uint32_t *cl, const uint32_t *c0, int src_l, int R, i
     return 0;
 }
 
-int launch_keys_frac(const double *kd, int S, int K, int widen, uint64_t *margin, uint64_t *margin88, int16_t *k16,
-                     int *neq, hipStream_t st)
+int launch_keys_build(const uint32_t *sk, int S, int K, const SparseY &y, int widen, uint64_t *margin,
+                      uint64_t *margin88, int16_t *k16, unsigned int *maxabs, int *neq, hipStream_t st)
 {
     if (S <= 0) return 0;
-    if (widen < 0 || widen > 62) {
-        ipfe_set_error("fraction keys: widening 2^%d out of range", widen);
+    if (widen < 0 || widen > 62 || K < IPFE_N || K > IPFE_N + IPFE_L + 15) {
+        ipfe_set_error("keys: widening 2^%d, %d columns", widen, K);
         return -1;
     }
-    hipLaunchKernelGGL(k_keys_frac, dim3((unsigned)S), dim3(256), 0, st, kd, S, K, widen, margin, margin88, k16,
-                       neq);
+    hipLaunchKernelGGL(k_keys_build, dim3((unsigned)S), dim3(256), 0, st, sk, S, K, y, widen, margin, margin88, k16,
+                       maxabs, neq);
     HIP_OK(hipGetLastError());
     return 0;
 }

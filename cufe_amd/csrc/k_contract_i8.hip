@@ -913,6 +913,40 @@ __global__ void k_keys_digits(const double *__restrict__ kd, int S, int K, int s
     }
 }
 
+// The same store with two digits from int16 keys [S][K] that are the same
+// integers in every limb (K a multiple of 16): 16 columns of a key a thread,
+// one 16-byte fragment per digit and limb.
+__global__ void k_keys_digits16(const int16_t *__restrict__ k16, int S, int K, int spad, int ksteps,
+                                int8_t *__restrict__ dig)
+{
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (size_t)spad * ksteps * 2) return;
+    const int lane = (int)(i & 63), ks = (int)(i / 64 % ksteps), kb = (int)(i / 64 / ksteps);
+    const int key = kb * 32 + (lane & 31), k = ks * 32 + (lane >> 5) * 16;
+    int4 in[2] = {};
+    if (key < S && k < K) {
+        const int4 *src = reinterpret_cast<const int4 *>(k16 + (size_t)key * K + k);
+        in[0] = src[0];
+        in[1] = src[1];
+    }
+    const int *w = &in[0].x;
+    uint32_t d[2][4] = {};
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        int v = u & 1 ? w[u / 2] >> 16 : (int)(short)w[u / 2];
+        const int lo = digit_split(v);
+        d[0][u / 4] |= (uint32_t)(uint8_t)(int8_t)lo << (8 * (u & 3));
+        d[1][u / 4] |= (uint32_t)(uint8_t)(int8_t)v << (8 * (u & 3));
+    }
+    const size_t limb_bytes = (size_t)spad / 32 * ksteps * 2 * 1024;
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            *reinterpret_cast<uint4 *>(dig + s * limb_bytes + (((size_t)kb * ksteps + ks) * 2 + e) * 1024 + lane * 16) =
+                make_uint4(d[e][0], d[e][1], d[e][2], d[e][3]);
+}
+
 // 128 rows past the capacity: a tile of up to 4 row blocks may start at any
 // 32-row boundary below the capacity
 size_t rows_digit_limb_bytes(int cap, int ksteps) { return (size_t)(cap + 128) / 32 * ksteps * DG_A * 1024; }
@@ -943,6 +977,20 @@ int launch_keys_digits(const double *kd, int S, int K, int spad, int ksteps, int
         return -1;
     }
     hipLaunchKernelGGL(k_keys_digits, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, kd, S, K, spad, ksteps, nb,
+                       dig);
+    HIP_OK(hipGetLastError());
+    return 0;
+}
+
+int launch_keys_digits16(const int16_t *k16, int S, int K, int spad, int ksteps, int8_t *dig, hipStream_t st)
+{
+    const size_t n = (size_t)spad * ksteps * 2;
+    if (n == 0) return 0;
+    if (spad % 128 || spad < S || ksteps * 32 < K || K % 16 || ((uintptr_t)k16 & 15) || ((uintptr_t)dig & 15)) {
+        ipfe_set_error("key digits: %d keys padded to %d, %d k steps for K=%d", S, spad, ksteps, K);
+        return -1;
+    }
+    hipLaunchKernelGGL(k_keys_digits16, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, k16, S, K, spad, ksteps,
                        dig);
     HIP_OK(hipGetLastError());
     return 0;

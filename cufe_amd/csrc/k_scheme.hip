@@ -239,6 +239,95 @@ int launch_crt_round(const uint32_t *d, int nvec, int coef, uint32_t *r, hipStre
     return 0;
 }
 
+// Sparse lists of dense vectors y [n][stride], one wave per vector: counts (into
+// off[v + 1]) with info[0] = the largest slot in use plus one and info[1] =
+// v stride + i of the first entry at a slot i >= limit, then, after the prefix
+// sums, the entries.
+__global__ __launch_bounds__(256) void k_sparse_count(const uint32_t *__restrict__ y, int n, int stride, int limit,
+                                                      int *__restrict__ off, unsigned int *__restrict__ info)
+{
+    const int v = blockIdx.x * 4 + threadIdx.x / 64, lane = threadIdx.x & 63;
+    if (v >= n) return;
+    const uint32_t *row = y + (size_t)v * stride;
+    int cnt = 0, last = -1;
+    for (int i0 = 0; i0 < stride; i0 += 64) {
+        const bool set = i0 + lane < stride && row[i0 + lane] != 0;
+        const uint64_t m = __ballot(set);
+        cnt += __popcll(m);
+        if (m) last = i0 + 63 - __clzll((long long)m);
+        const uint64_t over = __ballot(set && i0 + lane >= limit);
+        if (over && lane == 0) atomicMin(info + 1, (unsigned int)v * stride + i0 + __ffsll((unsigned long long)over) - 1);
+    }
+    if (lane) return;
+    off[v + 1] = cnt;
+    if (last + 1 > (int)__hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(info, (unsigned int)(last + 1));
+}
+
+// off[1 .. n] from counts to their running sum, off[0] = 0; one workgroup.
+__global__ __launch_bounds__(1024) void k_sparse_prefix(int *__restrict__ off, int n)
+{
+    __shared__ int wsum[16];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    int carry = 0;
+    if (tid == 0) off[0] = 0;
+    for (int i0 = 0; i0 < n; i0 += 1024) {
+        const int i = i0 + tid;
+        int x = i < n ? off[i + 1] : 0;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(x, d, 64);
+            if (lane >= d) x += o;
+        }
+        if (lane == 63) wsum[wv] = x;
+        __syncthreads();
+        int before = carry;
+        for (int j = 0; j < 16; ++j) {
+            before += j < wv ? wsum[j] : 0;
+            carry += wsum[j];
+        }
+        if (i < n) off[i + 1] = before + x;
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(256) void k_sparse_fill(const uint32_t *__restrict__ y, int n, int stride,
+                                                     const int *__restrict__ off, int *__restrict__ idx,
+                                                     uint32_t *__restrict__ val)
+{
+    const int v = blockIdx.x * 4 + threadIdx.x / 64, lane = threadIdx.x & 63;
+    if (v >= n) return;
+    const uint32_t *row = y + (size_t)v * stride;
+    int at = off[v];
+    for (int i0 = 0; i0 < stride; i0 += 64) {
+        const uint32_t t = i0 + lane < stride ? row[i0 + lane] : 0u;
+        const uint64_t m = __ballot(t != 0);
+        if (t) {
+            const int o = at + __popcll(m & ((1ull << lane) - 1));
+            idx[o] = i0 + lane;
+            val[o] = t;
+        }
+        at += __popcll(m);
+    }
+}
+
+int launch_sparse_count(const uint32_t *y, int n, int stride, int limit, int *off, unsigned int *info, hipStream_t st)
+{
+    if (n <= 0) return 0;
+    if (launch_fill_i32((int *)info, 0, 1, st) || launch_fill_i32((int *)info + 1, -1, 1, st)) return -1;
+    hipLaunchKernelGGL(k_sparse_count, dim3((unsigned)(n + 3) / 4), dim3(256), 0, st, y, n, stride, limit, off, info);
+    HIP_OK(hipGetLastError());
+    return 0;
+}
+
+int launch_sparse_fill(const uint32_t *y, int n, int stride, int *off, int *idx, uint32_t *val, hipStream_t st)
+{
+    if (n <= 0) return 0;
+    hipLaunchKernelGGL(k_sparse_prefix, dim3(1), dim3(1024), 0, st, off, n);
+    hipLaunchKernelGGL(k_sparse_fill, dim3((unsigned)(n + 3) / 4), dim3(256), 0, st, y, n, stride, off, idx, val);
+    HIP_OK(hipGetLastError());
+    return 0;
+}
+
 // Position-weighted checksum of a word array: sum of (2i+1) * w_i (mod 2^64),
 // so a moved, dropped or changed word changes it.  Grid-stride; one 64-bit
 // atomic add per workgroup.

@@ -35,6 +35,7 @@ size_t keys_digit_limb_bytes(int spad, int ksteps, int nb);
 int launch_rows_put(const uint32_t *cl, const uint32_t *c0, int src_l, int R, int r0, int cap, int ldr, int l_store,
                     int ksteps, int32_t *A, uint32_t *c0s, int8_t *dig, hipStream_t st);
 int launch_keys_digits(const double *kd, int S, int K, int spad, int ksteps, int nb, int8_t *dig, hipStream_t st);
+int launch_keys_digits16(const int16_t *k16, int S, int K, int spad, int ksteps, int8_t *dig, hipStream_t st);
 int launch_contract_i8(const int8_t *A, int ksteps_a, const int8_t *B, int ksteps, int nb, int R, int S, int s,
                        uint32_t *D, hipStream_t st, int variant = 0, const uint32_t *crt_d0 = nullptr,
                        const uint32_t *crt_d1 = nullptr, uint32_t *kval = nullptr);
@@ -76,13 +77,15 @@ size_t frac_digit_bytes(int cap, int ksteps);
 // (int16 D) into ref [cap][ksteps x 32]
 int launch_rows_frac(const uint32_t *cl, const uint32_t *c0, int src_l, int R, int r0, int cap, int ksteps,
                      int8_t *dig, int16_t *ref, hipStream_t st);
-// keys: *neq set unless every coefficient is the same integer (within int16)
-// in all limbs; margin[v] = the bound M_v on |x / Q - V 2^-72| in units of
-// 2^-72 (M_v ~ sum_k |kd[0][v][k]| / 2), margin88[v] the same at 88 bits,
-// both times 2^widen, at most 2^62 (widen <= 62; > 0 only in tests, to send
-// many pairs to the exact kernel); k16 [S][K] = limb 0's values
-int launch_keys_frac(const double *kd, int S, int K, int widen, uint64_t *margin, uint64_t *margin88, int16_t *k16,
-                     int *neq, hipStream_t st);
+// keys of fused models (y slots beside the N columns) from sk [S][3][N]:
+// largest |coefficient| per limb into maxabs (cleared before); *neq set unless
+// every coefficient is the same integer in all limbs; margin[v] = the bound M_v
+// on |x / Q - V 2^-72| in units of 2^-72 (M_v ~ sum_k |B_v[k]| / 2),
+// margin88[v] the same at 88 bits, both times 2^widen, at most 2^62 (widen <=
+// 62; > 0 only in tests, to send many pairs to the exact kernel); k16 [S][K] =
+// limb 0's values
+int launch_keys_build(const uint32_t *sk, int S, int K, const SparseY &y, int widen, uint64_t *margin,
+                      uint64_t *margin88, int16_t *k16, unsigned int *maxabs, int *neq, hipStream_t st);
 // A: fraction digits at the first row (a multiple of 32), B: limb 0's
 // two-digit key store
 int launch_contract_frac(const int8_t *A, int ksteps_a, const int8_t *B, int ksteps, int R, int S, const FracOut &out,

@@ -190,28 +190,23 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
         return -1;
     }
     const int nS = m->l;
-    std::vector<int> off(nS + 1), idx;
-    std::vector<uint32_t> val;
-    int mx = -1;
-    for (int v = 0; v < nS; ++v) {
-        off[v] = (int)idx.size();
-        for (int i = 0; i < IPFE_L; ++i) {
-            const uint32_t yv = m->sv[(size_t)v * IPFE_L + i];
-            if (!yv) continue;
-            if (i >= L) {
-                ipfe_set_error("model: SV %d has feature %d beyond the key length %d", v, i, L);
-                return -1;
-            }
-            idx.push_back(i);
-            val.push_back(yv);
-            mx = std::max(mx, i);
-        }
+    // the vectors' entries, listed on the device (the host took longer to look
+    // through 2,000 vectors of 785 slots than the upload takes)
+    DevBuf<uint32_t> dense;
+    DevBuf<int> off;  // takes y_off's place once the model is accepted
+    DevBuf<unsigned int> info;  // slots in use, first entry past the keys; then largest values, limbs unequal
+    unsigned int h_info[6] = {};
+    if (dense.alloc((size_t)nS * IPFE_L) || info.alloc(6) || off.alloc((size_t)nS + 1)) return -1;
+    if (copy_to_device(dense.get(), m->sv, (size_t)nS * IPFE_L * 4, st)) return -1;
+    if (launch_sparse_count(dense.get(), nS, IPFE_L, L, off.get(), info.get(), st)) return -1;
+    HIP_OK(hipMemcpyAsync(h_info, info.get(), 8, hipMemcpyDeviceToHost, st));
+    if (sync_stream(st)) return -1;
+    if (h_info[1] != ~0u) {
+        ipfe_set_error("model: SV %d has feature %d beyond the key length %d", (int)(h_info[1] / IPFE_L),
+                       (int)(h_info[1] % IPFE_L), L);
+        return -1;
     }
-    off[nS] = (int)idx.size();
-    if (idx.empty()) {
-        idx.push_back(0);
-        val.push_back(0);
-    }
+    const int mx = (int)h_info[0] - 1;
     int nsv_sum = 0;
     for (int i = 0; i < m->nr_class; ++i) nsv_sum += m->nSV[i];
     if (nsv_sum != nS) {
@@ -222,27 +217,44 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
     // canonical, so the sum part joins the contraction (key = [-s', y]).
     const bool fz = mx < L - 1;
     const int kk = fz ? IPFE_N + ((mx + 1 + 15) / 16) * 16 : IPFE_N;
-    if (y_off.alloc(off.size()) || y_idx.alloc(idx.size()) || y_val.alloc(val.size()) ||
-        sk.alloc((size_t)nS * kPoly) || kd.alloc((size_t)3 * nS * kk))
-        return -1;
-    HIP_OK(hipMemcpyAsync(y_off.get(), off.data(), off.size() * 4, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(y_idx.get(), idx.data(), idx.size() * 4, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(y_val.get(), val.data(), val.size() * 4, hipMemcpyHostToDevice, st));
+    const size_t entries = (size_t)nS * std::max(1, mx + 1);  // at most
+    if (y_idx.alloc(entries) || y_val.alloc(entries) || sk.alloc((size_t)nS * kPoly)) return -1;
+    y_off.swap(off);
+    if (launch_sparse_fill(dense.get(), nS, IPFE_L, y_off.get(), y_idx.get(), y_val.get(), st)) return -1;
     y.off = y_off.get();
     y.idx = y_idx.get();
     y.val = y_val.get();
     y.len = L;
     if (launch_fold(y, nS, msk_dev, sk.get(), device()->barrett, st)) return -1;
-    DevBuf<unsigned int> d_max;
-    if (d_max.alloc(3)) return -1;
-    if (launch_fill_i32((int *)d_max.get(), 0, 3, st)) return -1;
-    if (launch_contract_keys(sk.get(), nS, kk, fz ? -1 : 1, y, kd.get(), d_max.get(), st)) return -1;
-    HIP_OK(hipMemcpyAsync(maxabs, d_max.get(), 12, hipMemcpyDeviceToHost, st));
+    kdig.reset();
+    margin.reset();
+    margin88.reset();
+    k16.reset();
+    kd.reset();
+    S = nS;
+    kkey = kk;
+    fused = fz;
+    if (launch_fill_i32((int *)info.get() + 2, 0, 4, st)) return -1;
+    if (fz) {
+        // (CUFE_FRAC_WIDEN=w, for tests: margins 2^w times wider, so that many
+        // pairs go to the exact kernel)
+        const char *wv = getenv("CUFE_FRAC_WIDEN");
+        if (margin.alloc(nS) || margin88.alloc(nS) || k16.alloc((size_t)nS * kk) ||
+            launch_keys_build(sk.get(), nS, kk, y, wv ? atoi(wv) : 0, margin.get(), margin88.get(), k16.get(),
+                              info.get() + 2, (int *)info.get() + 5, st))
+            return -1;
+    } else {
+        if (kd.alloc((size_t)3 * nS * kk) ||
+            launch_contract_keys(sk.get(), nS, kk, 1, y, kd.get(), info.get() + 2, st))
+            return -1;
+    }
+    HIP_OK(hipMemcpyAsync(h_info + 2, info.get() + 2, 16, hipMemcpyDeviceToHost, st));
     const int npairs = m->nr_class * (m->nr_class - 1) / 2;
     if (coef.alloc((size_t)(m->nr_class - 1) * nS) || rho.alloc(npairs)) return -1;
     HIP_OK(hipMemcpyAsync(coef.get(), m->sv_coef, sizeof(double) * (m->nr_class - 1) * nS, hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(rho.get(), m->rho, sizeof(double) * npairs, hipMemcpyHostToDevice, st));
     if (sync_stream(st)) return -1;
+    for (int s = 0; s < 3; ++s) maxabs[s] = h_info[2 + s];
     SvmModelDev md{};
     md.nr_class = m->nr_class;
     int start = 0;
@@ -292,39 +304,41 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
     const unsigned int mx3 = std::max(maxabs[0], std::max(maxabs[1], maxabs[2]));
     nb = mx3 <= I8_KEY_MAX2 ? 2 : (mx3 <= I8_KEY_MAX3 ? 3 : 0);
     i8 = nb > 0;
-    kdig.reset();
-    margin.reset();
-    margin88.reset();
-    k16.reset();
-    frac = false;
+    // the fraction form needs keys that are the same integers in every limb
+    // (and its margins, int16 values and digits come from one pass over them);
+    // other keys go through the fp64 operand
+    frac = fz && nb == 2 && h_info[5] == 0;
+    if (!frac) {
+        margin.reset();
+        margin88.reset();
+        k16.reset();
+        if (ensure_kd(st)) return -1;
+    }
     if (i8) {
         spad = (nS + 127) / 128 * 128;
         ksteps = (kk + 31) / 32;
         if (kdig.alloc(3 * keys_digit_limb_bytes(spad, ksteps, nb))) return -1;
-        if (launch_keys_digits(kd.get(), nS, kk, spad, ksteps, nb, kdig.get(), st) || sync_stream(st)) return -1;
-    }
-    if (i8 && nb == 2 && fz) {
-        // the fraction form needs keys that are the same integers in every limb
-        // (CUFE_FRAC_WIDEN=w, for tests: margins 2^w times wider, so that many
-        // pairs go to the exact kernel)
-        DevBuf<int> neq;
-        int h_neq = 1;
-        const char *wv = getenv("CUFE_FRAC_WIDEN");
-        if (margin.alloc(nS) || margin88.alloc(nS) || k16.alloc((size_t)nS * kk) || neq.alloc(1) ||
-            launch_fill_i32(neq.get(), 0, 1, st) ||
-            launch_keys_frac(kd.get(), nS, kk, wv ? atoi(wv) : 0, margin.get(), margin88.get(), k16.get(), neq.get(),
-                             st))
+        if (frac ? launch_keys_digits16(k16.get(), nS, kk, spad, ksteps, kdig.get(), st)
+                 : launch_keys_digits(kd.get(), nS, kk, spad, ksteps, nb, kdig.get(), st))
             return -1;
-        HIP_OK(hipMemcpyAsync(&h_neq, neq.get(), 4, hipMemcpyDeviceToHost, st));
         if (sync_stream(st)) return -1;
-        frac = h_neq == 0;
     }
-    S = nS;
     nr_class = m->nr_class;
     maxidx = mx;
     l_key = L;
-    kkey = kk;
-    fused = fz;
+    return 0;
+}
+
+// The fp64 operand, complete when this returns (whichever stream reads it).
+int Model::ensure_kd(hipStream_t st) const
+{
+    if (kd.get()) return 0;
+    DevBuf<unsigned int> mx;
+    if (mx.alloc(3) || launch_fill_i32((int *)mx.get(), 0, 3, st) || kd.alloc((size_t)3 * S * kkey)) return -1;
+    if (launch_contract_keys(sk.get(), S, kkey, fused ? -1 : 1, y, kd.get(), mx.get(), st) || sync_stream(st)) {
+        kd.reset();
+        return -1;
+    }
     return 0;
 }
 
@@ -535,7 +549,8 @@ int predict_rows(const Model &m, const RowStore &rs, int row0, int nrows, Scratc
         }
         for (int s = 0; s < 3 && !split && !frac; ++s) {
             const int32_t *As = rs.A.get() + ((size_t)s * rs.cap + r0) * rs.ldr;
-            const double *Bs = m.kd.get() + (size_t)s * S * m.kkey;
+            if (!i8 && m.ensure_kd(st)) return -1;
+            const double *Bs = i8 ? nullptr : m.kd.get() + (size_t)s * S * m.kkey;
             uint32_t *Ds = sc.D.get() + (size_t)s * R * S;
             int rc;
             if (i8)

@@ -26,7 +26,9 @@ struct Model {
     DevBuf<uint32_t> y_val;
     SparseY y{};
     DevBuf<uint32_t> sk;  // [S][3][N]
-    DevBuf<double> kd;    // [3][S][kkey]
+    // [3][S][kkey] fp64: built with the model where its digits are made from it
+    // (three digits, unfused keys or none), else when a kernel first reads it
+    mutable DevBuf<double> kd;
     DevBuf<double> coef, rho;
     DevBuf<int32_t> icoef;  // integer coefficients for the exact two-class vote (else empty)
     SvmModelDev mdev{};
@@ -43,7 +45,8 @@ struct Model {
     DevBuf<int16_t> k16;  // [S][kkey] key values for the fraction form's exact kernel
 
     int build(const uint32_t *msk_dev, int l_key, const cufe_svm_model *m, hipStream_t st);
-    size_t bytes() const;
+    int ensure_kd(hipStream_t st) const;
+    size_t bytes() const;  // kd included
 };
 
 // Compact encrypted rows of l slots: c_L and coefficient 0 of c_0..c_{l-1},

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <utility>
 #include <vector>
 
 #include "host_tables.h"
@@ -65,6 +66,11 @@ struct DevBuf {
         return 0;
     }
     T *get() const { return p; }
+    void swap(DevBuf &o)
+    {
+        std::swap(p, o.p);
+        std::swap(n, o.n);
+    }
 };
 
 // One Gaussian stream request for the sampler driver.
