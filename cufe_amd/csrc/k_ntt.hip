@@ -195,7 +195,8 @@ __global__ __launch_bounds__(NTT_THREADS) void k_enc_poly(const EncItem *__restr
 // operands in [0, q].  One workgroup keeps the limb in registers and LDS from
 // sk to d: 48 KiB of HBM a limb, where separate transform, product, inverse and
 // difference kernels moved 192 KiB and needed c_L's transform copied per key
-// (100 keys: 22 us for 31 in four kernels and 99 copies of 2 us each).
+// (100 keys: 20 us for 31 in four kernels and 99 copies of 2 us each; loads at
+// their place of use: 22).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(NTT_THREADS) void k_dec_poly(const uint32_t *__restrict__ chat,
                                                            const uint32_t *__restrict__ sk, uint32_t *__restrict__ d,
@@ -205,17 +206,20 @@ __global__ __launch_bounds__(NTT_THREADS) void k_dec_poly(const uint32_t *__rest
     __shared__ uint32_t lds[NTT_LDS_WORDS];
     const int z = blockIdx.x, s = z % 3, tid = threadIdx.x;
     const uint32_t q = qmod(s);
-    uint32_t x[16];
+    uint32_t *dz = d + (size_t)z * IPFE_N;
+    uint32_t x[16], c[16], sum[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) x[r] = sk[(size_t)z * IPFE_N + posA(tid, r)];
+    for (int r = 0; r < 16; ++r) {
+        x[r] = sk[(size_t)z * IPFE_N + posA(tid, r)];
+        c[r] = chat[s * IPFE_N + posA(tid, r)];
+        sum[r] = dz[posA(tid, r)];
+    }
     if (__syncthreads_or(any_eq_q(x, q)))
         ntt_fwd_block<true>(x, lds, tw_fwd(tw_all, s), twp_fwd(tw_all, s), q);
     else
         ntt_fwd_block<false>(x, lds, tw_fwd(tw_all, s), twp_fwd(tw_all, s), q);
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-        x[r] = mul_exact(chat[s * IPFE_N + posA(tid, r)], x[r], s, bc.mu_hi[s], bc.mu_lo[s]);
-    uint32_t *dz = d + (size_t)z * IPFE_N;
+    for (int r = 0; r < 16; ++r) x[r] = mul_exact(c[r], x[r], s, bc.mu_hi[s], bc.mu_lo[s]);
     if (__syncthreads_or(any_eq_q(x, q))) {
         ntt_inv_block<true>(x, lds, tw_inv(tw_all, s), twp_inv(tw_all, s), q);
 #pragma unroll
@@ -226,7 +230,7 @@ __global__ __launch_bounds__(NTT_THREADS) void k_dec_poly(const uint32_t *__rest
         for (int r = 0; r < 16; ++r) x[r] = scale_ninv<false>(x[r], nc.ninv[s], nc.ninvp[s], nc.flag[s], q);
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) dz[posA(tid, r)] = sub_q(dz[posA(tid, r)], x[r], q);
+    for (int r = 0; r < 16; ++r) dz[posA(tid, r)] = sub_q(sum[r], x[r], q);
 }
 
 // ---------------------------------------------------------------------------

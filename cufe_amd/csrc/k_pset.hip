@@ -6,6 +6,7 @@
 // every set.
 #include <stdio.h>
 
+#include "fold_dev.h"
 #include "kernels_pset.h"
 #include "ntt_gen.h"
 
@@ -13,7 +14,12 @@ namespace ipfe {
 
 namespace {
 
-// Shape of the transforms inside the fused kernels, per log2 N.
+constexpr int FOLD_CHUNK = 16384;  // k_ps_fold: slots of a wave's 64-bit sums
+
+// Shape of the transforms inside the fused kernels, per log2 N: 16 coefficients a
+// thread, what setup's two transforms and their factors leave registers for.  At
+// N = 8192, 512 threads for 256 of 32: setup of 785 slots 341 -> 258 us, of 63
+// 31.4 -> 23.2; encryption 214 -> 167 and 25.7 -> 15.5 (with the noise loaded first).
 template <int LOGN>
 struct FusedShape;
 template <>
@@ -28,8 +34,8 @@ struct FusedShape<12> {
 };
 template <>
 struct FusedShape<13> {
-    static constexpr int T = 256;
-    using RAD = Rad<5, 4, 4>;
+    static constexpr int T = 512;
+    using RAD = Rad<4, 3, 3, 3>;
 };
 
 // mul_mod(a, b) for b with Shoup companion bp; exact for a, b in [0, q].
@@ -108,10 +114,12 @@ __global__ __launch_bounds__(FusedShape<LOGN>::T) void k_ps_enc_poly(const uint3
     const uint32_t *pk = mpk + ((size_t)i * ps.nmod + s) * N;
     const uint32_t *rh = rhat + ((size_t)b * ps.nmod + s) * N;
     const uint32_t *rhp = rhatp + ((size_t)b * ps.nmod + s) * N;
-    uint32_t v[E], rv[E], rvp[E];
+    uint32_t *cz = c + (size_t)z * N;
+    uint32_t v[E], rv[E], rvp[E], f[E];
     bool hq = false;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
+        f[e] = cz[G::first_idx(t, e)];
         v[e] = pk[G::last_idx(t, e)];
         rv[e] = rh[G::last_idx(t, e)];
         rvp[e] = rhp[G::last_idx(t, e)];
@@ -122,7 +130,6 @@ __global__ __launch_bounds__(FusedShape<LOGN>::T) void k_ps_enc_poly(const uint3
         const uint32_t mj = ps_mod_prime(ps, x_msg[(size_t)b * l + i], s);
         madd = ps_mod_prime(ps, (uint64_t)mj * ps.scale[s], s);
     }
-    uint32_t *cz = c + (size_t)z * N;
     const bool exact = __syncthreads_or(hq);
     if (exact) {
 #pragma unroll
@@ -140,7 +147,7 @@ __global__ __launch_bounds__(FusedShape<LOGN>::T) void k_ps_enc_poly(const uint3
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int idx = G::first_idx(t, e);
-        uint32_t w = add_q(v[e], cz[idx], q);
+        uint32_t w = add_q(v[e], f[e], q);
         if (i < l) w = ps_mod_prime(ps, (uint64_t)(uint32_t)(w + madd), s);  // mod_prime(c + m), src/rlwe_sife.c:173
         cz[idx] = w;
     }
@@ -148,24 +155,48 @@ __global__ __launch_bounds__(FusedShape<LOGN>::T) void k_ps_enc_poly(const uint3
 
 // out[v][s][k] = fold over i < l of mod_prime(y_v[i] P[i][s][k] + acc) -- the
 // dense loops of rlwe_sife_keygen (src/rlwe_sife.c:232-240, P = msk) and of
-// rlwe_sife_decrypt_gmp (:265-273, P = c), literally, per limb.
-__global__ void k_ps_fold(const uint32_t *__restrict__ y, int nvec, int l, const uint32_t *__restrict__ P,
-                          uint32_t *__restrict__ out, PsetDev ps)
+// rlwe_sife_decrypt_gmp (:265-273, P = c), per limb, as a sum (fold_dev.h).  One
+// vector fills few waves and its loads are the latency to hide: 64 coefficients a
+// workgroup, the slots dealt to four waves, eight loads in flight each.  One
+// vector of 63 slots at N = 8192, 4 limbs: 8.5 us (57 as one chain of folds
+// a coefficient).  Grid nvec nmod N / 64.
+__global__ __launch_bounds__(64 * FOLD_WAVES) void k_ps_fold(const uint32_t *__restrict__ y, int l,
+                                                            const uint32_t *__restrict__ P,
+                                                            uint32_t *__restrict__ out, PsetDev ps)
 {
+    __shared__ uint32_t part[FOLD_WAVES][64];
+    const int per_limb = ps.N / 64, limb = (int)(blockIdx.x / per_limb);  // limb s of vector v: v nmod + s
+    const int v = limb / ps.nmod, s = limb % ps.nmod, lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const size_t per_vec = (size_t)ps.nmod * ps.N;
-    const size_t total = (size_t)nvec * per_vec;
-    for (size_t w = (size_t)blockIdx.x * blockDim.x + threadIdx.x; w < total; w += (size_t)gridDim.x * blockDim.x) {
-        const int v = (int)(w / per_vec);
-        const size_t sk = w % per_vec;
-        const int s = (int)(sk / ps.N);
-        const uint32_t *yv = y + (size_t)v * l;
-        uint32_t acc = 0;
-        for (int i = 0; i < l; ++i) {
-            const uint64_t yi = ps_mod_prime(ps, yv[i], s);
-            acc = ps_mod_prime(ps, yi * P[(size_t)i * per_vec + sk] + acc, s);
-        }
-        out[w] = acc;
+    const int k = (int)(blockIdx.x % per_limb) * 64 + lane;
+    const uint32_t q = ps.q[s], mu_hi = ps.mu_hi[s], mu_lo = ps.mu_lo[s];
+    const uint32_t *base = P + (size_t)s * ps.N + k, *yv = y + (size_t)v * l;
+    auto y_mod = [&](int i) { return yv[i] >> 16 ? ps_mod_prime(ps, yv[i], s) : yv[i]; };  // every q is above 2^16
+    uint64_t sum = 0;
+    // FOLD_CHUNK slots at a time stay within FoldSum
+    for (int i0 = w; i0 < l; i0 += FOLD_WAVES * FOLD_CHUNK) {
+        const int i1 = l - i0 < FOLD_WAVES * FOLD_CHUNK ? l : i0 + FOLD_WAVES * FOLD_CHUNK;
+        FoldSum acc;
+#pragma unroll 8
+        for (int i = i0; i < i1; i += FOLD_WAVES) acc.add(y_mod(i), base[(size_t)i * per_vec]);
+        sum += acc.value(q, mu_hi, mu_lo);
     }
+    part[w][lane] = (uint32_t)(sum % q);
+    __syncthreads();
+    if (w) return;
+    sum = 0;
+#pragma unroll
+    for (int j = 0; j < FOLD_WAVES; ++j) sum += part[j][lane];
+    uint32_t r = (uint32_t)(sum % q);
+    if (r == 0)
+        r = fold_zero(l, l, q, [&](uint64_t m) { return ps_mod_prime(ps, m, s); },
+                      [&](int e, uint32_t &yy, uint32_t &vv, int &i) {
+                          i = e;
+                          yy = ps_mod_prime(ps, yv[e], s);
+                          vv = base[(size_t)e * per_vec];
+                      });
+    out[(size_t)limb * ps.N + k] = r;
 }
 
 // Shoup companions floor(v 2^32 / q) of [n][nmod][N] residues (q stands for 0).
@@ -180,23 +211,50 @@ __global__ void k_ps_shoup(const uint32_t *__restrict__ v, uint32_t *__restrict_
     }
 }
 
-// out = mul_mod(a, b) (point_mul, src/ntt.c:28-36), exact for operands in [0, q].
-__global__ void k_ps_point_mul(const uint32_t *__restrict__ a, const uint32_t *__restrict__ b,
-                               uint32_t *__restrict__ out, size_t total, PsetDev ps)
+// Second half of rlwe_sife_decrypt_gmp (src/rlwe_sife.c:274-284) for limb s of
+// key v (block z = v nmod + s), the transforms given: d = sub_mod(d,
+// INTT(chat (.) skhat)), each product mul_mod exact for operands in [0, q]
+// (point_mul, src/ntt.c:28-36; poly_sub_mod, src/arith_rns.c:95-103).  A single
+// key has nmod workgroups and is all latency: every load is issued before the
+// transform, and product, inverse and difference are one launch.  At N = 8192, 4
+// limbs 12 us, for 4 + 10.4 + 3.4 in three and 4.5 for a copy of c_L's transform.
+template <int LOGN>
+__global__ __launch_bounds__(FusedShape<LOGN>::T) void k_ps_dec_poly(const uint32_t *__restrict__ chat,
+                                                                   const uint32_t *__restrict__ skhat,
+                                                                   uint32_t *__restrict__ d,
+                                                                   const uint32_t *__restrict__ tw_all, PsetDev ps)
 {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-        const int s = (int)((i / ps.N) % ps.nmod);
-        out[i] = ps_mul_exact(ps, a[i], b[i], s);
+    using G = NttGen<LOGN, FusedShape<LOGN>::T, typename FusedShape<LOGN>::RAD>;
+    constexpr int N = G::N, E = G::E;
+    __shared__ uint32_t lds[G::LDS_WORDS];
+    const int z = blockIdx.x, s = z % ps.nmod, t = threadIdx.x;
+    const uint32_t q = ps.q[s];
+    const uint32_t *tw = tw_all + (size_t)(2 * ps.nmod + s) * N, *twp = tw_all + (size_t)(3 * ps.nmod + s) * N;
+    uint32_t *dz = d + (size_t)z * N;
+    uint32_t x[E], c[E], sum[E];
+    bool hq = false;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        x[e] = skhat[(size_t)z * N + G::last_idx(t, e)];
+        c[e] = chat[(size_t)s * N + G::last_idx(t, e)];
+        sum[e] = dz[G::first_idx(t, e)];
     }
-}
-
-// d = sub_mod(d, prod) (poly_sub_mod, src/arith_rns.c:95-103).
-__global__ void k_ps_sub(uint32_t *__restrict__ d, const uint32_t *__restrict__ prod, size_t total, PsetDev ps)
-{
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-        const int s = (int)((i / ps.N) % ps.nmod);
-        d[i] = sub_q(d[i], prod[i], ps.q[s]);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        x[e] = ps_mul_exact(ps, c[e], x[e], s);
+        hq |= x[e] == q;
     }
+    if (__syncthreads_or(hq)) {
+        G::template inv<true>(x, lds, tw, twp, q, t);
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] = scale_ninv<true>(x[e], ps.ninv[s], ps.ninvp[s], ps.ninvf[s], q);
+    } else {
+        G::template inv<false>(x, lds, tw, twp, q, t);
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] = scale_ninv<false>(x[e], ps.ninv[s], ps.ninvp[s], ps.ninvf[s], q);
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) dz[G::first_idx(t, e)] = sub_q(sum[e], x[e], q);
 }
 
 // CRT + rounding of coefficient `coef` (all coefficients when coef < 0) of
@@ -272,9 +330,13 @@ int ps_launch_enc_poly(const PsetState &st, const uint32_t *mpk, const uint32_t 
 int ps_launch_fold(const PsetState &st, const uint32_t *y, int nvec, int l, const uint32_t *P, uint32_t *out,
                    hipStream_t s)
 {
-    const size_t total = (size_t)nvec * st.dev.nmod * st.dev.N;
-    if (total == 0) return 0;
-    hipLaunchKernelGGL(k_ps_fold, dim3(grid_for(total)), dim3(256), 0, s, y, nvec, l, P, out, st.dev);
+    const size_t wgs = (size_t)nvec * st.dev.nmod * (st.dev.N / 64);
+    if (wgs == 0) return 0;
+    if (wgs >> 31) {
+        ipfe_set_error("fold: %d vectors are too many", nvec);
+        return -1;
+    }
+    hipLaunchKernelGGL(k_ps_fold, dim3((unsigned)wgs), dim3(64 * FOLD_WAVES), 0, s, y, l, P, out, st.dev);
     HIP_OK(hipGetLastError());
     return 0;
 }
@@ -287,19 +349,19 @@ int ps_launch_shoup(const PsetState &st, const uint32_t *v, uint32_t *vp, size_t
     return 0;
 }
 
-int ps_launch_point_mul(const PsetState &st, const uint32_t *a, const uint32_t *b, uint32_t *out, size_t total,
-                        hipStream_t s)
+int ps_launch_dec_poly(const PsetState &st, const uint32_t *chat, const uint32_t *skhat, uint32_t *d, int nvec,
+                       hipStream_t s)
 {
-    if (total == 0) return 0;
-    hipLaunchKernelGGL(k_ps_point_mul, dim3(grid_for(total)), dim3(256), 0, s, a, b, out, total, st.dev);
-    HIP_OK(hipGetLastError());
-    return 0;
-}
-
-int ps_launch_sub(const PsetState &st, uint32_t *d, const uint32_t *prod, size_t total, hipStream_t s)
-{
-    if (total == 0) return 0;
-    hipLaunchKernelGGL(k_ps_sub, dim3(grid_for(total)), dim3(256), 0, s, d, prod, total, st.dev);
+    if (nvec <= 0) return 0;
+    const dim3 grid((unsigned)((size_t)nvec * st.dev.nmod));
+#define DEC(LOGN)                                                                                                      hipLaunchKernelGGL(k_ps_dec_poly<LOGN>, grid, dim3(FusedShape<LOGN>::T), 0, s, chat, skhat, d, st.tw, st.dev);     break
+    switch (st.dev.logN) {
+    case 11: DEC(11);
+    case 12: DEC(12);
+    case 13: DEC(13);
+    default: ipfe_set_error("decrypt: unsupported N"); return -1;
+    }
+#undef DEC
     HIP_OK(hipGetLastError());
     return 0;
 }

@@ -13,6 +13,7 @@
 #include <algorithm>
 
 #include "crt_dev.h"
+#include "fold_dev.h"
 #include "kernels.h"
 
 namespace ipfe {
@@ -20,67 +21,16 @@ namespace ipfe {
 // y_v[i] mod q_s as the fold takes it; below 2^16 it is y itself
 __device__ __forceinline__ uint32_t fold_y(uint32_t y, int s) { return y >> 16 ? mod_prime_exact(y, s) : y; }
 
-// The fold's result where its sum is 0 mod q: entries 0 .. n-1 with term(e, y,
-// v, i) giving y mod q, v and the slot i of entry e (ascending; slots between
-// entries hold y = 0, which only map acc = q to 0), len slots.  Before the last
-// entry whose product is not 0 mod q, acc is the canonical residue that cancels
-// it, whatever came before; from there on the fold is run literally.  (Sums of
-// small keys are 0 often enough, 10 coefficients of 128 keys over 785 slots,
-// that running the whole fold there took that kernel 205 us instead of 62.)
-template <class Term>
-__device__ uint32_t fold_zero(int n, int len, int s, Term term)
-{
-    const uint32_t q = qmod(s);
-    uint32_t y, v;
-    int i, e = n - 1;
-    uint64_t t = 0;
-    for (; e >= 0; --e) {
-        term(e, y, v, i);
-        t = (uint64_t)y * v % q;
-        if (t) break;
-    }
-    uint32_t acc = e >= 0 ? q - (uint32_t)t : 0u;
-    int last = -1;
-    if (e >= 0) {
-        acc = mod_prime_exact((uint64_t)y * v + acc, s);
-        last = i;
-    }
-    for (++e; e < n; ++e) {
-        term(e, y, v, i);
-        if (i > last + 1 && acc == q) acc = 0;
-        acc = mod_prime_exact((uint64_t)y * v + acc, s);
-        last = i;
-    }
-    if (last < len - 1 && acc == q) acc = 0;
-    return acc;
-}
-
-struct FoldSum {
-    uint64_t lo = 0, hi = 0;
-    __device__ __forceinline__ void add(uint32_t y, uint32_t v)
-    {
-        lo += (uint64_t)(y & 0xffffu) * v;
-        if (y >> 16) hi += (uint64_t)(y >> 16) * v;
-    }
-    __device__ __forceinline__ uint32_t value(int s, const BarrettConsts &bc) const
-    {
-        const uint64_t h = hi ? reduce64(hi, qmod(s), bc.mu_hi[s], bc.mu_lo[s]) : 0u;
-        return reduce64(lo + (h << 16), qmod(s), bc.mu_hi[s], bc.mu_lo[s]);
-    }
-};
-
 // fold_zero of vector v at the coefficient base points at
 __device__ uint32_t fold_zero_sparse(const SparseY &y, int v, int s, const uint32_t *base)
 {
     const int e0 = y.off[v];
-    return fold_zero(y.off[v + 1] - e0, y.len, s, [&](int e, uint32_t &yy, uint32_t &vv, int &i) {
+    return fold_zero(y.off[v + 1] - e0, y.len, qmod(s), [s](uint64_t m) { return mod_prime_exact(m, s); }, [&](int e, uint32_t &yy, uint32_t &vv, int &i) {
         i = y.idx[e0 + e];
         yy = fold_y(y.val[e0 + e], s);
         vv = base[(size_t)i * 3 * IPFE_N];
     });
 }
-
-constexpr int FOLD_WAVES = 4;  // waves of a workgroup, each with its share of the terms
 
 // Few sparse vectors: 64 coefficients a workgroup, the entries dealt to four
 // waves, so that one vector's 12,288 chains are 768 waves of a quarter of the
@@ -98,7 +48,7 @@ __global__ __launch_bounds__(64 * FOLD_WAVES) void k_fold_few(SparseY y, const u
 #pragma unroll 8
     for (int e = e0 + w; e < e1; e += FOLD_WAVES)
         acc.add(fold_y(y.val[e], s), base[(size_t)y.idx[e] * 3 * IPFE_N]);
-    part[w][lane] = acc.value(s, bc);
+    part[w][lane] = acc.value(qmod(s), bc.mu_hi[s], bc.mu_lo[s]);
     __syncthreads();
     if (w) return;
     uint64_t t = 0;
@@ -132,7 +82,7 @@ __global__ __launch_bounds__(256) void k_fold_many(SparseY y, const uint32_t *__
     uint32_t r[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-        r[u] = acc[u].value(s, bc);
+        r[u] = acc[u].value(qmod(s), bc.mu_hi[s], bc.mu_lo[s]);
         if (r[u] == 0) r[u] = fold_zero_sparse(y, v, s, base + u);
     }
     *reinterpret_cast<uint4 *>(out + ((size_t)v * 3 + s) * IPFE_N + k) = make_uint4(r[0], r[1], r[2], r[3]);
@@ -184,7 +134,7 @@ __global__ __launch_bounds__(64 * FOLD_WAVES) void k_fold_dense(const uint32_t *
         uint32_t r = (uint32_t)(t % qmod(s));
         if (r == 0) {
             const uint32_t *yv = y + (size_t)(v0 + j) * len;
-            r = fold_zero(len, len, s, [&](int e, uint32_t &yy, uint32_t &vv, int &i) {
+            r = fold_zero(len, len, qmod(s), [s](uint64_t m) { return mod_prime_exact(m, s); }, [&](int e, uint32_t &yy, uint32_t &vv, int &i) {
                 i = e;
                 yy = yv[e];
                 vv = base[(size_t)e * 3 * IPFE_N];

@@ -61,9 +61,9 @@ int ps_launch_enc_poly(const PsetState &st, const uint32_t *mpk, const uint32_t 
 int ps_launch_fold(const PsetState &st, const uint32_t *y, int nvec, int l, const uint32_t *P, uint32_t *out,
                    hipStream_t s);
 int ps_launch_shoup(const PsetState &st, const uint32_t *v, uint32_t *vp, size_t total, hipStream_t s);
-int ps_launch_point_mul(const PsetState &st, const uint32_t *a, const uint32_t *b, uint32_t *out, size_t total,
-                        hipStream_t s);
-int ps_launch_sub(const PsetState &st, uint32_t *d, const uint32_t *prod, size_t total, hipStream_t s);
+// d [nvec][nmod][N] -= INTT(chat (.) skhat), chat [nmod][N], skhat [nvec][nmod][N] in the NTT domain
+int ps_launch_dec_poly(const PsetState &st, const uint32_t *chat, const uint32_t *skhat, uint32_t *d, int nvec,
+                       hipStream_t s);
 // ntrans limb transforms ([npoly][nmod][N], transform z on limb z % nmod) of
 // set st with its tuned shape (in == out allowed).
 int ps_ntt(const PsetState &st, bool inverse, const uint32_t *in, uint32_t *out, int ntrans, hipStream_t s);

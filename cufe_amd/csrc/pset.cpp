@@ -437,24 +437,19 @@ extern "C" int cufe_ps_decrypt(int pset, const uint32_t *c, const uint32_t *y, c
     if (repeat == 0) return 0;
     hipStream_t s = device()->stream;
     const size_t pw = poly_words(*st), nk = (size_t)repeat * pw;
-    DevBuf<uint32_t> d_c, d_y, d_sk, d_d, d_cl;
-    if (d_c.alloc((size_t)(l + 1) * pw) || d_y.alloc((size_t)repeat * l) || d_sk.alloc(nk) || d_d.alloc(nk) ||
-        d_cl.alloc(nk))
+    DevBuf<uint32_t> d_c, d_y, d_sk, d_d;
+    if (d_c.alloc((size_t)(l + 1) * pw) || d_y.alloc((size_t)repeat * l) || d_sk.alloc(nk) || d_d.alloc(nk))
         return -1;
     if (copy_to_device(d_c.get(), c, (size_t)(l + 1) * pw * 4, s)) return -1;
     if (copy_to_device(d_y.get(), y, (size_t)repeat * l * 4, s)) return -1;
     if (copy_to_device(d_sk.get(), sk, nk * 4, s)) return -1;
     // sum part: fold over the l slots
     if (ps_launch_fold(*st, d_y.get(), repeat, l, d_c.get(), d_d.get(), s)) return -1;
-    // poly_mul_ntt(c_L, sk_v) (src/ntt.c:10-26): NTT(c_L) once, copied per key
+    // - poly_mul_ntt(c_L, sk_v) (src/ntt.c:10-26), NTT(c_L) once
     uint32_t *cl = d_c.get() + (size_t)l * pw;
-    if (ps_ntt(*st, false, cl, cl, st->dev.nmod, s)) return -1;
-    for (int v = 0; v < repeat; ++v)
-        HIP_OK(hipMemcpyAsync(d_cl.get() + (size_t)v * pw, cl, pw * 4, hipMemcpyDeviceToDevice, s));
-    if (ps_ntt(*st, false, d_sk.get(), d_sk.get(), repeat * st->dev.nmod, s) ||
-        ps_launch_point_mul(*st, d_cl.get(), d_sk.get(), d_cl.get(), nk, s) ||
-        ps_ntt(*st, true, d_cl.get(), d_cl.get(), repeat * st->dev.nmod, s) ||
-        ps_launch_sub(*st, d_d.get(), d_cl.get(), nk, s))
+    if (ps_ntt(*st, false, cl, cl, st->dev.nmod, s) ||
+        ps_ntt(*st, false, d_sk.get(), d_sk.get(), repeat * st->dev.nmod, s) ||
+        ps_launch_dec_poly(*st, cl, d_sk.get(), d_d.get(), repeat, s))
         return -1;
     if (copy_to_host(d, d_d.get(), nk * 4, s)) return -1;
     return sync_stream(s);
