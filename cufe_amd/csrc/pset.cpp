@@ -382,7 +382,6 @@ extern "C" int cufe_ps_encrypt(int pset, const uint32_t *m, const uint32_t *mpk,
     if (d_mpk.alloc((size_t)(l + 1) * pw) || d_c.alloc((size_t)repeat * ct) || d_r.alloc((size_t)repeat * pw) ||
         d_rp.alloc((size_t)repeat * pw) || d_x.alloc((size_t)repeat * l + 1))
         return -1;
-    if (copy_to_device(d_mpk.get(), mpk, (size_t)(l + 1) * pw * 4, s)) return -1;
     if (l > 0 && copy_to_device(d_x.get(), m, (size_t)repeat * l * 4, s)) return -1;
     const PsetSpec &sp = *pset_spec(pset);
     std::vector<StreamReq> reqs;
@@ -393,7 +392,10 @@ extern "C" int cufe_ps_encrypt(int pset, const uint32_t *m, const uint32_t *mpk,
         reqs.push_back(make_stream_ps(sp, seed2, nonce, 2, 2, d_r.get() + (size_t)b * pw, cb + (size_t)l * pw, 0));
         if (l > 0) reqs.push_back(make_stream_ps(sp, seed3, nonce, 3, l, cb, cb + pw, (long long)pw));
     }
-    if (run_gauss(reqs, s)) return -1;
+    // the public key is uploaded beside the sampling
+    if (run_gauss(reqs, s, kGaussScratch,
+                  [&] { return copy_to_device_beside(d_mpk.get(), mpk, (size_t)(l + 1) * pw * 4, s); }))
+        return -1;
     if (ps_ntt(*st, false, d_r.get(), d_r.get(), repeat * st->dev.nmod, s) ||
         ps_launch_shoup(*st, d_r.get(), d_rp.get(), (size_t)repeat * pw, s) ||
         ps_launch_enc_poly(*st, d_mpk.get(), d_r.get(), d_rp.get(), d_x.get(), d_c.get(), repeat, l, s))

@@ -366,20 +366,26 @@ int GaussPlan::check(hipStream_t st, int *overflow, int *need_full)
     return 0;
 }
 
-static int run_gauss_group(const StreamReq *reqs, int n, int level, hipStream_t st, int *overflow)
+static int run_gauss_group(const StreamReq *reqs, int n, int level, hipStream_t st, int *overflow,
+                           std::function<int()> &beside)
 {
     GaussPlan p;
     if (p.build(reqs, n, level) || p.alloc_scratch()) return -1;
     for (;;) {
         int need_full = 0;
-        if (p.upload(st) || p.launch(st) || p.check(st, overflow, &need_full)) return -1;
+        if (p.upload(st) || p.launch(st)) return -1;
+        if (beside && beside()) return -1;
+        beside = nullptr;
+        if (p.check(st, overflow, &need_full)) return -1;
         if (!need_full || p.full) return 0;
         p.full = 1;  // a chunk needed the AES blocks the default set omits
     }
 }
 
-int run_gauss(const std::vector<StreamReq> &reqs, hipStream_t st, size_t scratch_budget)
+int run_gauss(const std::vector<StreamReq> &reqs, hipStream_t st, size_t scratch_budget,
+              const std::function<int()> &beside)
 {
+    std::function<int()> once = beside;
     size_t i = 0;
     while (i < reqs.size()) {
         // group streams so that the chunk scratch stays within budget
@@ -397,7 +403,7 @@ int run_gauss(const std::vector<StreamReq> &reqs, hipStream_t st, size_t scratch
         int level = 0;
         for (;;) {
             int overflow = 0;
-            if (run_gauss_group(reqs.data() + i, (int)(j - i), level, st, &overflow)) return -1;
+            if (run_gauss_group(reqs.data() + i, (int)(j - i), level, st, &overflow, once)) return -1;
             if (!overflow) break;
             if (++level > 6) {
                 ipfe_set_error("Gaussian sampler: speculative window exhausted");

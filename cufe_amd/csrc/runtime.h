@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <functional>
 #include <utility>
 #include <vector>
 
@@ -42,6 +43,9 @@ void dev_free(void *p);
 // hipMemcpyAsync).  Not for a stream that is being captured.
 int copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t st);
 int copy_to_device(void *dst, const void *src, size_t bytes, hipStream_t st);
+// copy_to_device into a block no work has been given yet: a large pageable copy
+// runs beside what st holds, instead of after it.
+int copy_to_device_beside(void *dst, const void *src, size_t bytes, hipStream_t st);
 
 template <typename T>
 struct DevBuf {
@@ -96,9 +100,13 @@ struct PsetSpec;
 StreamReq make_stream_ps(const PsetSpec &ps, const uint8_t key[32], uint16_t nonce, int which, int ncalls,
                          uint32_t *out0, uint32_t *out1, long long out_stride);
 
+constexpr size_t kGaussScratch = (size_t)8 << 30;
 // Samples every request (device outputs), bit-exact with the reference
-// sequential sampler; splits into groups that fit scratch_budget bytes.
-int run_gauss(const std::vector<StreamReq> &reqs, hipStream_t st, size_t scratch_budget = (size_t)8 << 30);
+// sequential sampler; splits into groups that fit scratch_budget bytes.  beside
+// (if given) is called once, with the first group's kernels launched and their
+// outcome not yet awaited, for host work that should overlap them.
+int run_gauss(const std::vector<StreamReq> &reqs, hipStream_t st, size_t scratch_budget = kGaussScratch,
+              const std::function<int()> &beside = {});
 
 // One group of sampler streams, split into host planning, table upload, the
 // kernel launches (no host round trip, so a graph can capture them) and the

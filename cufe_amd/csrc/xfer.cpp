@@ -176,16 +176,16 @@ public:
         return it->second;
     }
 
-    // Copies; false when another copy holds the threads (nothing done).
-    bool run(uint8_t *dst, const uint8_t *src, size_t bytes, bool to_host, hipStream_t st, hipError_t *err)
+    // Copies, after what st holds already unless beside is set; false when
+    // another copy holds the threads (nothing done).
+    bool run(uint8_t *dst, const uint8_t *src, size_t bytes, bool to_host, hipStream_t st, bool beside, hipError_t *err)
     {
         std::unique_lock<std::mutex> own(busy, std::try_to_lock);
         if (!own.owns_lock()) return false;
-        // the chunks follow what st holds already
-        hipError_t e = hipEventRecord(start, st);
+        hipError_t e = beside ? hipSuccess : hipEventRecord(start, st);
         if (e == hipSuccess) {
             std::unique_lock<std::mutex> lk(mu);
-            job = Job{dst, src, bytes, to_host};
+            job = Job{dst, src, bytes, to_host, beside};
             next = 0;
             error = hipSuccess;
             left = (int)threads.size();
@@ -206,7 +206,7 @@ private:
         uint8_t *dst;
         const uint8_t *src;
         size_t bytes;
-        bool to_host;
+        bool to_host, beside;
     };
     bool ok = false;
     int device;
@@ -291,7 +291,7 @@ private:
     void work(Lane &l)
     {
         const Job j = job;
-        hipError_t e = hipStreamWaitEvent(l.st, start, 0);
+        hipError_t e = j.beside ? hipSuccess : hipStreamWaitEvent(l.st, start, 0);
         bool used[2] = {false, false};
         size_t at[2] = {0, 0}, len[2] = {0, 0};
         auto drain = [&](int s) {  // the slot's transfer is over, and for a download its bytes with the caller
@@ -337,14 +337,14 @@ bool pageable(const void *p)
     return a.type == hipMemoryTypeUnregistered;
 }
 
-int copy(void *dst, const void *src, size_t bytes, bool to_host, hipStream_t st)
+int copy(void *dst, const void *src, size_t bytes, bool to_host, hipStream_t st, bool beside)
 {
     if (bytes >= kStageMin && pageable(to_host ? dst : src)) {
         int dev = 0;
         HIP_OK(hipGetDevice(&dev));
         Copier *c = Copier::get(dev);
         hipError_t e = hipSuccess;
-        if (c && c->run((uint8_t *)dst, (const uint8_t *)src, bytes, to_host, st, &e)) {
+        if (c && c->run((uint8_t *)dst, (const uint8_t *)src, bytes, to_host, st, beside, &e)) {
             if (e == hipSuccess) return 0;
             ipfe_set_error("copy of %zu bytes failed: %s", bytes, hipGetErrorString(e));
             return -1;
@@ -356,10 +356,17 @@ int copy(void *dst, const void *src, size_t bytes, bool to_host, hipStream_t st)
 
 }  // namespace
 
-int copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t st) { return copy(dst, src, bytes, true, st); }
+int copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t st)
+{
+    return copy(dst, src, bytes, true, st, false);
+}
 int copy_to_device(void *dst, const void *src, size_t bytes, hipStream_t st)
 {
-    return copy(dst, src, bytes, false, st);
+    return copy(dst, src, bytes, false, st, false);
+}
+int copy_to_device_beside(void *dst, const void *src, size_t bytes, hipStream_t st)
+{
+    return copy(dst, src, bytes, false, st, true);
 }
 
 }  // namespace ipfe

@@ -88,3 +88,50 @@ def test_results_do_not_depend_on_earlier_calls(gpu):
     for n in (1, 7, 30):
         gpu.gauss_sample([h(b"c%d" % t) for t in range(n)], list(range(n)), 1 + n % 3, 3)
         assert np.array_equal(gpu.encrypt(x, mpk, h(b"c2"), h(b"c3")), first)
+
+
+# 84 / 85 slots: 85 and 86 polynomials of the public key, around the staged size
+@pytest.mark.parametrize("pinned", [False, True])
+@pytest.mark.parametrize("l", [84, 85, 120])
+def test_encryption_beside_the_key_upload(gpu, po, l, pinned):
+    """The public key is uploaded while the noise is sampled: calls in turn with
+    different keys, each message the oracle's."""
+    print(f"[gpu-copy] encrypt {l} slots, pinned {pinned}", flush=True)
+    rng = np.random.default_rng(l)
+    x = rng.integers(0, 5, (2, l)).astype(np.uint32)
+    ks = []
+    for k in range(2):
+        mpk = np.stack([rng.integers(0, q, (l + 1, N), dtype=np.uint32) for q in Q], axis=1)
+        if pinned:
+            p = gpu.host_empty(mpk.shape)
+            p[...] = mpk
+            mpk = p
+        ks.append(mpk)
+    for i in range(4):
+        c = gpu.encrypt(x, ks[i % 2], h(b"e2%d" % i), h(b"e3%d" % i), 7)
+        for b in range(2):
+            assert np.array_equal(c[b], po.encrypt(x[b], ks[i % 2], h(b"e2%d" % i), h(b"e3%d" % i), 7 + b)), (i, b)
+
+
+def test_threads_encrypting_at_once(gpu):
+    rng = np.random.default_rng(2)
+    ls = [90, 150, 20, 120]
+    mpks = [np.stack([rng.integers(0, q, (l + 1, N), dtype=np.uint32) for q in Q], axis=1) for l in ls]
+    xs = [rng.integers(0, 5, (1, l)).astype(np.uint32) for l in ls]
+    want = [gpu.encrypt(x, m, h(b"t2%d" % t), h(b"t3")) for t, (x, m) in enumerate(zip(xs, mpks))]
+    bad = []
+
+    def one(t):
+        try:
+            for _ in range(5):
+                if not np.array_equal(gpu.encrypt(xs[t], mpks[t], h(b"t2%d" % t), h(b"t3")), want[t]):
+                    bad.append(t)
+        except Exception as e:  # noqa: BLE001 -- reported by the test's own thread
+            bad.append((t, repr(e)))
+
+    threads = [threading.Thread(target=one, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not bad, bad
