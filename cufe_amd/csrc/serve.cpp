@@ -170,16 +170,26 @@ int launch_batch(cufe_server *s, Slot &sl)
         ipfe_set_error("server: batch layout of %d rows exceeds the slot capacity %d", row, s->cap);
         return -1;
     }
-    // upload: c_L rows to their slot rows, each request's c0 packed after
-    // them.  Buffers in pinned memory from cufe_host_alloc are copied by DMA
-    // directly; others are first copied into the slot's pinned staging.
+    // upload: c_L rows to their slot rows, the requests' c0 packed after them in
+    // the order of those rows.  Buffers in pinned memory from cufe_host_alloc are
+    // copied by DMA directly; others are first copied into the slot's pinned
+    // staging.  So is c0 of up to kStageC0 bytes, and the staged c0 goes up in one
+    // transfer a run: a transfer of a few KB is 7 us on the stream and as much to
+    // issue, the copy of 128 KiB 5.
+    constexpr size_t kStageC0 = (size_t)128 << 10;
     uint32_t *h_c0 = sl.h_stage + (size_t)s->cap * kPoly;
     uint32_t *d_c0 = sl.d_stage.get() + (size_t)s->cap * kPoly;
-    std::vector<size_t> c0_off(sl.reqs.size());
+    std::vector<size_t> order(sl.reqs.size()), c0_off(sl.reqs.size());
+    for (size_t i = 0; i < order.size(); ++i) order[i] = i;
+    std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return sl.req_row[x] < sl.req_row[y]; });
     size_t c0_words = 0;
+    for (size_t i : order) {
+        c0_off[i] = c0_words;
+        c0_words += (size_t)sl.reqs[i]->n * sl.reqs[i]->l * 3;
+    }
     for (size_t i = 0; i < sl.reqs.size(); ++i) {
         const Req &r = *sl.reqs[i];
-        const size_t cl_bytes = (size_t)r.n * kPoly * 4, c0_bytes = (size_t)r.n * r.l * 12;
+        const size_t cl_bytes = (size_t)r.n * kPoly * 4;
         const size_t cl_at = (size_t)sl.req_row[i] * kPoly;
         const uint32_t *src = r.cl;
         if (!host_pinned(r.cl, cl_bytes)) {
@@ -187,31 +197,39 @@ int launch_batch(cufe_server *s, Slot &sl)
             src = sl.h_stage + cl_at;
         }
         HIP_OK(hipMemcpyAsync(sl.d_stage.get() + cl_at, src, cl_bytes, hipMemcpyHostToDevice, sl.st));
-        c0_off[i] = c0_words;
-        src = r.c0;
-        if (!host_pinned(r.c0, c0_bytes)) {
-            memcpy(h_c0 + c0_words, r.c0, c0_bytes);
-            src = h_c0 + c0_words;
-        }
-        HIP_OK(hipMemcpyAsync(d_c0 + c0_words, src, c0_bytes, hipMemcpyHostToDevice, sl.st));
-        c0_words += (size_t)r.n * r.l * 3;
     }
-    // one conversion launch per run of requests whose rows and c0 words follow
-    // each other and whose rows have the same length (every request of a
-    // one-model batch)
-    for (size_t i = 0; i < sl.reqs.size();) {
-        const int l = sl.reqs[i]->l;
-        int n = sl.reqs[i]->n;
-        size_t j = i + 1;
-        while (j < sl.reqs.size() && sl.reqs[j]->l == l && sl.req_row[j] == sl.req_row[i] + n &&
-               c0_off[j] == c0_off[i] + (size_t)n * l * 3) {
-            n += sl.reqs[j]->n;
-            ++j;
+    size_t staged = 0, staged_to = 0;  // c0 words in the staging, not yet sent
+    auto send_staged = [&]() -> int {
+        if (staged_to > staged)
+            HIP_OK(hipMemcpyAsync(d_c0 + staged, h_c0 + staged, (staged_to - staged) * 4, hipMemcpyHostToDevice, sl.st));
+        return 0;
+    };
+    for (size_t i : order) {
+        const Req &r = *sl.reqs[i];
+        const size_t words = (size_t)r.n * r.l * 3;
+        if (words * 4 > kStageC0 && host_pinned(r.c0, words * 4)) {
+            HIP_OK(hipMemcpyAsync(d_c0 + c0_off[i], r.c0, words * 4, hipMemcpyHostToDevice, sl.st));
+            continue;
         }
+        if (staged_to != c0_off[i]) {
+            if (send_staged()) return -1;
+            staged = c0_off[i];
+        }
+        memcpy(h_c0 + c0_off[i], r.c0, words * 4);
+        staged_to = c0_off[i] + words;
+    }
+    if (send_staged()) return -1;
+    // one conversion launch per run of requests whose rows follow each other and
+    // have the same length (every request of one model)
+    for (size_t k = 0; k < order.size();) {
+        const size_t i = order[k];
+        const int l = sl.reqs[i]->l;
+        int n = 0;
+        for (; k < order.size() && sl.reqs[order[k]]->l == l && sl.req_row[order[k]] == sl.req_row[i] + n; ++k)
+            n += sl.reqs[order[k]]->n;
         if (sl.rows.put(sl.req_row[i], n, sl.d_stage.get() + (size_t)sl.req_row[i] * kPoly, d_c0 + c0_off[i], sl.st,
                         l))
             return -1;
-        i = j;
     }
     // small groups take the low-latency split-K launch unless another slot
     // runs a large range (full-GPU launches, which under load the split launch
