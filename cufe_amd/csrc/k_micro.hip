@@ -93,8 +93,7 @@ __global__ __launch_bounds__(256) void k_mb_aes_rep(const uint32_t *__restrict__
     out[blockIdx.x * blockDim.x + threadIdx.x] = x;
 }
 
-// T0 and T2 bank-replicated (64 KiB): the sampler's default AES, in
-// 512-thread workgroups as the sampler runs it (two per CU).
+// T0 and T2 bank-replicated (64 KiB), in 512-thread workgroups (two per CU).
 __global__ __launch_bounds__(512) void k_mb_aes_rep2(const uint32_t *__restrict__ rk,
                                                      const uint32_t *__restrict__ te_global,
                                                      uint32_t nblocks_per_thread, uint32_t *__restrict__ out)

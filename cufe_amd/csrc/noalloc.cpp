@@ -11,8 +11,8 @@
 // device with that device current, and only that address is used.
 //
 // Every call on one GPU shares that GPU's array and leaves its contents
-// behind; nothing it reads is assumed to start at zero (the status words and
-// labels are cleared by fill kernels in each launch, counts are written for
+// behind; nothing it reads is assumed to start at zero (the status words are
+// cleared by a fill kernel in each launch, counts and labels are written for
 // every chunk before they are read, values only where they are read).  Calls
 // from several threads of one process are serialised by a mutex; calls that
 // overlap on one GPU from other code paths sharing the array would race.
