@@ -278,7 +278,7 @@ struct AesLayout<3> {
 };
 
 constexpr int CAND_NT = 1024, CAND_WAVES = CAND_NT / 64;
-constexpr int SUB_CHUNKS = 16, SUB_WORDS = 28;
+constexpr int SUB_CHUNKS = 16, SUB_WORDS = 28, TILE_CHUNKS = 64;
 constexpr int CAND_WINDOWS = 8;  // of 256 counters: a 64-chunk tile's 1,536 touch at most seven
 static_assert(SUB_CHUNKS * SUB_WORDS + 8 * CAND_WINDOWS == 512, "the wave's buffer");
 
@@ -380,8 +380,8 @@ __device__ Cand cand_whole(const Tab &tb, const GaussStream *S, long long chunk,
 
 template <int TM>
 __global__ __launch_bounds__(CAND_NT) void k_gauss_candidates(const GaussStream *__restrict__ streams, int nstreams,
-                                                               const long long *__restrict__ tile_prefix,
-                                                               long long ntiles, int tile_chunks,
+                                                               const long long *__restrict__ chunk_prefix,
+                                                               long long nchunks_total,
                                                                const uint32_t *__restrict__ te_global,
                                                                uint8_t *__restrict__ cnt, uint64_t *__restrict__ vals,
                                                                int *__restrict__ status, int full, int ulim, int whole)
@@ -393,23 +393,33 @@ __global__ __launch_bounds__(CAND_NT) void k_gauss_candidates(const GaussStream 
     __syncthreads();
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // this wave's run of consecutive tiles; the first waves of all workgroups
-    // come first, so that a short plan spreads over the CUs
-    const long long waves = (long long)gridDim.x * CAND_WAVES, me = (long long)wv * gridDim.x + blockIdx.x;
-    const long long t0 = me * ntiles / waves, t1 = (me + 1) * ntiles / waves;
-    if (t0 >= t1) return;
+    // This wave's run of groups of 16 chunks, taken in tiles of up to four groups
+    // within a stream (one window pass and, for stored values, one round of sign
+    // blocks a tile: 64 chunks fill its lanes).  Runs end on any group: dealt in
+    // whole tiles of one size, a plan of a few tiles a wave left most waves
+    // idle in its last round (full streams of S3, 800 calls: 305 -> 280 us, 126: 93
+    // -> 85).  The first waves of all workgroups come first: fewer groups than waves
+    // spread over all CUs (4 calls: 22 -> 14 us), and a plan's full streams, whose
+    // chunks cost more, over many (all in a few workgroups they made 2,048 rows 7%
+    // slower).
+    const long long groups = nchunks_total / SUB_CHUNKS;
+    const long long waves = min((long long)gridDim.x * CAND_WAVES, groups), me = (long long)wv * gridDim.x + blockIdx.x;
+    if (me >= waves) return;
+    const long long t0 = me * groups / waves * SUB_CHUNKS, t1 = (me + 1) * groups / waves * SUB_CHUNKS;
     const Tab tb(te);
     uint32_t *buf = bufs[wv], *win = buf + SUB_CHUNKS * SUB_WORDS;
-    int si = __builtin_amdgcn_readfirstlane(find_stream(tile_prefix, nstreams, t0));
+    int si = __builtin_amdgcn_readfirstlane(find_stream(chunk_prefix, nstreams, t0));
     auto wave_sync = [] {  // the wave's LDS accesses stay in order across this point
         asm volatile("" ::: "memory");
         __builtin_amdgcn_wave_barrier();
     };
-    for (long long tile = t0; tile < t1; ++tile) {
-        while (si + 1 < nstreams && tile_prefix[si + 1] <= tile) ++si;
+    for (long long t = t0; t < t1;) {  // the run's part of each stream it meets
+        while (si + 1 < nstreams && chunk_prefix[si + 1] <= t) ++si;
         const GaussStream *S = streams + si;
-        const long long chunk0 = (tile - tile_prefix[si]) * tile_chunks;
-        const int nch = (int)min((long long)tile_chunks, (long long)S->nchunks - chunk0);
+        const long long stream0 = chunk_prefix[si];
+        const long long t_next = si + 1 < nstreams ? min(t1, chunk_prefix[si + 1]) : t1;
+        const int chunk_first = (int)(t - stream0), chunk_end = min((int)(t_next - stream0), S->nchunks);
+        t = t_next;
         const WidthConsts wc(S->which);
         const bool store_vals = !S->coef0_only;
         const uint32_t nonce = S->nonce;
@@ -422,101 +432,104 @@ __global__ __launch_bounds__(CAND_NT) void k_gauss_candidates(const GaussStream 
             asm volatile("" : "+s"(a));
             return (RoundKeys)a;
         };
-        // windows of 256 counters the tile touches (counters wrap at 2^32)
-        const uint32_t c_lo = (uint32_t)(chunk0 * 24), w0 = c_lo >> 8;
-        const int nw = (int)(((c_lo & 255u) + (uint32_t)(nch * 24 - 1)) >> 8) + 1;
-        wave_sync();
-        if (lane < nw) aes256_ctr_window(tb, keys(), nonce, (w0 + lane) & 0xffffffu, win + 8 * lane);
-        wave_sync();
-        auto window = [&](uint32_t ctr) { return win + 8 * (((ctr >> 8) - w0) & (CAND_WINDOWS - 1)); };
-        uint32_t sign = 0;  // lane l: the sign word of the tile's chunk l
-        if (store_vals) {
-            const uint32_t ctr = (uint32_t)((chunk0 + min(lane, nch - 1)) * 24 + 17);
-            uint32_t o[4];
-            const RoundKeys rk = keys();
-            aes256_ctr_block_win<4>(tb, rk, rk + 60, window(ctr), ctr, o);
-            sign = o[2];
-        }
-        for (int s = 0; s < nch; s += SUB_CHUNKS) {
-            const int nsub = min(SUB_CHUNKS, nch - s);
-            {
-                const int k = lane >> 2, j = lane & 3;
-                const uint32_t base = (uint32_t)((chunk0 + s + min(k, nsub - 1)) * 24);
-                uint32_t *d = buf + SUB_WORDS * k;
+        for (int chunk0 = chunk_first; chunk0 < chunk_end; chunk0 += TILE_CHUNKS) {
+            const int nch = min(TILE_CHUNKS, chunk_end - chunk0);
+            // windows of 256 counters the tile touches (counters wrap at 2^32)
+            const uint32_t c_lo = (uint32_t)chunk0 * 24u, w0 = c_lo >> 8;
+            const int nw = (int)(((c_lo & 255u) + (uint32_t)(nch * 24 - 1)) >> 8) + 1;
+            wave_sync();
+            if (lane < nw) aes256_ctr_window(tb, keys(), nonce, (w0 + lane) & 0xffffffu, win + 8 * lane);
+            wave_sync();
+            auto window = [&](uint32_t ctr) { return win + 8 * (((ctr >> 8) - w0) & (CAND_WINDOWS - 1)); };
+            uint32_t sign = 0;  // lane l: the sign word of the tile's chunk l
+            if (store_vals) {
+                const uint32_t ctr = (uint32_t)(chunk0 + min(lane, nch - 1)) * 24u + 17u;
                 uint32_t o[4];
-                {
-                    const uint32_t ctr = base + 2 + j;
-                    const RoundKeys rk = keys();
-                    aes256_ctr_block_win<2 | 8>(tb, rk, rk + 60, window(ctr), ctr, o);
-                    *reinterpret_cast<uint2 *>(d + 2 * j) = make_uint2(o[1], o[3]);
-                }
-                {
-                    const uint32_t ctr = base + 8 + j;
-                    const RoundKeys rk = keys();
-                    aes256_ctr_block_win<1 | 4>(tb, rk, rk + 60, window(ctr), ctr, o);
-                    *reinterpret_cast<uint2 *>(d + 8 + 2 * j) = make_uint2(o[0], o[2]);
-                }
-                {
-                    const uint32_t ctr = base + (j == 0 ? 6 : 11 + j);
-                    const RoundKeys rk = keys();
-                    aes256_ctr_block_win(tb, rk, rk + 60, window(ctr), ctr, o);
-                    if (j == 0)
-                        d[8] = o[0];  // over block 8's first word, which no candidate reads
-                    else
-                        *reinterpret_cast<uint4 *>(d + 12 + 4 * j) = make_uint4(o[0], o[1], o[2], o[3]);
-                }
+                const RoundKeys rk = keys();
+                aes256_ctr_block_win<4>(tb, rk, rk + 60, window(ctr), ctr, o);
+                sign = o[2];
             }
-            wave_sync();
-#pragma unroll 1
-            for (int e = 0; e < 2; ++e) {
-                const int k = 8 * e + (lane >> 3), c = lane & 7, sh = lane & 56;
-                const bool valid = k < nsub;
-                const uint32_t *q = buf + SUB_WORDS * k;
-                // the c-th uniform word below UQ
-                uint32_t w = q[18 + c];
-                bool open = false;
-                const uint64_t kept = __ballot(w < wc.UQ);
-                if (kept != ~0ull) {
-                    const uint32_t bad = ~((uint32_t)((kept >> sh) & 0xffu) | (q[26] < wc.UQ ? 256u : 0u) |
-                                           (q[27] < wc.UQ ? 512u : 0u));
-                    // its position: c plus the rejected words up to it
-                    int pos = c;
-#pragma unroll
-                    for (int it = 0; it < 3; ++it) pos = c + __popc(bad & ((2u << min(pos, 15)) - 1u));
-                    open = pos >= min(ulim, 10) || pos != c + __popc(bad & ((2u << min(pos, 15)) - 1u));
-                    w = q[18 + min(pos, 9)];
+            for (int s = 0; s < nch; s += SUB_CHUNKS) {
+                const int nsub = min(SUB_CHUNKS, nch - s);
+                {
+                    const int k = lane >> 2, j = lane & 3;
+                    const uint32_t base = (uint32_t)(chunk0 + s + min(k, nsub - 1)) * 24u;
+                    uint32_t *d = buf + SUB_WORDS * k;
+                    uint32_t o[4];
+                    {
+                        const uint32_t ctr = base + 2 + j;
+                        const RoundKeys rk = keys();
+                        aes256_ctr_block_win<2 | 8>(tb, rk, rk + 60, window(ctr), ctr, o);
+                        *reinterpret_cast<uint2 *>(d + 2 * j) = make_uint2(o[1], o[3]);
+                    }
+                    {
+                        const uint32_t ctr = base + 8 + j;
+                        const RoundKeys rk = keys();
+                        aes256_ctr_block_win<1 | 4>(tb, rk, rk + 60, window(ctr), ctr, o);
+                        *reinterpret_cast<uint2 *>(d + 8 + 2 * j) = make_uint2(o[0], o[2]);
+                    }
+                    {
+                        const uint32_t ctr = base + (j == 0 ? 6 : 11 + j);
+                        const RoundKeys rk = keys();
+                        aes256_ctr_block_win(tb, rk, rk + 60, window(ctr), ctr, o);
+                        if (j == 0)
+                            d[8] = o[0];  // over block 8's first word, which no candidate reads
+                        else
+                            *reinterpret_cast<uint4 *>(d + 12 + 4 * j) = make_uint4(o[0], o[1], o[2], o[3]);
+                    }
                 }
-                const uint32_t y = uniform_y(w, wc);
-                // CDT rank by the high word
-                const uint32_t r2h = q[c < 4 ? c : c + 5] & 0x7fffffffu;
-                uint32_t xs = 0;
-                bool tie = r2h == 0;  // the entries from the sixth on have a zero high word
-#pragma unroll
-                for (int i = 0; i < 5; ++i) {
-                    xs += r2h < kCdtHigh[i];
-                    tie = tie || r2h == kCdtHigh[i];
+                wave_sync();
+    #pragma unroll 1
+                for (int e = 0; e < 2; ++e) {
+                    const int k = 8 * e + (lane >> 3), c = lane & 7, sh = lane & 56;
+                    const bool valid = k < nsub;
+                    const uint32_t *q = buf + SUB_WORDS * k;
+                    // the c-th uniform word below UQ
+                    uint32_t w = q[18 + c];
+                    bool open = false;
+                    const uint64_t kept = __ballot(w < wc.UQ);
+                    if (kept != ~0ull) {
+                        const uint32_t bad = ~((uint32_t)((kept >> sh) & 0xffu) | (q[26] < wc.UQ ? 256u : 0u) |
+                                               (q[27] < wc.UQ ? 512u : 0u));
+                        // its position: c plus the rejected words up to it
+                        int pos = c;
+    #pragma unroll
+                        for (int it = 0; it < 3; ++it) pos = c + __popc(bad & ((2u << min(pos, 15)) - 1u));
+                        open = pos >= min(ulim, 10) || pos != c + __popc(bad & ((2u << min(pos, 15)) - 1u));
+                        w = q[18 + min(pos, 9)];
+                    }
+                    const uint32_t y = uniform_y(w, wc);
+                    // CDT rank by the high word
+                    const uint32_t r2h = q[c < 4 ? c : c + 5] & 0x7fffffffu;
+                    uint32_t xs = 0;
+                    bool tie = r2h == 0;  // the entries from the sixth on have a zero high word
+    #pragma unroll
+                    for (int i = 0; i < 5; ++i) {
+                        xs += r2h < kCdtHigh[i];
+                        tie = tie || r2h == kCdtHigh[i];
+                    }
+                    Cand cd;
+                    const uint64_t res = cand_exp(xs, y, wc, cd.z);
+                    const uint32_t rm_hi = q[c < 4 ? 4 + c : 9 + c], bytes = q[c < 4 ? 8 : 17];
+                    const uint32_t res_hi = (uint32_t)(res >> 32);
+                    const uint32_t mant = (res_hi & 0xfffffu) | 0x100000u, rmant = rm_hi & 0x1fffffu;
+                    const bool bit = (rmant < mant && bernoulli_exp_less(res_hi, rm_hi, (bytes >> (8 * (c & 3))) & 255u)) ||
+                                     res == 0x3FF0000000000000ull;
+                    open = valid && (whole || open || tie || rmant == mant || (!store_vals && cd.z == 0));
+                    cd.sgn = store_vals ? (__shfl(sign, s + k, 64) >> c) & 1u : 0u;
+                    cd.acc = valid && bit && (store_vals ? (cd.z != 0 || cd.sgn != 0) : true);
+                    if (open) cd = cand_whole(tb, S, chunk0 + s + k, c, wc, status, full, ulim, !store_vals);
+                    const uint64_t am = __ballot(cd.acc);
+                    const uint32_t gm = (uint32_t)((am >> sh) & 0xffu);
+                    if (valid) {
+                        const long long gc = S->chunk_base + chunk0 + s + k;
+                        if (c == 0) cnt[gc] = (uint8_t)__popc(gm);
+                        if (store_vals && cd.acc)
+                            vals[gc * 8 + __popc(gm & ((1u << c) - 1u))] = cd.z | ((uint64_t)cd.sgn << 63);
+                    }
                 }
-                Cand cd;
-                const uint64_t res = cand_exp(xs, y, wc, cd.z);
-                const uint32_t rm_hi = q[c < 4 ? 4 + c : 9 + c], bytes = q[c < 4 ? 8 : 17];
-                const uint32_t res_hi = (uint32_t)(res >> 32);
-                const uint32_t mant = (res_hi & 0xfffffu) | 0x100000u, rmant = rm_hi & 0x1fffffu;
-                const bool bit = (rmant < mant && bernoulli_exp_less(res_hi, rm_hi, (bytes >> (8 * (c & 3))) & 255u)) ||
-                                 res == 0x3FF0000000000000ull;
-                open = valid && (whole || open || tie || rmant == mant || (!store_vals && cd.z == 0));
-                cd.sgn = store_vals ? (__shfl(sign, s + k, 64) >> c) & 1u : 0u;
-                cd.acc = valid && bit && (store_vals ? (cd.z != 0 || cd.sgn != 0) : true);
-                if (open) cd = cand_whole(tb, S, chunk0 + s + k, c, wc, status, full, ulim, !store_vals);
-                const uint64_t am = __ballot(cd.acc);
-                const uint32_t gm = (uint32_t)((am >> sh) & 0xffu);
-                if (valid) {
-                    const long long gc = S->chunk_base + chunk0 + s + k;
-                    if (c == 0) cnt[gc] = (uint8_t)__popc(gm);
-                    if (store_vals && cd.acc)
-                        vals[gc * 8 + __popc(gm & ((1u << c) - 1u))] = cd.z | ((uint64_t)cd.sgn << 63);
-                }
+                wave_sync();
             }
-            wave_sync();
         }
     }
 }
@@ -705,25 +718,23 @@ static int candidate_blocks()
     return cus;
 }
 
-int gauss_candidate_waves() { return candidate_blocks() * CAND_WAVES; }
-
-int launch_gauss_candidates(const GaussStream *d_streams, int nstreams, const long long *d_tile_prefix,
-                            long long ntiles, int tile, uint8_t *cnt, uint64_t *vals, int *status, int full,
+int launch_gauss_candidates(const GaussStream *d_streams, int nstreams, const long long *d_chunk_prefix,
+                            long long nchunks_total, uint8_t *cnt, uint64_t *vals, int *status, int full,
                             hipStream_t st)
 {
-    if (ntiles <= 0) return 0;
-    if (tile != 16 && tile != 32 && tile != 64) {
-        ipfe_set_error("Gaussian candidates: tiles of %d chunks", tile);
+    if (nchunks_total <= 0) return 0;
+    if (nchunks_total % SUB_CHUNKS) {
+        ipfe_set_error("Gaussian candidates: %lld chunks, not a multiple of 16", nchunks_total);
         return -1;
     }
-    const unsigned grid = (unsigned)std::min<long long>(ntiles, candidate_blocks());
+    const unsigned grid = (unsigned)std::min<long long>(nchunks_total / SUB_CHUNKS, candidate_blocks());
     const int rep = aes_rep_mode();
     // CUFE_GAUSS_WHOLE=1 (tests): every candidate from whole words
     const char *w = getenv("CUFE_GAUSS_WHOLE");
     const int whole = w && atoi(w) != 0;
 #define CAND(TM)                                                                                                   \
-    hipLaunchKernelGGL(k_gauss_candidates<TM>, dim3(grid), dim3(CAND_NT), 0, st, d_streams, nstreams, d_tile_prefix, \
-                       ntiles, tile, g_aes_te, cnt, vals, status, full, scan_limit(), whole)
+    hipLaunchKernelGGL(k_gauss_candidates<TM>, dim3(grid), dim3(CAND_NT), 0, st, d_streams, nstreams, d_chunk_prefix, \
+                       nchunks_total, g_aes_te, cnt, vals, status, full, scan_limit(), whole)
     if (rep >= 4)
         CAND(3);
     else if (rep == 3)

@@ -74,14 +74,12 @@ struct GaussStream {
 
 // Candidate pass: for every chunk of every stream, AES + CDT + Bernoulli;
 // writes the accepted count and the accepted (z | sign << 63) values in order.
-// tile_prefix counts tiles of `tile` chunks per stream (16, 32 or 64).
+// chunk_prefix: each stream's first chunk, multiples of 16, as is nchunks_total.
 // full: a chunk whose uniform scan runs past the words the default AES blocks
 // hold is scanned on (else it sets status bit 4)
-int launch_gauss_candidates(const GaussStream *d_streams, int nstreams, const long long *d_tile_prefix,
-                            long long ntiles, int tile, uint8_t *cnt, uint64_t *vals, int *status, int full,
+int launch_gauss_candidates(const GaussStream *d_streams, int nstreams, const long long *d_chunk_prefix,
+                            long long nchunks_total, uint8_t *cnt, uint64_t *vals, int *status, int full,
                             hipStream_t st);
-// Waves the candidate pass runs at once (tiles are dealt to them).
-int gauss_candidate_waves();
 // Walk (k_gauss_walk.hip): per stream, the call boundaries from the counts;
 // writes per chunk of the full streams (call << 13 | offset) or -1, padding
 // included.  status[stream] = 1 when the window was short (else it stays).

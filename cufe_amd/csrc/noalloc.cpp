@@ -4,7 +4,7 @@
 //
 // The caller passes the keys, nonces and a device output buffer it owns.
 // Every other device buffer the sampler's kernels use -- stream descriptors,
-// tile / chunk prefixes, status words and the per-chunk counts, accepted
+// chunk prefixes, status words and the per-chunk counts, accepted
 // values and call labels -- is carved out of `scratch`, a static device array
 // of kScratchBytes.  Host code never passes the array's name to a kernel: the
 // array's device address comes from hipGetSymbolAddress, resolved once per

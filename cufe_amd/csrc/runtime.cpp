@@ -179,10 +179,9 @@ int GaussPlan::build(const StreamReq *reqs, int count, int lvl, bool alloc_meta)
     n = count;
     level = lvl;
     hs.assign(n, GaussStream{});
-    tile_prefix.assign(n, 0);
     chunk_prefix.assign(n, 0);
     first_prefix.assign(n, 0);
-    tiles = chunks = full_chunks = nfirst = map_words = 0;
+    chunks = full_chunks = nfirst = map_words = 0;
     max_chunks = 0;
     // full streams first, so per-chunk values and labels cover only their chunks
     std::vector<int> order;
@@ -225,32 +224,11 @@ int GaussPlan::build(const StreamReq *reqs, int count, int lvl, bool alloc_meta)
             full_chunks = chunks;
         }
     }
-    // Chunks per tile of the candidate pass.  A wave's tile takes three rounds
-    // of AES per 16 chunks, and for full streams one more for the tile's sign
-    // blocks, of which a 64-chunk tile fills every lane; smaller tiles spread a
-    // short plan over more waves.  The size whose busiest wave has the fewest
-    // rounds, larger on a tie.
-    const long long waves = gauss_candidate_waves();
-    long long best = 0;
-    for (int t : {64, 32, 16}) {
-        long long nt = 0;
-        for (const GaussStream &g : hs) nt += (g.nchunks + t - 1) / t;
-        const long long rounds = (nt + waves - 1) / waves * (3 * t / 16 + (full_chunks > 0));
-        if (best == 0 || rounds < best) {
-            best = rounds;
-            tile = t;
-        }
-    }
-    for (int i = 0; i < n; ++i) {
-        tile_prefix[i] = tiles;
-        tiles += (hs[i].nchunks + tile - 1) / tile;
-    }
     if (!alloc_meta) return 0;
-    if (d_streams.alloc(n) || d_tp.alloc(n) || d_cp.alloc(n) || d_fp.alloc(n) || d_status.alloc(n + 1) ||
+    if (d_streams.alloc(n) || d_cp.alloc(n) || d_fp.alloc(n) || d_status.alloc(n + 1) ||
         d_first.alloc((size_t)nfirst + 1))
         return -1;
     m_streams = d_streams.get();
-    m_tp = d_tp.get();
     m_cp = d_cp.get();
     m_fp = d_fp.get();
     m_first = d_first.get();
@@ -262,6 +240,8 @@ static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 size_t GaussPlan::meta_bytes() const
 {
+    // three arrays of n: one more than bound, so that the largest plan a given
+    // region takes stays what it was
     return align256(sizeof(GaussStream) * n) + 3 * align256(sizeof(long long) * n) +
            align256(sizeof(long long) * ((size_t)nfirst + 1)) + align256(sizeof(int) * ((size_t)n + 1));
 }
@@ -270,8 +250,6 @@ int GaussPlan::bind_meta(uint8_t *base)
 {
     m_streams = (GaussStream *)base;
     base += align256(sizeof(GaussStream) * n);
-    m_tp = (long long *)base;
-    base += align256(sizeof(long long) * n);
     m_cp = (long long *)base;
     base += align256(sizeof(long long) * n);
     m_fp = (long long *)base;
@@ -334,7 +312,6 @@ void GaussPlan::rekey(const StreamReq *reqs)
 int GaussPlan::upload(hipStream_t st)
 {
     HIP_OK(hipMemcpyAsync(m_streams, hs.data(), sizeof(GaussStream) * n, hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(m_tp, tile_prefix.data(), sizeof(long long) * n, hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(m_cp, chunk_prefix.data(), sizeof(long long) * n, hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(m_fp, first_prefix.data(), sizeof(long long) * n, hipMemcpyHostToDevice, st));
     return 0;
@@ -344,7 +321,7 @@ int GaussPlan::upload(hipStream_t st)
 int GaussPlan::launch(hipStream_t st)
 {
     if (launch_fill_i32(m_status, 0, n + 1, st)) return -1;
-    if (launch_gauss_candidates(m_streams, n, m_tp, tiles, tile, s_cnt, s_vals, m_status + n, full, st)) return -1;
+    if (launch_gauss_candidates(m_streams, n, m_cp, chunks, s_cnt, s_vals, m_status + n, full, st)) return -1;
     if (launch_gauss_walk(m_streams, n, max_chunks, s_cnt, s_pos, s_map, m_first, m_status, st)) return -1;
     if (launch_gauss_scatter(m_streams, n, m_cp, full_chunks, s_cnt, s_vals, s_pos, st)) return -1;
     if (launch_gauss_firsts(m_streams, n, m_fp, m_first, nfirst, m_status + n, full, st)) return -1;

@@ -114,19 +114,18 @@ int run_gauss(const std::vector<StreamReq> &reqs, hipStream_t st, size_t scratch
 struct GaussPlan {
     int n = 0, level = 0;
     int full = 0;  // scan a chunk past its default AES blocks (set after one needed it)
-    long long tiles = 0, chunks = 0, full_chunks = 0, nfirst = 0;
+    long long chunks = 0, full_chunks = 0, nfirst = 0;
     long long map_words = 0;  // of the walk's maps of the compact streams
     int max_chunks = 0;
-    int tile = 16;  // chunks per tile of the candidate pass
     std::vector<GaussStream> hs;
-    std::vector<long long> tile_prefix, chunk_prefix, first_prefix;
+    std::vector<long long> chunk_prefix, first_prefix;
     DevBuf<GaussStream> d_streams;
-    DevBuf<long long> d_tp, d_cp, d_fp, d_first;
+    DevBuf<long long> d_cp, d_fp, d_first;
     DevBuf<int> d_status;
     // device metadata the kernels read: the buffers above, or a region bound
     // with bind_meta
     GaussStream *m_streams = nullptr;
-    long long *m_tp = nullptr, *m_cp = nullptr, *m_fp = nullptr, *m_first = nullptr;
+    long long *m_cp = nullptr, *m_fp = nullptr, *m_first = nullptr;
     int *m_status = nullptr;
     DevBuf<uint8_t> own_cnt;
     DevBuf<uint64_t> own_vals;
