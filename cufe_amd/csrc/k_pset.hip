@@ -19,7 +19,10 @@ constexpr int FOLD_CHUNK = 16384;  // k_ps_fold: slots of a wave's 64-bit sums
 // Shape of the transforms inside the fused kernels, per log2 N: 16 coefficients a
 // thread, what setup's two transforms and their factors leave registers for.  At
 // N = 8192, 512 threads for 256 of 32: setup of 785 slots 341 -> 258 us, of 63
-// 31.4 -> 23.2; encryption 214 -> 167 and 25.7 -> 15.5 (with the noise loaded first).
+// 31.4 -> 23.2; encryption 214 -> 165 and 25.7 -> 15.5, with the noise loaded first
+// (loaded at its use 147 and 18.5: two workgroups a CU instead of one, where
+// there are that many; at N = 2048 and 4096 first is better at both, 8 and 20.5
+// against 12.5 and 23.3).
 template <int LOGN>
 struct FusedShape;
 template <>
