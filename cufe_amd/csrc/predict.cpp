@@ -213,6 +213,9 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
         ipfe_set_error("model: sum of nSV (%d) != l (%d)", nsv_sum, nS);
         return -1;
     }
+    // accepted: the model before is let go of, and S, which every reader asks
+    // for first, is set when all the rest is
+    *this = Model();
     // With a zero slot after the last feature the reference's fold ends
     // canonical, so the sum part joins the contraction (key = [-s', y]).
     const bool fz = mx < L - 1;
@@ -226,12 +229,6 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
     y.val = y_val.get();
     y.len = L;
     if (launch_fold(y, nS, msk_dev, sk.get(), device()->barrett, st)) return -1;
-    kdig.reset();
-    margin.reset();
-    margin88.reset();
-    k16.reset();
-    kd.reset();
-    S = nS;
     kkey = kk;
     fused = fz;
     if (launch_fill_i32((int *)info.get() + 2, 0, 4, st)) return -1;
@@ -279,7 +276,6 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
         md.exact_int = integral && abs_sum * 50241.0 < 9007199254740992.0;
         // the two-class vote then reads 4-byte coefficients (half the bytes of
         // the doubles) and sums in 64-bit integers: the same exact sum
-        icoef.reset();
         bool fits = md.exact_int != 0;
         for (int k = 0; fits && k < (m->nr_class - 1) * nS; ++k) fits = fabs(m->sv_coef[k]) < 2147483648.0;
         if (fits) {
@@ -312,7 +308,7 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
         margin.reset();
         margin88.reset();
         k16.reset();
-        if (ensure_kd(st)) return -1;
+        if (!kd.get() && make_kd(nS, st)) return -1;
     }
     if (i8) {
         spad = (nS + 127) / 128 * 128;
@@ -326,16 +322,17 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
     nr_class = m->nr_class;
     maxidx = mx;
     l_key = L;
+    S = nS;
     return 0;
 }
 
-// The fp64 operand, complete when this returns (whichever stream reads it).
-int Model::ensure_kd(hipStream_t st) const
+// The fp64 operand of nS keys, complete when this returns (whichever stream
+// reads it).
+int Model::make_kd(int nS, hipStream_t st) const
 {
-    if (kd.get()) return 0;
     DevBuf<unsigned int> mx;
-    if (mx.alloc(3) || launch_fill_i32((int *)mx.get(), 0, 3, st) || kd.alloc((size_t)3 * S * kkey)) return -1;
-    if (launch_contract_keys(sk.get(), S, kkey, fused ? -1 : 1, y, kd.get(), mx.get(), st) || sync_stream(st)) {
+    if (mx.alloc(3) || launch_fill_i32((int *)mx.get(), 0, 3, st) || kd.alloc((size_t)3 * nS * kkey)) return -1;
+    if (launch_contract_keys(sk.get(), nS, kkey, fused ? -1 : 1, y, kd.get(), mx.get(), st) || sync_stream(st)) {
         kd.reset();
         return -1;
     }

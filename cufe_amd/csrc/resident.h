@@ -44,8 +44,12 @@ struct Model {
     DevBuf<uint64_t> margin, margin88;  // the same bound at 88 bits (units of 2^-88) for the refinement
     DevBuf<int16_t> k16;  // [S][kkey] key values for the fraction form's exact kernel
 
+    // A model that is refused (its vectors or class sizes do not fit) leaves the
+    // one before it in place; a failure after that (an allocation, a launch)
+    // leaves none, S = 0.
     int build(const uint32_t *msk_dev, int l_key, const cufe_svm_model *m, hipStream_t st);
-    int ensure_kd(hipStream_t st) const;
+    int ensure_kd(hipStream_t st) const { return kd.get() ? 0 : make_kd(S, st); }
+    int make_kd(int nS, hipStream_t st) const;
     size_t bytes() const;  // kd included
 };
 

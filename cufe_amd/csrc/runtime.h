@@ -54,6 +54,12 @@ struct DevBuf {
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
+    DevBuf &operator=(DevBuf &&o)
+    {
+        reset();
+        swap(o);
+        return *this;
+    }
     ~DevBuf() { reset(); }
     void reset()
     {
