@@ -333,13 +333,15 @@ int ps_launch_enc_poly(const PsetState &st, const uint32_t *mpk, const uint32_t 
 int ps_launch_fold(const PsetState &st, const uint32_t *y, int nvec, int l, const uint32_t *P, uint32_t *out,
                    hipStream_t s)
 {
-    const size_t wgs = (size_t)nvec * st.dev.nmod * (st.dev.N / 64);
-    if (wgs == 0) return 0;
-    if (wgs >> 31) {
-        ipfe_set_error("fold: %d vectors are too many", nvec);
-        return -1;
+    // a launch takes fewer than 2^32 threads (2^24 of these workgroups): whole
+    // vectors, 2^23 workgroups at most
+    const int wgs = st.dev.nmod * (st.dev.N / 64), step = (1 << 23) / wgs;
+    const size_t words = (size_t)st.dev.nmod * st.dev.N;
+    for (long long v0 = 0; v0 < nvec; v0 += step) {
+        const int n = (int)(nvec - v0 < step ? nvec - v0 : step);
+        hipLaunchKernelGGL(k_ps_fold, dim3((unsigned)(n * wgs)), dim3(64 * FOLD_WAVES), 0, s, y + (size_t)v0 * l, l, P,
+                           out + v0 * words, st.dev);
     }
-    hipLaunchKernelGGL(k_ps_fold, dim3((unsigned)wgs), dim3(64 * FOLD_WAVES), 0, s, y, l, P, out, st.dev);
     HIP_OK(hipGetLastError());
     return 0;
 }
