@@ -191,8 +191,8 @@ int launch_crt_round(const uint32_t *d, int nvec, int coef, uint32_t *r, hipStre
 
 // Sparse lists of dense vectors y [n][stride], one wave per vector: counts (into
 // off[v + 1]) with info[0] = the largest slot in use plus one and info[1] =
-// v stride + i of the first entry at a slot i >= limit, then, after the prefix
-// sums, the entries.
+// v stride + i of the first entry at a slot i >= limit, then their prefix sums, then
+// the entries.
 __global__ __launch_bounds__(256) void k_sparse_count(const uint32_t *__restrict__ y, int n, int stride, int limit,
                                                       int *__restrict__ off, unsigned int *__restrict__ info)
 {
@@ -214,8 +214,9 @@ __global__ __launch_bounds__(256) void k_sparse_count(const uint32_t *__restrict
         atomicMax(info, (unsigned int)(last + 1));
 }
 
-// off[1 .. n] from counts to their running sum, off[0] = 0; one workgroup.
-__global__ __launch_bounds__(1024) void k_sparse_prefix(int *__restrict__ off, int n)
+// off[1 .. n] from counts to their running sum, off[0] = 0, info[2] = their sum;
+// one workgroup.
+__global__ __launch_bounds__(1024) void k_sparse_prefix(int *__restrict__ off, int n, unsigned int *__restrict__ info)
 {
     __shared__ int wsum[16];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -238,6 +239,7 @@ __global__ __launch_bounds__(1024) void k_sparse_prefix(int *__restrict__ off, i
         if (i < n) off[i + 1] = before + x;
         __syncthreads();
     }
+    if (tid == 0) info[2] = (unsigned int)carry;
 }
 
 __global__ __launch_bounds__(256) void k_sparse_fill(const uint32_t *__restrict__ y, int n, int stride,
@@ -265,14 +267,14 @@ int launch_sparse_count(const uint32_t *y, int n, int stride, int limit, int *of
     if (n <= 0) return 0;
     if (launch_fill_i32((int *)info, 0, 1, st) || launch_fill_i32((int *)info + 1, -1, 1, st)) return -1;
     hipLaunchKernelGGL(k_sparse_count, dim3((unsigned)(n + 3) / 4), dim3(256), 0, st, y, n, stride, limit, off, info);
+    hipLaunchKernelGGL(k_sparse_prefix, dim3(1), dim3(1024), 0, st, off, n, info);
     HIP_OK(hipGetLastError());
     return 0;
 }
 
-int launch_sparse_fill(const uint32_t *y, int n, int stride, int *off, int *idx, uint32_t *val, hipStream_t st)
+int launch_sparse_fill(const uint32_t *y, int n, int stride, const int *off, int *idx, uint32_t *val, hipStream_t st)
 {
     if (n <= 0) return 0;
-    hipLaunchKernelGGL(k_sparse_prefix, dim3(1), dim3(1024), 0, st, off, n);
     hipLaunchKernelGGL(k_sparse_fill, dim3((unsigned)(n + 3) / 4), dim3(256), 0, st, y, n, stride, off, idx, val);
     HIP_OK(hipGetLastError());
     return 0;

@@ -117,12 +117,11 @@ struct SparseY {
     const uint32_t *dense = nullptr;
     uint32_t *dense_packed = nullptr;
 };
-// The lists of dense vectors y [n][stride] (device): counts and info first
+// The lists of dense vectors y [n][stride] (device): off [n + 1] and info first
 // (info[0]: the largest slot in use plus one, info[1]: v stride + i of the first
-// entry at a slot i >= limit, or ~0), then off [n + 1], idx and val (room for
-// every entry).
+// entry at a slot i >= limit, or ~0, info[2]: the entries), then idx and val.
 int launch_sparse_count(const uint32_t *y, int n, int stride, int limit, int *off, unsigned int *info, hipStream_t st);
-int launch_sparse_fill(const uint32_t *y, int n, int stride, int *off, int *idx, uint32_t *val, hipStream_t st);
+int launch_sparse_fill(const uint32_t *y, int n, int stride, const int *off, int *idx, uint32_t *val, hipStream_t st);
 // out[v][3][N] = sum_i y_v[i] P[i] with the reference's sequential fold: keygen
 // (P = msk) and the first half of rlwe_sife_decrypt_gmp (P = c).
 int launch_fold(const SparseY &y, int nvec, const uint32_t *P, uint32_t *out, const BarrettConsts &bc,

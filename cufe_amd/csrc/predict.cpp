@@ -194,12 +194,14 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
     // through 2,000 vectors of 785 slots than the upload takes)
     DevBuf<uint32_t> dense;
     DevBuf<int> off;  // takes y_off's place once the model is accepted
-    DevBuf<unsigned int> info;  // slots in use, first entry past the keys; then largest values, limbs unequal
+    // slots in use, first entry past the keys, entries; then (from 2 on) largest
+    // values, limbs unequal
+    DevBuf<unsigned int> info;
     unsigned int h_info[6] = {};
-    if (dense.alloc((size_t)nS * IPFE_L) || info.alloc(6) || off.alloc((size_t)nS + 1)) return -1;
+    if (dense.alloc((size_t)nS * IPFE_L) || info.alloc(6) || off.alloc((size_t)nS + 1, true)) return -1;
     if (copy_to_device(dense.get(), m->sv, (size_t)nS * IPFE_L * 4, st)) return -1;
     if (launch_sparse_count(dense.get(), nS, IPFE_L, L, off.get(), info.get(), st)) return -1;
-    HIP_OK(hipMemcpyAsync(h_info, info.get(), 8, hipMemcpyDeviceToHost, st));
+    HIP_OK(hipMemcpyAsync(h_info, info.get(), 12, hipMemcpyDeviceToHost, st));
     if (sync_stream(st)) return -1;
     if (h_info[1] != ~0u) {
         ipfe_set_error("model: SV %d has feature %d beyond the key length %d", (int)(h_info[1] / IPFE_L),
@@ -220,8 +222,8 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
     // canonical, so the sum part joins the contraction (key = [-s', y]).
     const bool fz = mx < L - 1;
     const int kk = fz ? IPFE_N + ((mx + 1 + 15) / 16) * 16 : IPFE_N;
-    const size_t entries = (size_t)nS * std::max(1, mx + 1);  // at most
-    if (y_idx.alloc(entries) || y_val.alloc(entries) || sk.alloc((size_t)nS * kPoly)) return -1;
+    const size_t entries = std::max(1u, h_info[2]);
+    if (y_idx.alloc(entries, true) || y_val.alloc(entries, true) || sk.alloc((size_t)nS * kPoly, true)) return -1;
     y_off.swap(off);
     if (launch_sparse_fill(dense.get(), nS, IPFE_L, y_off.get(), y_idx.get(), y_val.get(), st)) return -1;
     y.off = y_off.get();
@@ -236,18 +238,18 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
         // (CUFE_FRAC_WIDEN=w, for tests: margins 2^w times wider, so that many
         // pairs go to the exact kernel)
         const char *wv = getenv("CUFE_FRAC_WIDEN");
-        if (margin.alloc(nS) || margin88.alloc(nS) || k16.alloc((size_t)nS * kk) ||
+        if (margin.alloc(nS, true) || margin88.alloc(nS, true) || k16.alloc((size_t)nS * kk, true) ||
             launch_keys_build(sk.get(), nS, kk, y, wv ? atoi(wv) : 0, margin.get(), margin88.get(), k16.get(),
                               info.get() + 2, (int *)info.get() + 5, st))
             return -1;
     } else {
-        if (kd.alloc((size_t)3 * nS * kk) ||
+        if (kd.alloc((size_t)3 * nS * kk, true) ||
             launch_contract_keys(sk.get(), nS, kk, 1, y, kd.get(), info.get() + 2, st))
             return -1;
     }
     HIP_OK(hipMemcpyAsync(h_info + 2, info.get() + 2, 16, hipMemcpyDeviceToHost, st));
     const int npairs = m->nr_class * (m->nr_class - 1) / 2;
-    if (coef.alloc((size_t)(m->nr_class - 1) * nS) || rho.alloc(npairs)) return -1;
+    if (coef.alloc((size_t)(m->nr_class - 1) * nS, true) || rho.alloc(npairs, true)) return -1;
     HIP_OK(hipMemcpyAsync(coef.get(), m->sv_coef, sizeof(double) * (m->nr_class - 1) * nS, hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(rho.get(), m->rho, sizeof(double) * npairs, hipMemcpyHostToDevice, st));
     if (sync_stream(st)) return -1;
@@ -281,7 +283,7 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
         if (fits) {
             std::vector<int32_t> h((size_t)(m->nr_class - 1) * nS);
             for (size_t k = 0; k < h.size(); ++k) h[k] = (int32_t)m->sv_coef[k];
-            if (icoef.alloc(h.size())) return -1;
+            if (icoef.alloc(h.size(), true)) return -1;
             HIP_OK(hipMemcpyAsync(icoef.get(), h.data(), h.size() * 4, hipMemcpyHostToDevice, st));
             if (sync_stream(st)) return -1;
             md.sv_icoef = icoef.get();
@@ -313,7 +315,7 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
     if (i8) {
         spad = (nS + 127) / 128 * 128;
         ksteps = (kk + 31) / 32;
-        if (kdig.alloc(3 * keys_digit_limb_bytes(spad, ksteps, nb))) return -1;
+        if (kdig.alloc(3 * keys_digit_limb_bytes(spad, ksteps, nb), true)) return -1;
         if (frac ? launch_keys_digits16(k16.get(), nS, kk, spad, ksteps, kdig.get(), st)
                  : launch_keys_digits(kd.get(), nS, kk, spad, ksteps, nb, kdig.get(), st))
             return -1;
@@ -331,7 +333,7 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
 int Model::make_kd(int nS, hipStream_t st) const
 {
     DevBuf<unsigned int> mx;
-    if (mx.alloc(3) || launch_fill_i32((int *)mx.get(), 0, 3, st) || kd.alloc((size_t)3 * nS * kkey)) return -1;
+    if (mx.alloc(3) || launch_fill_i32((int *)mx.get(), 0, 3, st) || kd.alloc((size_t)3 * nS * kkey, true)) return -1;
     if (launch_contract_keys(sk.get(), nS, kkey, fused ? -1 : 1, y, kd.get(), mx.get(), st) || sync_stream(st)) {
         kd.reset();
         return -1;
@@ -365,14 +367,15 @@ int RowStore::reserve(int cap_rows, int len, bool fractions)
     const int cp = ((cap_rows + 63) / 64) * 64;  // whole 64-row tiles of the blocked store
     const int ks = (IPFE_N + ((len + 31) / 32) * 32) / 32;
     A64.reset();
-    if (A.alloc((size_t)3 * cp * ld) || c0.alloc((size_t)cp * len * 3) || Adig.alloc(3 * rows_digit_limb_bytes(cp, ks)))
+    if (A.alloc((size_t)3 * cp * ld, true) || c0.alloc((size_t)cp * len * 3, true) ||
+        Adig.alloc(3 * rows_digit_limb_bytes(cp, ks), true))
         return -1;
     HIP_OK(hipMemset(A.get(), 0, (size_t)3 * cp * ld * 4));
     HIP_OK(hipMemset(Adig.get(), 0, Adig.n));
     Fdig.reset();
     Fref.reset();
     if (fractions) {
-        if (Fdig.alloc(frac_digit_bytes(cp, ks)) || Fref.alloc((size_t)cp * ks * 32)) return -1;
+        if (Fdig.alloc(frac_digit_bytes(cp, ks), true) || Fref.alloc((size_t)cp * ks * 32, true)) return -1;
         HIP_OK(hipMemset(Fdig.get(), 0, Fdig.n));
         HIP_OK(hipMemset(Fref.get(), 0, Fref.n * 2));
     }
@@ -403,7 +406,7 @@ int RowStore::put(int r0, int n, const uint32_t *cl_dev, const uint32_t *c0_dev,
 int RowStore::ensure_a64(int r0, int R, hipStream_t st) const
 {
     if (!A64.get()) {
-        if (A64.alloc((size_t)3 * (cap + 64) * ldr)) return -1;
+        if (A64.alloc((size_t)3 * (cap + 64) * ldr, true)) return -1;
         if (launch_fill_i32((int *)A64.get(), 0, A64.n * 2, st)) return -1;
     }
     const int b1 = (r0 + R + 63) / 64;
@@ -442,12 +445,13 @@ size_t Scratch::split_bytes(int rows, int S)
 int Scratch::reserve(int rows, int S)
 {
     if (D.n < (size_t)3 * rows * S || kval.n < (size_t)rows * S || labels.n < (size_t)rows) {
-        if (D.alloc((size_t)3 * rows * S) || kval.alloc((size_t)rows * S) || labels.alloc(rows)) return -1;
+        if (D.alloc((size_t)3 * rows * S, true) || kval.alloc((size_t)rows * S, true) || labels.alloc(rows, true))
+            return -1;
     }
     // split-K slices of the small row ranges that fit: up to 3 x 16 x the
     // pairs (allocated here, not while serving)
     const size_t part = split_bytes(rows, S) / 4;
-    if (Dpart.n < part && Dpart.alloc(part)) return -1;
+    if (Dpart.n < part && Dpart.alloc(part, true)) return -1;
     if (!flag.get() && flag.alloc(1)) return -1;
     return 0;
 }
@@ -513,7 +517,7 @@ int predict_rows(const Model &m, const RowStore &rs, int row0, int nrows, Scratc
         if (split) {
             // at most 16 slices: Scratch::reserve holds 48 x 2^19 words
             const size_t need = (size_t)3 * split_k_slices(R, S, m.ksteps) * R * S;
-            if (sc.Dpart.n < need && sc.Dpart.alloc(need)) return -1;
+            if (sc.Dpart.n < need && sc.Dpart.alloc(need, true)) return -1;
             if (launch_contract_i8_split(rs.Adig.get() + (size_t)(r0 / 32) * rs.ksteps * 4 * 1024,
                                          rows_digit_limb_bytes(rs.cap, rs.ksteps), rs.ksteps, m.kdig.get(),
                                          keys_digit_limb_bytes(m.spad, m.ksteps, m.nb), m.ksteps, R, S,

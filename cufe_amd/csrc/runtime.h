@@ -33,9 +33,12 @@ Device *device();
 // A device block of at least `bytes` bytes, uninitialised, and its release.
 // Released blocks are kept for the next allocation (xfer.cpp): bounded, from
 // any thread; a block is not handed out again before the device has finished
-// the work issued before its release.
-int dev_alloc(void **out, size_t bytes);
+// the work issued before its release.  exact: a block of that size (to 512 bytes),
+// for buffers that stay; others may be an eighth larger.
+int dev_alloc(void **out, size_t bytes, bool exact = false);
 void dev_free(void *p);
+// Frees the blocks kept.
+void dev_trim();
 
 // Copies between device memory and the caller's, after the work st holds; what
 // st is given later follows a copy_to_device.  Large copies to or from
@@ -67,11 +70,11 @@ struct DevBuf {
         p = nullptr;
         n = 0;
     }
-    int alloc(size_t count)
+    int alloc(size_t count, bool exact = false)
     {
         reset();
         if (count == 0) return 0;
-        if (dev_alloc((void **)&p, count * sizeof(T))) return -1;
+        if (dev_alloc((void **)&p, count * sizeof(T), exact)) return -1;
         n = count;
         return 0;
     }

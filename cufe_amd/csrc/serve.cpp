@@ -544,10 +544,11 @@ extern "C" int cufe_server_start(cufe_server *s)
     s->slot_bytes = (size_t)s->cap * per_row + split;
     const int nslots = (int)std::max<size_t>(2, std::min<size_t>(4, avail / s->slot_bytes));
     const size_t stage_words = (size_t)s->cap * (kPoly + (size_t)s->l_max * 3);
+    dev_trim();  // what the models' builds left: the budget is for models and slots
     for (int i = 0; i < nslots; ++i) {
         s->slots.push_back(std::make_unique<Slot>());
         Slot &sl = *s->slots.back();
-        if (sl.rows.reserve(s->cap, s->l_max) || sl.sc.reserve(s->cap, s->S_max) || sl.d_stage.alloc(stage_words))
+        if (sl.rows.reserve(s->cap, s->l_max) || sl.sc.reserve(s->cap, s->S_max) || sl.d_stage.alloc(stage_words, true))
             return -1;
         HIP_OK(hipHostMalloc((void **)&sl.h_stage, stage_words * 4, hipHostMallocDefault));
         HIP_OK(hipHostMalloc((void **)&sl.h_labels, sizeof(double) * s->cap, hipHostMallocDefault));

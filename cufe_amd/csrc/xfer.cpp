@@ -6,9 +6,13 @@
 // 0.4 ms each, and calls that follow one another wait for the driver to give
 // the freed memory out again (a 2,000-SV model rebuilt in a loop: 2.2 to 9.9 ms
 // a pass, 1.4 with the blocks kept).  Blocks are therefore kept when a DevBuf
-// lets go of them and handed to the next one of the same size class, up to
+// lets go of them and handed to the next one they fit, up to
 // kPoolBytes per process; what exceeds that is freed, and everything kept is
-// freed when an allocation fails.  hipFree also waited for the device, so a
+// freed when an allocation fails.  A block of up to kClassMax bytes is rounded up
+// by an eighth at most, so that calls of similar sizes share it (8 MiB at most
+// lost); a larger one has its own size, and is kept for requests down to eight
+// ninths of it.  Buffers that stay and are counted against a budget or fill the
+// card (models, row stores, a server's slots) are exact: their own size, new or kept.  hipFree also waited for the device, so a
 // block could be let go of with work in flight (an error return between
 // launches); here the device is waited for before a block released since the
 // last wait is handed out again.
@@ -45,6 +49,7 @@ namespace ipfe {
 namespace {
 
 constexpr size_t kPoolBytes = (size_t)4 << 30;  // kept at most; larger blocks are never kept
+constexpr size_t kClassMax = (size_t)64 << 20;  // rounded up to here
 
 struct Block {
     void *p;
@@ -53,7 +58,7 @@ struct Block {
 
 struct Pool {
     std::mutex mu;
-    std::map<std::pair<int, size_t>, std::vector<Block>> free;  // by device and class size
+    std::map<std::pair<int, size_t>, std::vector<Block>> free;  // by device and size
     std::map<void *, std::pair<int, size_t>> live;
     size_t kept = 0;
     uint64_t releases = 0, waited = 0;  // blocks released up to `waited` are idle
@@ -67,11 +72,13 @@ Pool &pool()
     return *p;
 }
 
-// Sizes share a block within an eighth of the next power of two.
-size_t size_class(size_t bytes)
+// A request's own size, and the size a new block for it has.
+size_t own_size(size_t bytes) { return (bytes + 511) / 512 * 512; }
+size_t block_size(size_t bytes, bool exact)
 {
-    size_t step = 512;
-    while (step * 8 < bytes) step *= 2;
+    if (exact || bytes > kClassMax) return own_size(bytes);
+    size_t step = 512;  // of the sizes from 8 to 16 steps
+    while (step * 16 <= bytes) step *= 2;
     return (bytes + step - 1) / step * step;
 }
 
@@ -86,32 +93,36 @@ void drop_all(Pool &pl)
 
 }  // namespace
 
-int dev_alloc(void **out, size_t bytes)
+int dev_alloc(void **out, size_t bytes, bool exact)
 {
     *out = nullptr;
     Pool &pl = pool();
     int dev = 0;
     HIP_OK(hipGetDevice(&dev));
-    const std::pair<int, size_t> key(dev, size_class(bytes));
+    std::pair<int, size_t> key(dev, block_size(bytes, exact));
     std::lock_guard<std::mutex> lk(pl.mu);
-    auto it = pl.free.find(key);
-    if (it != pl.free.end() && !it->second.empty()) {
+    // the smallest kept block that holds it
+    auto it = pl.free.lower_bound(key);
+    while (it != pl.free.end() && it->first.first == dev && it->second.empty()) it = pl.free.erase(it);
+    if (it != pl.free.end() && it->first.first == dev &&
+        it->first.second <= (exact ? key.second : key.second + key.second / 8)) {
         // the block released first is the likeliest to be idle already
         const Block b = it->second.front();
         if (b.released <= pl.waited || hipDeviceSynchronize() == hipSuccess) {
             if (b.released > pl.waited) pl.waited = pl.releases;
             it->second.erase(it->second.begin());
-            pl.kept -= key.second;
-            pl.live[b.p] = key;
+            pl.kept -= it->first.second;
+            pl.live[b.p] = it->first;
             *out = b.p;
             return 0;
         }
         (void)hipGetLastError();
     }
     hipError_t e = hipMalloc(out, key.second);
-    if (e != hipSuccess && pl.kept > 0) {
+    if (e != hipSuccess) {
         (void)hipGetLastError();
         drop_all(pl);
+        key.second = own_size(bytes);
         e = hipMalloc(out, key.second);
     }
     if (e != hipSuccess) {
@@ -122,6 +133,13 @@ int dev_alloc(void **out, size_t bytes)
     }
     pl.live[*out] = key;
     return 0;
+}
+
+void dev_trim()
+{
+    Pool &pl = pool();
+    std::lock_guard<std::mutex> lk(pl.mu);
+    drop_all(pl);
 }
 
 void dev_free(void *p)

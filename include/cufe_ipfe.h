@@ -332,7 +332,8 @@ typedef struct cufe_server cufe_server;
  * device bytes for keys and the batch slots (0 = 16 GiB): a slot holds up to
  * max_batch_rows rows (0 = 4096) if two such slots fit, fewer otherwise, and
  * the budget left over buys up to two more slots; batching 0 runs one request
- * (part) per batch. */
+ * (part) per batch.  Device blocks that the library keeps from calls that have
+ * returned, for the next ones (at most 4 GiB a process), are not part of it. */
 int cufe_server_create(cufe_ctx *ctx, size_t hbm_budget, int max_batch_rows, int batching, cufe_server **out);
 /* Generates and keeps the functional keys of one model (before start). */
 int cufe_server_add_model(cufe_server *srv, const cufe_svm_model *model, int *model_id);
