@@ -61,7 +61,8 @@ struct Pool {
     std::map<std::pair<int, size_t>, std::vector<Block>> free;  // by device and size
     std::map<void *, std::pair<int, size_t>> live;
     size_t kept = 0;
-    uint64_t releases = 0, waited = 0;  // blocks released up to `waited` are idle
+    uint64_t releases = 0;
+    std::map<int, uint64_t> waited;  // a device's blocks released up to here are idle
 };
 
 // Never destroyed: the process's end gives the blocks back, in no set order
@@ -108,8 +109,9 @@ int dev_alloc(void **out, size_t bytes, bool exact)
         it->first.second <= (exact ? key.second : key.second + key.second / 8)) {
         // the block released first is the likeliest to be idle already
         const Block b = it->second.front();
-        if (b.released <= pl.waited || hipDeviceSynchronize() == hipSuccess) {
-            if (b.released > pl.waited) pl.waited = pl.releases;
+        uint64_t &waited = pl.waited[dev];
+        if (b.released <= waited || hipDeviceSynchronize() == hipSuccess) {
+            if (b.released > waited) waited = pl.releases;
             it->second.erase(it->second.begin());
             pl.kept -= it->first.second;
             pl.live[b.p] = it->first;

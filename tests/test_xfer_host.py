@@ -1,6 +1,6 @@
 """The pool of device blocks and the staged copies on the CPU, over a HIP runtime
 that tests/xfer_host/xfer_host.cpp brings itself: sizes asked of the driver, which
-kept block a request takes, and what is freed when.  The HIP headers are
+kept block a request takes, what it waits for, and what is freed when.  The HIP headers are
 needed, a GPU is not."""
 import os
 import subprocess
@@ -21,7 +21,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["sizes", "card"])
+@pytest.mark.parametrize("check", ["sizes", "card", "devices"])
 def test_pool(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr

@@ -166,11 +166,33 @@ void card()
     dev_free(q);
     dev_free(p);
 }
+
+// a block is waited for on its own device before it is handed out again
+void devices()
+{
+    void *a[2];
+    for (drv.device = 0; drv.device < 2; ++drv.device) a[drv.device] = take(MiB);
+    for (int d : {0, 1}) dev_free(a[d]);
+    for (drv.device = 0; drv.device < 2; ++drv.device) {
+        EXPECT(drv.syncs[drv.device] == 0);
+        EXPECT(take(MiB) == a[drv.device]);
+        EXPECT(drv.syncs[drv.device] == 1);
+    }
+    drv.device = 1;
+    dev_free(a[0]);  // device 0's, released with device 1 current
+    EXPECT(take(MiB) != a[0]);
+    drv.device = 0;
+    EXPECT(take(MiB) == a[0] && drv.syncs[0] == 2);
+    // one wait covers every block released before it
+    void *p[3] = {take(2 * MiB), take(3 * MiB), take(5 * MiB)};
+    for (void *q : p) dev_free(q);
+    EXPECT(take(5 * MiB) == p[2] && take(2 * MiB) == p[0] && take(3 * MiB) == p[1] && drv.syncs[0] == 3);
+}
 }  // namespace
 
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"sizes", sizes}, {"card", card}};
+    const std::map<std::string, void (*)()> checks = {{"sizes", sizes}, {"card", card}, {"devices", devices}};
     EXPECT(argc == 2 && checks.count(argv[1]));
     checks.at(argv[1])();
     printf("%s ok\n", argv[1]);
