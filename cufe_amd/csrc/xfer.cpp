@@ -6,13 +6,15 @@
 // 0.4 ms each, and calls that follow one another wait for the driver to give
 // the freed memory out again (a 2,000-SV model rebuilt in a loop: 2.2 to 9.9 ms
 // a pass, 1.4 with the blocks kept).  Blocks are therefore kept when a DevBuf
-// lets go of them and handed to the next one they fit, up to
-// kPoolBytes per process; what exceeds that is freed, and everything kept is
-// freed when an allocation fails.  A block of up to kClassMax bytes is rounded up
-// by an eighth at most, so that calls of similar sizes share it (8 MiB at most
-// lost); a larger one has its own size, and is kept for requests down to eight
-// ninths of it.  Buffers that stay and are counted against a budget or fill the
-// card (models, row stores, a server's slots) are exact: their own size, new or kept.  hipFree also waited for the device, so a
+// lets go of them and handed to the next one they fit, up to kPoolBytes per
+// process; beyond that those released longest ago are freed (a process whose
+// sizes change would otherwise sit on blocks it no longer asks for), and
+// everything kept is freed when an allocation fails.  A block of up to kClassMax
+// bytes is rounded up by an eighth at most, so that calls of similar sizes share
+// it (8 MiB at most lost); a larger one has its own size, and is kept for
+// requests down to eight ninths of it.  Buffers that stay and are counted against
+// a budget or fill the card (models, row stores, a server's slots) are exact:
+// their own size, new or kept.  hipFree also waited for the device, so a
 // block could be let go of with work in flight (an error return between
 // launches); here the device is waited for before a block released since the
 // last wait is handed out again.
@@ -58,7 +60,7 @@ struct Block {
 
 struct Pool {
     std::mutex mu;
-    std::map<std::pair<int, size_t>, std::vector<Block>> free;  // by device and size
+    std::map<std::pair<int, size_t>, std::vector<Block>> free;  // by device and size; none empty
     std::map<void *, std::pair<int, size_t>> live;
     size_t kept = 0;
     uint64_t releases = 0;
@@ -92,6 +94,18 @@ void drop_all(Pool &pl)
     pl.kept = 0;
 }
 
+// Frees the block kept longest (mu held, something is kept).
+void drop_oldest(Pool &pl)
+{
+    auto old = pl.free.end();
+    for (auto it = pl.free.begin(); it != pl.free.end(); ++it)
+        if (old == pl.free.end() || it->second.front().released < old->second.front().released) old = it;
+    (void)hipFree(old->second.front().p);
+    pl.kept -= old->first.second;
+    old->second.erase(old->second.begin());
+    if (old->second.empty()) pl.free.erase(old);
+}
+
 }  // namespace
 
 int dev_alloc(void **out, size_t bytes, bool exact)
@@ -104,7 +118,6 @@ int dev_alloc(void **out, size_t bytes, bool exact)
     std::lock_guard<std::mutex> lk(pl.mu);
     // the smallest kept block that holds it
     auto it = pl.free.lower_bound(key);
-    while (it != pl.free.end() && it->first.first == dev && it->second.empty()) it = pl.free.erase(it);
     if (it != pl.free.end() && it->first.first == dev &&
         it->first.second <= (exact ? key.second : key.second + key.second / 8)) {
         // the block released first is the likeliest to be idle already
@@ -112,9 +125,10 @@ int dev_alloc(void **out, size_t bytes, bool exact)
         uint64_t &waited = pl.waited[dev];
         if (b.released <= waited || hipDeviceSynchronize() == hipSuccess) {
             if (b.released > waited) waited = pl.releases;
-            it->second.erase(it->second.begin());
-            pl.kept -= it->first.second;
             pl.live[b.p] = it->first;
+            pl.kept -= it->first.second;
+            it->second.erase(it->second.begin());
+            if (it->second.empty()) pl.free.erase(it);
             *out = b.p;
             return 0;
         }
@@ -153,10 +167,11 @@ void dev_free(void *p)
     if (it == pl.live.end()) return;
     const std::pair<int, size_t> key = it->second;
     pl.live.erase(it);
-    if (pl.kept + key.second > kPoolBytes) {
+    if (key.second > kPoolBytes) {
         (void)hipFree(p);
         return;
     }
+    while (pl.kept + key.second > kPoolBytes) drop_oldest(pl);
     pl.kept += key.second;
     pl.free[key].push_back(Block{p, ++pl.releases});
 }

@@ -188,11 +188,42 @@ void devices()
     for (void *q : p) dev_free(q);
     EXPECT(take(5 * MiB) == p[2] && take(2 * MiB) == p[0] && take(3 * MiB) == p[1] && drv.syncs[0] == 3);
 }
+
+// beyond 4 GiB kept, the blocks released longest ago are freed, and calls of a
+// size not seen before find their blocks again
+void bound()
+{
+    std::vector<void *> v;
+    for (int i = 0; i < 9; ++i) v.push_back(take(512 * MiB + 512 * i));
+    for (void *p : v) dev_free(p);
+    EXPECT(drv.freed == std::vector<void *>({v[0], v[1]}));  // seven of them stay below 4 GiB
+    EXPECT(drv.used <= 4 * GiB);
+    const int mallocs = drv.mallocs;
+    for (int i = 0; i < 5; ++i) {
+        void *p = take(100 * MiB);
+        dev_free(p);
+    }
+    EXPECT(drv.mallocs == mallocs + 1 && drv.used <= 4 * GiB);
+    void *p = take(450 * MiB);
+    dev_free(p);
+    EXPECT(drv.freed == std::vector<void *>({v[0], v[1], v[2]}) && take(450 * MiB) == p);
+    dev_free(p);
+    p = take(4 * GiB + 1);  // never kept, and nothing goes for it
+    dev_free(p);
+    EXPECT(drv.freed.size() == 4 && drv.freed.back() == p);
+    p = take(4 * GiB);
+    dev_free(p);
+    EXPECT(drv.used == 4 * GiB && take(4 * GiB) == p);
+    dev_free(p);
+    dev_trim();
+    EXPECT(drv.used == 0 && drv.blocks.empty());
+    dev_free(nullptr);
+}
 }  // namespace
 
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"sizes", sizes}, {"card", card}, {"devices", devices}};
+    const std::map<std::string, void (*)()> checks = {{"sizes", sizes}, {"card", card}, {"devices", devices}, {"bound", bound}};
     EXPECT(argc == 2 && checks.count(argv[1]));
     checks.at(argv[1])();
     printf("%s ok\n", argv[1]);
