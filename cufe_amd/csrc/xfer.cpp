@@ -108,9 +108,8 @@ void drop_oldest(Pool &pl)
 
 }  // namespace
 
-int dev_alloc(void **out, size_t bytes, bool exact)
+static int take_block(void **out, size_t bytes, bool exact)
 {
-    *out = nullptr;
     Pool &pl = pool();
     int dev = 0;
     HIP_OK(hipGetDevice(&dev));
@@ -147,8 +146,27 @@ int dev_alloc(void **out, size_t bytes, bool exact)
         ipfe_set_error("hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
         return -1;
     }
-    pl.live[*out] = key;
+    try {
+        pl.live[*out] = key;
+    } catch (...) {
+        (void)hipFree(*out);
+        *out = nullptr;
+        throw;
+    }
     return 0;
+}
+
+// Callers are entry points of the C ABI and destructors: host memory that runs
+// out for the pool's own records is an error like the device's.
+int dev_alloc(void **out, size_t bytes, bool exact)
+{
+    *out = nullptr;
+    try {
+        return take_block(out, bytes, exact);
+    } catch (...) {
+        ipfe_set_error("no host memory to record a block of %zu bytes", bytes);
+        return -1;
+    }
 }
 
 void dev_trim()
@@ -172,8 +190,19 @@ void dev_free(void *p)
         return;
     }
     while (pl.kept + key.second > kPoolBytes) drop_oldest(pl);
-    pl.kept += key.second;
-    pl.free[key].push_back(Block{p, ++pl.releases});
+    try {
+        auto &kept = pl.free[key];
+        try {
+            kept.push_back(Block{p, pl.releases + 1});
+        } catch (...) {
+            if (kept.empty()) pl.free.erase(key);
+            throw;
+        }
+        ++pl.releases;
+        pl.kept += key.second;
+    } catch (...) {
+        (void)hipFree(p);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -193,20 +222,18 @@ struct Lane {  // one copy thread's stream and pinned chunks
 
 class Copier {
 public:
-    // nullptr where the threads or their pinned memory cannot be had
+    // nullptr where the threads, their pinned or other memory cannot be had
     static Copier *get(int dev)
     {
         static std::mutex mu;
-        static std::map<int, Copier *> all;  // never destroyed, as the pool
+        static std::map<int, Copier *> &all = *new std::map<int, Copier *>();  // never destroyed, as the pool
         std::lock_guard<std::mutex> lk(mu);
         auto it = all.find(dev);
         if (it == all.end()) {
+            it = all.emplace(dev, nullptr).first;
             Copier *c = new Copier(dev);
-            if (!c->ok) {
-                delete c;
-                c = nullptr;
-            }
-            it = all.emplace(dev, c).first;
+            if (c->ok) it->second = c;
+            else delete c;
         }
         return it->second;
     }
@@ -265,15 +292,16 @@ private:
         if (sched_getaffinity(0, sizeof set, &set) == 0) cpus = CPU_COUNT(&set);
         const int n = std::max(1, std::min(kMaxCopyThreads, cpus / 2));
         bool good = hipEventCreateWithFlags(&start, hipEventDisableTiming) == hipSuccess;
-        for (int i = 0; i < n && good; ++i) {
-            Lane l;
-            good = hipStreamCreateWithFlags(&l.st, hipStreamNonBlocking) == hipSuccess;
-            for (int j = 0; j < 2 && good; ++j)
-                good = hipHostMalloc((void **)&l.slot[j], kChunk, hipHostMallocDefault) == hipSuccess &&
-                       hipEventCreateWithFlags(&l.ev[j], hipEventDisableTiming) == hipSuccess;
-            lanes.push_back(l);
-        }
         try {
+            lanes.reserve(n);
+            for (int i = 0; i < n && good; ++i) {
+                Lane l;
+                good = hipStreamCreateWithFlags(&l.st, hipStreamNonBlocking) == hipSuccess;
+                for (int j = 0; j < 2 && good; ++j)
+                    good = hipHostMalloc((void **)&l.slot[j], kChunk, hipHostMallocDefault) == hipSuccess &&
+                           hipEventCreateWithFlags(&l.ev[j], hipEventDisableTiming) == hipSuccess;
+                lanes.push_back(l);
+            }
             for (int i = 0; i + 1 < n && good; ++i) threads.emplace_back([this, i] { loop(i); });
         } catch (...) {
             good = false;
@@ -377,7 +405,11 @@ int copy(void *dst, const void *src, size_t bytes, bool to_host, hipStream_t st,
     if (bytes >= kStageMin && pageable(to_host ? dst : src)) {
         int dev = 0;
         HIP_OK(hipGetDevice(&dev));
-        Copier *c = Copier::get(dev);
+        Copier *c = nullptr;
+        try {
+            c = Copier::get(dev);
+        } catch (...) {  // no host memory for it: the runtime's copy
+        }
         hipError_t e = hipSuccess;
         if (c && c->run((uint8_t *)dst, (const uint8_t *)src, bytes, to_host, st, beside, &e)) {
             if (e == hipSuccess) return 0;

@@ -10,6 +10,7 @@
 
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -38,10 +39,30 @@ std::string last_error;
             exit(1);                                                   \
         }                                                              \
     } while (0)
+
+// this thread's allocations still to succeed; -1: all of them
+thread_local long allow = -1;
+struct Fed {  // this file's own records, whatever the library may allocate
+    long left = allow;
+    Fed() { allow = -1; }
+    ~Fed() { allow = left; }
+};
 }  // namespace
+
+void *operator new(size_t n)
+{
+    if (allow == 0) throw std::bad_alloc();
+    if (allow > 0) --allow;
+    void *p = malloc(n);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
 
 void ipfe_set_error(const char *fmt, ...)
 {
+    Fed fed;
     char b[512];
     va_list ap;
     va_start(ap, fmt);
@@ -58,6 +79,7 @@ const char *hipGetErrorString(hipError_t) { return "fake"; }
 hipError_t hipDeviceSynchronize(void) { ++drv.syncs[drv.device]; return hipSuccess; }
 hipError_t hipMalloc(void **p, size_t n)
 {
+    Fed fed;
     std::lock_guard<std::mutex> lk(drv.mu);
     if (drv.used + n > drv.card) return hipErrorOutOfMemory;
     ++drv.mallocs;
@@ -69,6 +91,7 @@ hipError_t hipMalloc(void **p, size_t n)
 }
 hipError_t hipFree(void *p)
 {
+    Fed fed;
     std::lock_guard<std::mutex> lk(drv.mu);
     EXPECT(drv.blocks.count(p));
     drv.used -= drv.blocks[p].first;
@@ -219,11 +242,68 @@ void bound()
     EXPECT(drv.used == 0 && drv.blocks.empty());
     dev_free(nullptr);
 }
+
+// f with n allocations left
+template <class F>
+auto starved(long n, F f)
+{
+    allow = n;
+    auto r = f();
+    allow = -1;
+    return r;
+}
+
+// host memory that runs out is an error, and no block is lost or ends the process
+void starve()
+{
+    for (int n = 0; n < 4; ++n) {
+        void *p = (void *)1;
+        if (starved(n, [&] { return dev_alloc(&p, MiB); })) {
+            EXPECT(!p && drv.used == 0);
+            EXPECT(last_error.find("no host memory") == 0);
+        } else {
+            EXPECT(p && size_of(p) == MiB);
+            starved(0, [&] { dev_free(p); return 0; });  // cannot be recorded: freed
+            EXPECT(drv.used == 0);
+        }
+    }
+    void *p = take(MiB);
+    dev_free(p);
+    EXPECT(take(MiB) == p);  // the records are sound
+    // a copy that cannot have its threads goes through the runtime
+    drv.backed = true;
+    std::vector<uint8_t> a(6 * MiB, 7), b(6 * MiB);
+    EXPECT(starved(0, [&] { return copy_to_device(b.data(), a.data(), a.size(), nullptr); }) == 0);
+    EXPECT(a == b);
+}
+
+// large copies of several threads at once, each to and from its own arrays: all
+// end, with their own bytes, whichever of them has the copy threads
+void copies()
+{
+    std::atomic<int> done{0};
+    std::vector<std::thread> t;
+    for (int k = 0; k < 6; ++k)
+        t.emplace_back([k, &done] {
+            for (int i = 0; i < 12; ++i) {
+                const size_t n = 4 * MiB + (size_t)k * 777777 + i * 131071;
+                std::vector<uint8_t> a(n), b(n), c(n);
+                for (size_t j = 0; j < n; ++j) a[j] = (uint8_t)(j * 31 + j / 4096 + k + i);
+                EXPECT((i & 1 ? copy_to_device : copy_to_device_beside)(b.data(), a.data(), n, nullptr) == 0);
+                EXPECT(copy_to_host(c.data(), b.data(), n, nullptr) == 0);
+                EXPECT(a == b && a == c);
+                ++done;
+            }
+        });
+    for (auto &x : t) x.join();
+    EXPECT(done == 72);
+}
 }  // namespace
 
 int main(int argc, char **argv)
 {
-    const std::map<std::string, void (*)()> checks = {{"sizes", sizes}, {"card", card}, {"devices", devices}, {"bound", bound}};
+    const std::map<std::string, void (*)()> checks = {{"sizes", sizes}, {"card", card}, {"devices", devices}, {"bound", bound},
+                                                      {"starve", starve}, {"copies", copies}};
     EXPECT(argc == 2 && checks.count(argv[1]));
     checks.at(argv[1])();
     printf("%s ok\n", argv[1]);
