@@ -223,9 +223,11 @@ int Model::build(const uint32_t *msk_dev, int L, const cufe_svm_model *m, hipStr
     const bool fz = mx < L - 1;
     const int kk = fz ? IPFE_N + ((mx + 1 + 15) / 16) * 16 : IPFE_N;
     const size_t entries = std::max(1u, h_info[2]);
-    if (y_idx.alloc(entries, true) || y_val.alloc(entries, true) || sk.alloc((size_t)nS * kPoly, true)) return -1;
+    if (y_idx.alloc(entries, true) || y_val.alloc(entries, true)) return -1;
     y_off.swap(off);
     if (launch_sparse_fill(dense.get(), nS, IPFE_L, y_off.get(), y_idx.get(), y_val.get(), st)) return -1;
+    dense.reset();  // not beside the keys: 3 KB a vector
+    if (sk.alloc((size_t)nS * kPoly, true)) return -1;
     y.off = y_off.get();
     y.idx = y_idx.get();
     y.val = y_val.get();
@@ -1015,15 +1017,32 @@ extern "C" int cufe_ctx_export_rows(const cufe_ctx *c, int row0, int n, uint32_t
     }
     const RowStore &rs = c->rows;
     hipStream_t st = device()->stream;
-    // canonical words in blocks of rows, so that the copy out is one
+    // canonical words in blocks of rows, so that the copy out is one; a store that
+    // fills the card leaves no room for a block, and its words are made here
     constexpr int kBlock = 4096;
     DevBuf<uint32_t> out;
-    if (out.alloc((size_t)std::min(n, kBlock) * kPoly)) return -1;
-    for (int r = 0; r < n; r += kBlock) {
-        const int k = std::min(kBlock, n - r);
-        if (launch_rows_export(rs.A.get(), rs.cap, rs.ldr, row0 + r, k, out.get(), st) ||
-            copy_to_host(cl + (size_t)r * kPoly, out.get(), (size_t)k * kPoly * 4, st) || sync_stream(st))
-            return -1;
+    if (!out.alloc((size_t)std::min(n, kBlock) * kPoly)) {
+        for (int r = 0; r < n; r += kBlock) {
+            const int k = std::min(kBlock, n - r);
+            if (launch_rows_export(rs.A.get(), rs.cap, rs.ldr, row0 + r, k, out.get(), st) ||
+                copy_to_host(cl + (size_t)r * kPoly, out.get(), (size_t)k * kPoly * 4, st) || sync_stream(st))
+                return -1;
+        }
+    } else {
+        std::vector<int32_t> a((size_t)std::min(n, kBlock) * rs.ldr);
+        for (int r0 = 0; r0 < n; r0 += kBlock)
+            for (int s = 0; s < 3; ++s) {
+                const int k = std::min(kBlock, n - r0);
+                if (copy_to_host(a.data(), rs.A.get() + ((size_t)s * rs.cap + row0 + r0) * rs.ldr,
+                                 (size_t)k * rs.ldr * 4, st) ||
+                    sync_stream(st))
+                    return -1;
+                for (int r = 0; r < k; ++r) {
+                    uint32_t *dst = cl + ((size_t)(r0 + r) * 3 + s) * IPFE_N;
+                    const int32_t *src = a.data() + (size_t)r * rs.ldr;
+                    for (int j = 0; j < IPFE_N; ++j) dst[j] = (uint32_t)src[j] + (src[j] < 0 ? qmod(s) : 0u);
+                }
+            }
     }
     if (copy_to_host(c0, rs.c0.get() + (size_t)row0 * rs.l * 3, (size_t)n * rs.l * 3 * 4, st)) return -1;
     return sync_stream(st);
