@@ -544,7 +544,6 @@ extern "C" int cufe_server_start(cufe_server *s)
     s->slot_bytes = (size_t)s->cap * per_row + split;
     const int nslots = (int)std::max<size_t>(2, std::min<size_t>(4, avail / s->slot_bytes));
     const size_t stage_words = (size_t)s->cap * (kPoly + (size_t)s->l_max * 3);
-    dev_trim();  // what the models' builds left: the budget is for models and slots
     for (int i = 0; i < nslots; ++i) {
         s->slots.push_back(std::make_unique<Slot>());
         Slot &sl = *s->slots.back();
@@ -557,6 +556,7 @@ extern "C" int cufe_server_start(cufe_server *s)
         HIP_OK(hipStreamCreateWithFlags(&sl.st, hipStreamNonBlocking));
         HIP_OK(hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));
     }
+    dev_trim();  // what the models' builds left is not beside them
     HIP_OK(hipDeviceSynchronize());
     // Run every model once per power-of-two batch size on the (zeroed) rows of
     // slot 0, with and without the split-K launch for small batches (a batch
