@@ -19,15 +19,21 @@
 // launches); here the device is waited for before a block released since the
 // last wait is handed out again.
 //
-// Copies.  A copy to pageable memory runs at 17 GB/s through the runtime, at 9
-// to 10 GB/s when the buffer's pages are new (a caller's fresh array), and at
-// 29 GB/s from pageable memory; one core copying and taking the page faults is
-// the limit, not the link (57 GB/s).  Copies of kStageMin bytes and more go
-// through pinned chunks instead, a few threads each copying a chunk to or from
-// the caller while the others' chunks cross the link: 33 GB/s to new arrays and 42
-// from pageable ones (the reference's 38.6 MB keys: 4.4 -> 1.2 ms out, 1.4 -> 0.9
-// in).  Six threads and eight give the same, more than eight are slower; chunks
-// of 1 MiB load at 30 GB/s.
+// Copies.  A copy to pageable memory runs at 17 GB/s through the runtime, and
+// one from it at 29 to 39; one core copying and taking the page faults is the
+// limit, not the link (57 GB/s).  Large copies go through pinned chunks
+// instead, a few threads each copying a chunk to or from the caller while the
+// others' chunks cross the link: the reference's 38.6 MB keys 2.2 -> 0.95 ms out,
+// 1.35 -> 0.9 in (a whole key generation).  Waking the threads, filling and
+// draining their chunks costs a small copy some 0.06 ms, so it gains less: out 16.8 MB 0.97 -> 0.47 ms,
+// 8.4 MB 0.49 -> 0.31, 6.3 MB 0.37 -> 0.27, 4.2 MB level, and from kStageDown bytes on
+// they take them.  In, a key generation over 4.2, 6.3, 8.4, 12.6 and 16.8 MB
+// takes 181, 228, 293, 395 and 510 us with the runtime's copy where the caches hold the
+// source, 226, 295, 380, 522 and 678 where they do not, and 245, 270, 305, 400 and
+// 465 (280, 312, 357, 434 and 537) with the threads: from kStageUp on, except
+// beside a stream's work, where the runtime's copy would wait for it.  Six
+// threads and eight give the same, more than eight are slower; chunks of 1 MiB
+// load at 30 GB/s.
 #include <hip/hip_runtime.h>
 #include <sched.h>
 #include <stdint.h>
@@ -210,7 +216,7 @@ void dev_free(void *p)
 // ---------------------------------------------------------------------------
 namespace {
 
-constexpr size_t kStageMin = (size_t)4 << 20;
+constexpr size_t kStageDown = (size_t)4 << 20, kStageUp = (size_t)8 << 20;
 constexpr size_t kChunk = (size_t)2 << 20;
 constexpr int kMaxCopyThreads = 8;
 
@@ -402,7 +408,7 @@ bool pageable(const void *p)
 
 int copy(void *dst, const void *src, size_t bytes, bool to_host, hipStream_t st, bool beside)
 {
-    if (bytes >= kStageMin && pageable(to_host ? dst : src)) {
+    if (bytes >= (to_host || beside ? kStageDown : kStageUp) && pageable(to_host ? dst : src)) {
         int dev = 0;
         HIP_OK(hipGetDevice(&dev));
         Copier *c = nullptr;

@@ -21,7 +21,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["sizes", "card", "devices", "bound", "starve", "copies"])
+@pytest.mark.parametrize("check", ["sizes", "card", "devices", "bound", "starve", "copies", "paths"])
 def test_pool(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr

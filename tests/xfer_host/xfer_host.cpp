@@ -8,6 +8,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <new>
@@ -29,6 +30,7 @@ struct Driver {
     std::vector<void *> freed;  // in order
     uintptr_t next = 0x7000000000ull;
     int device = 0, mallocs = 0, syncs[4] = {};
+    std::atomic<int> copies{0};
 } drv;
 std::string last_error;
 
@@ -112,7 +114,7 @@ hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuc
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = malloc(n); return hipSuccess; }
 hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *) { a->type = hipMemoryTypeUnregistered; return hipSuccess; }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { memcpy(d, s, n); ++drv.copies; return hipSuccess; }
 }
 
 namespace {
@@ -272,9 +274,23 @@ void starve()
     EXPECT(take(MiB) == p);  // the records are sound
     // a copy that cannot have its threads goes through the runtime
     drv.backed = true;
-    std::vector<uint8_t> a(6 * MiB, 7), b(6 * MiB);
+    std::vector<uint8_t> a(9 * MiB, 7), b(9 * MiB);
     EXPECT(starved(0, [&] { return copy_to_device(b.data(), a.data(), a.size(), nullptr); }) == 0);
     EXPECT(a == b);
+}
+
+// where a copy goes through the threads' chunks (2 MiB each) and where in one
+void paths()
+{
+    std::vector<uint8_t> a(8 * MiB, 3), b(8 * MiB);
+    auto transfers = [&](auto copy, size_t n) {
+        const int before = drv.copies;
+        EXPECT(copy(b.data(), a.data(), n, nullptr) == 0);
+        return drv.copies - before;
+    };
+    EXPECT(transfers(copy_to_host, 4 * MiB - 1) == 1 && transfers(copy_to_host, 4 * MiB) == 2);
+    EXPECT(transfers(copy_to_device, 8 * MiB - 1) == 1 && transfers(copy_to_device, 8 * MiB) == 4);
+    EXPECT(transfers(copy_to_device_beside, 4 * MiB - 1) == 1 && transfers(copy_to_device_beside, 4 * MiB) == 2);
 }
 
 // large copies of several threads at once, each to and from its own arrays: all
@@ -286,7 +302,7 @@ void copies()
     for (int k = 0; k < 6; ++k)
         t.emplace_back([k, &done] {
             for (int i = 0; i < 12; ++i) {
-                const size_t n = 4 * MiB + (size_t)k * 777777 + i * 131071;
+                const size_t n = 8 * MiB + (size_t)k * 777777 + i * 131071;
                 std::vector<uint8_t> a(n), b(n), c(n);
                 for (size_t j = 0; j < n; ++j) a[j] = (uint8_t)(j * 31 + j / 4096 + k + i);
                 EXPECT((i & 1 ? copy_to_device : copy_to_device_beside)(b.data(), a.data(), n, nullptr) == 0);
@@ -303,7 +319,7 @@ void copies()
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> checks = {{"sizes", sizes}, {"card", card}, {"devices", devices}, {"bound", bound},
-                                                      {"starve", starve}, {"copies", copies}};
+                                                      {"starve", starve}, {"copies", copies}, {"paths", paths}};
     EXPECT(argc == 2 && checks.count(argv[1]));
     checks.at(argv[1])();
     printf("%s ok\n", argv[1]);
