@@ -220,12 +220,17 @@ __device__ __forceinline__ Cand eval_candidate(const uint32_t *ch, int c, int wh
 // equals a CDT entry's high word, so blocks 0, 1 and 7 (r1 alone) and block 15
 // (the uniform words past the tenth) are not computed; nor is more than the
 // high 32 bits of r2 and of the Bernoulli word looked at, whose low halves
-// decide only where the high halves tie.  A candidate that such a tie (6 in
-// 2^31, 1 in 2^21) or a third rejected uniform word (7e-5 of chunks) leaves
-// open is recomputed by its lane from whole words.  That leaves the 12 blocks
-// 2..6, 8..14 of 24 a chunk -- and block 17, the sign, for streams whose
-// values are stored; without them only a zero candidate's acceptance depends
-// on its sign -- where all words of blocks 0..15 took 16 (17).
+// decide only where the high halves tie.  That leaves the 12 blocks 2..6, 8..14
+// of 24 a chunk -- and block 17, the sign, for streams whose values are stored --
+// where all words of blocks 0..15 took 16 (17).  What that leaves open is looked
+// at by the candidate's lane with the block it needs: the next uniform words
+// after a third rejected one among ten (7e-5 of chunks), the sign of a zero
+// candidate of a stream that stores no values (0.2% of S1's), the whole words
+// after a tie (6 in 2^31, 1 in 2^21).  A lane's blocks go through the tile's
+// windows and scalar round keys as the others' do: 1 call of S1 13.6 us, 64 of S2
+// and S3 32 and 35, 500 streams of 3 S1 calls 275 (with every open candidate
+// recomputed from up to nine whole blocks, each from the first round: 68, 60, 71
+// and 641; the kernel for all words 15, 42, 55 and 560).
 //
 // Each wave works alone: 16 chunks are 192 blocks, three full rounds of the
 // wave (blocks 2-5, 8-11 and 6, 12-14, so that a round's lanes need the same
@@ -318,62 +323,43 @@ __device__ __forceinline__ bool bernoulli_exp_less(uint32_t res_hi, uint32_t rm_
     return e < 64u && (r_exp >> min(e, 31u)) == 0;
 }
 
-// One candidate from whole words of its chunk, AES block by AES block, for the
-// lanes whose candidate the high words leave open.  status: as eval_candidate.
-template <class Tab>
-__device__ Cand cand_whole(const Tab &tb, const GaussStream *S, long long chunk, int c, const WidthConsts &wc,
-                           int *status, int full, int ulim, bool lazy_sign)
+// One candidate from whole words of its chunk, for the lanes whose candidate the
+// high words leave open; y of its uniform word, block(b, o): AES block b of
+// the chunk.
+template <class Block>
+__device__ Cand cand_whole(const Block &block, int c, uint32_t y, const WidthConsts &wc, bool lazy_sign)
 {
+    const int g = c >> 2, ln = c & 3;
     uint32_t o[4] = {0, 0, 0, 0};
     int cur = -1;
-    auto word = [&](int i) -> uint32_t {
-        if (cur != i >> 2) {
-            cur = i >> 2;
-            aes256_ctr_block_t(tb, &S->rk[0], &S->rkf[0], S->nonce, (uint32_t)(chunk * 24 + cur), o);
-        }
-        const uint32_t lo = (i & 1) ? o[1] : o[0], hi = (i & 1) ? o[3] : o[2];
-        return (i & 2) ? hi : lo;
-    };
-    const int g = c >> 2, ln = c & 3;
-    uint32_t w[9];  // uniform, r1, r2, Bernoulli (low, high each), byte word, sign
-    int need = -1, seen = 0;
-#pragma unroll 1
-    for (int u = 0; u < 46 && need < 0; ++u) {
-        if (!full && u >= ulim) break;
-        const uint32_t t = word(50 + u);
-        if (t < wc.UQ && seen++ == c) {
-            w[0] = t;
-            need = u;
-        }
-    }
-    if (need < 0) {
-        atomicOr(status, full ? 2 : 4);
-        w[0] = 0;
-    }
+    uint32_t w[8];  // r1, r2, Bernoulli (low, high each), byte word, sign
     const int at[8] = {25 * g + 2 * ln,      25 * g + 2 * ln + 1,  25 * g + 8 + 2 * ln, 25 * g + 9 + 2 * ln,
                        25 * g + 16 + 2 * ln, 25 * g + 17 + 2 * ln, 25 * g + 24,         70};
 #pragma unroll 1
     for (int j = 0; j < 8; ++j) {
         int i = at[0];
-        uint32_t t;
 #pragma unroll
         for (int v = 1; v < 8; ++v) i = j == v ? at[v] : i;
-        t = word(i);
+        if (cur != i >> 2) {
+            cur = i >> 2;
+            block(cur, o);
+        }
+        const uint32_t lo = (i & 1) ? o[1] : o[0], hi = (i & 1) ? o[3] : o[2], t = (i & 2) ? hi : lo;
 #pragma unroll
-        for (int v = 0; v < 8; ++v) w[1 + v] = j == v ? t : w[1 + v];
+        for (int v = 0; v < 8; ++v) w[v] = j == v ? t : w[v];
     }
-    const uint64_t r1 = (((uint64_t)w[2] << 32) | w[1]) & 0x7fffffffffffffffull;
-    const uint64_t r2 = (((uint64_t)w[4] << 32) | w[3]) & 0x7fffffffffffffffull;
+    const uint64_t r1 = (((uint64_t)w[1] << 32) | w[0]) & 0x7fffffffffffffffull;
+    const uint64_t r2 = (((uint64_t)w[3] << 32) | w[2]) & 0x7fffffffffffffffull;
     uint32_t xs = 0;
 #pragma unroll
     for (int i = 0; i < 9; ++i) xs += (r2 < c_CDT[i][1]) | ((r2 == c_CDT[i][1]) & (r1 < c_CDT[i][0]));
     Cand out;
-    const uint64_t res = cand_exp(xs, uniform_y(w[0], wc), wc, out.z);
-    const uint64_t rm = ((uint64_t)w[6] << 32) | w[5];
+    const uint64_t res = cand_exp(xs, y, wc, out.z);
+    const uint64_t rm = ((uint64_t)w[5] << 32) | w[4];
     const uint64_t res_mant = (res & ((1ull << 52) - 1)) | (1ull << 52), r_mant = rm & ((1ull << 53) - 1);
-    const bool bit = (r_mant < res_mant && bernoulli_exp_less((uint32_t)(res >> 32), w[6], (w[7] >> (8 * ln)) & 255u)) ||
+    const bool bit = (r_mant < res_mant && bernoulli_exp_less((uint32_t)(res >> 32), w[5], (w[6] >> (8 * ln)) & 255u)) ||
                      res == 0x3FF0000000000000ull;
-    out.sgn = (!lazy_sign || out.z == 0) ? (w[8] >> c) & 1u : 0u;
+    out.sgn = (!lazy_sign || out.z == 0) ? (w[7] >> c) & 1u : 0u;
     out.acc = bit && (out.z != 0 || out.sgn != 0);
     return out;
 }
@@ -484,9 +470,14 @@ __global__ __launch_bounds__(CAND_NT) void k_gauss_candidates(const GaussStream 
                     const int k = 8 * e + (lane >> 3), c = lane & 7, sh = lane & 56;
                     const bool valid = k < nsub;
                     const uint32_t *q = buf + SUB_WORDS * k;
+                    // a block of the lane's chunk beyond the ones in the buffer
+                    auto block = [&](int b, uint32_t (&o)[4]) {
+                        const uint32_t ctr = (uint32_t)(chunk0 + s + k) * 24u + b;
+                        const RoundKeys rk = keys();
+                        aes256_ctr_block_win(tb, rk, rk + 60, window(ctr), ctr, o);
+                    };
                     // the c-th uniform word below UQ
                     uint32_t w = q[18 + c];
-                    bool open = false;
                     const uint64_t kept = __ballot(w < wc.UQ);
                     if (kept != ~0ull) {
                         const uint32_t bad = ~((uint32_t)((kept >> sh) & 0xffu) | (q[26] < wc.UQ ? 256u : 0u) |
@@ -495,8 +486,27 @@ __global__ __launch_bounds__(CAND_NT) void k_gauss_candidates(const GaussStream 
                         int pos = c;
     #pragma unroll
                         for (int it = 0; it < 3; ++it) pos = c + __popc(bad & ((2u << min(pos, 15)) - 1u));
-                        open = pos >= min(ulim, 10) || pos != c + __popc(bad & ((2u << min(pos, 15)) - 1u));
+                        const bool far = pos >= min(ulim, 10) || pos != c + __popc(bad & ((2u << min(pos, 15)) - 1u));
                         w = q[18 + min(pos, 9)];
+                        if (far && valid) {  // past the tenth word, after a chain of rejections or past the limit
+                            uint32_t o[4];
+                            int seen = 0, u = 0;
+                            const int end = full ? 46 : ulim;
+                            for (; u < end; ++u) {
+                                uint32_t t = q[18 + min(u, 9)];
+                                if (u >= 10) {
+                                    const int i = 50 + u;
+                                    if ((i & 3) == 0) block(i >> 2, o);
+                                    const uint32_t lo = (i & 1) ? o[1] : o[0], hi = (i & 1) ? o[3] : o[2];
+                                    t = (i & 2) ? hi : lo;
+                                }
+                                if (t < wc.UQ && seen++ == c) {
+                                    w = t;
+                                    break;
+                                }
+                            }
+                            if (u == end) atomicOr(status, full ? 2 : 4);
+                        }
                     }
                     const uint32_t y = uniform_y(w, wc);
                     // CDT rank by the high word
@@ -515,10 +525,15 @@ __global__ __launch_bounds__(CAND_NT) void k_gauss_candidates(const GaussStream 
                     const uint32_t mant = (res_hi & 0xfffffu) | 0x100000u, rmant = rm_hi & 0x1fffffu;
                     const bool bit = (rmant < mant && bernoulli_exp_less(res_hi, rm_hi, (bytes >> (8 * (c & 3))) & 255u)) ||
                                      res == 0x3FF0000000000000ull;
-                    open = valid && (whole || open || tie || rmant == mant || (!store_vals && cd.z == 0));
                     cd.sgn = store_vals ? (__shfl(sign, s + k, 64) >> c) & 1u : 0u;
                     cd.acc = valid && bit && (store_vals ? (cd.z != 0 || cd.sgn != 0) : true);
-                    if (open) cd = cand_whole(tb, S, chunk0 + s + k, c, wc, status, full, ulim, !store_vals);
+                    if (valid && (whole || tie || rmant == mant)) {
+                        cd = cand_whole(block, c, y, wc, !store_vals);
+                    } else if (!store_vals && cd.acc && cd.z == 0) {  // accepted if its sign is set
+                        uint32_t o[4];
+                        block(17, o);
+                        cd.acc = (o[2] >> c) & 1u;
+                    }
                     const uint64_t am = __ballot(cd.acc);
                     const uint32_t gm = (uint32_t)((am >> sh) & 0xffu);
                     if (valid) {

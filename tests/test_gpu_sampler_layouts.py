@@ -48,3 +48,31 @@ def test_rows(gpu, variant):
         variant()
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
     ctx.close()
+
+
+@pytest.mark.parametrize("which,k", [(2, 304214978), (3, 608429953)])
+@pytest.mark.parametrize("limit", ["14", "8"])
+def test_uniform_words_past_the_tenth(gpu, po, monkeypatch, which, k, limit):
+    """Three rejected uniform words among a chunk's first ten (7e-5 of chunks)
+    send its last candidates past the words that every chunk leaves: streams that
+    have such chunks, beside chains of rejections within the ten, against the
+    oracle."""
+    bound = k * ((1 << 32) // k)
+    n = 900 if which == 2 else 1250  # chunks below any call's length
+    keys, nonces = [], []
+    for t in range(1000):
+        key = h(b"far%d-%d" % (which, t))
+        words = np.frombuffer(gpu.aes256ctr(key, t, 0, 24 * n), np.uint32).reshape(n, 96)
+        if ((words[:, 50:60] >= bound).sum(axis=1) >= 3).any():
+            keys.append(key)
+            nonces.append(t)
+        if len(keys) == 6:
+            break
+    print(f"[gpu-sampler] S{which}: streams {nonces}", flush=True)
+    assert len(keys) == 6
+    monkeypatch.setenv("CUFE_GAUSS_SCAN", limit)
+    full = gpu.gauss_sample(keys, nonces, which, 1)
+    first = gpu.gauss_sample_first(keys, nonces, which, 1)
+    for t, key in enumerate(keys):
+        assert np.array_equal(full[t], po.gauss_calls(key, nonces[t], which, 1)), nonces[t]
+    assert np.array_equal(first, full[:, :, :, 0])
