@@ -15,7 +15,9 @@
 // One wave per stream walking all its calls in order (5.2 us a call, whatever
 // the number of streams) took 4.07 ms for the 785 calls of one message at the
 // reference's key length, seven times the candidates before it; the three
-// launches take 0.07 ms (the whole call went from 11.1 to 7.2 ms).
+// launches take 0.07 ms (the whole call went from 11.1 to 7.2 ms).  Where every
+// stream fits one window its entry is chunk 0 and the third launch does alone
+// (one call of S1: 4.5 us, 21.5 in three launches).
 #include "kernels.h"
 
 namespace ipfe {
@@ -186,11 +188,13 @@ __global__ void k_walk_chain(const GaussStream *__restrict__ streams, int nstrea
 }
 
 // Full streams: pos[chunk] = call << 13 | first output position, or -1.
-// Compact streams: firsts of the calls that start in the window.
+// Compact streams: firsts of the calls that start in the window.  one: the
+// streams have one window each and no map was made.
 __global__ __launch_bounds__(WALK_THREADS) void k_walk_fill(const GaussStream *__restrict__ streams, int maxw,
                                                              const uint8_t *__restrict__ cnt, int *__restrict__ pos,
                                                              uint32_t *__restrict__ map,
-                                                             long long *__restrict__ firsts)
+                                                             long long *__restrict__ firsts, int one,
+                                                             int *__restrict__ status)
 {
     __shared__ __align__(16) uint16_t P[WALK_WIN + WALK_HALO];
     __shared__ uint32_t wsum[2][8];
@@ -202,8 +206,8 @@ __global__ __launch_bounds__(WALK_THREADS) void k_walk_fill(const GaussStream *_
     const WalkWindow W(S, w, pos, map);
     const bool compact = S->coef0_only != 0;
     const long long base = S->chunk_base + (long long)w * WALK_WIN;
-    const uint32_t entry = W.slot[0], slen = (uint32_t)S->slen;
-    const int k = (int)W.slot[1];
+    const uint32_t entry = one ? 0u : W.slot[0], slen = (uint32_t)S->slen;
+    const int k = one ? 0 : (int)W.slot[1];
     const int npad = (W.nwin + 15) & ~15;  // the plan's padding carries no call
     if (entry & WALK_OPEN) {
         __syncthreads();  // every thread has read the slots
@@ -232,6 +236,7 @@ __global__ __launch_bounds__(WALK_THREADS) void k_walk_fill(const GaussStream *_
         if (lane == 0) {
             start[n] = c;
             s_n = n;
+            if (one && n < ncalls) status[blockIdx.x] = 1;
         }
     }
     __syncthreads();
@@ -281,11 +286,14 @@ int launch_gauss_walk(const GaussStream *d_streams, int nstreams, int max_chunks
         ipfe_set_error("Gaussian walk: %d streams of up to %d chunks", nstreams, max_chunks);
         return -1;
     }
-    hipLaunchKernelGGL(k_walk_map, dim3((unsigned)blocks), dim3(WALK_THREADS), 0, st, d_streams, maxw, cnt, pos, map);
-    hipLaunchKernelGGL(k_walk_chain, dim3((unsigned)((nstreams + 63) / 64)), dim3(64), 0, st, d_streams, nstreams, pos,
-                       map, status);
+    if (maxw > 1) {
+        hipLaunchKernelGGL(k_walk_map, dim3((unsigned)blocks), dim3(WALK_THREADS), 0, st, d_streams, maxw, cnt, pos,
+                           map);
+        hipLaunchKernelGGL(k_walk_chain, dim3((unsigned)((nstreams + 63) / 64)), dim3(64), 0, st, d_streams, nstreams,
+                           pos, map, status);
+    }
     hipLaunchKernelGGL(k_walk_fill, dim3((unsigned)blocks), dim3(WALK_THREADS), 0, st, d_streams, maxw, cnt, pos, map,
-                       firsts);
+                       firsts, maxw == 1, status);
     HIP_OK(hipGetLastError());
     return 0;
 }
