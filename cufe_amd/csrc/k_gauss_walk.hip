@@ -282,7 +282,9 @@ int launch_gauss_walk(const GaussStream *d_streams, int nstreams, int max_chunks
     if (nstreams <= 0) return 0;
     const int maxw = (max_chunks + WALK_WIN - 1) / WALK_WIN;
     const long long blocks = (long long)nstreams * maxw;
-    if (maxw < 1 || blocks > 0x7fffffffll) {
+    // a launch takes fewer than 2^32 threads (a group of 2^28 chunks at most, with
+    // streams of up to 65 windows beside the shortest: half of that)
+    if (maxw < 1 || blocks >= (1ll << 32) / WALK_THREADS) {
         ipfe_set_error("Gaussian walk: %d streams of up to %d chunks", nstreams, max_chunks);
         return -1;
     }

@@ -274,8 +274,6 @@ int GaussPlan::bind_scratch_region(uint8_t *base)
     return bind_scratch(cnt, vals, (int *)base);
 }
 
-size_t GaussPlan::scratch_bytes() const { return (size_t)chunks + (size_t)full_chunks * (64 + 4) + 64; }
-
 int GaussPlan::bind_scratch(uint8_t *cnt, uint64_t *vals, int *pos)
 {
     s_cnt = cnt;

@@ -154,9 +154,8 @@ struct GaussPlan {
     // the chunk scratch as one region of 256-byte aligned pieces
     size_t bound_scratch_bytes() const;
     int bind_scratch_region(uint8_t *base);
-    // chunk scratch: own allocation, or a caller's buffer of scratch_bytes()
-    // (chunks counts, then 8 values and 1 position per full-stream chunk)
-    size_t scratch_bytes() const;
+    // chunk scratch: own allocation, or a caller's buffers (a count per chunk;
+    // 8 values and a position per full-stream chunk)
     int alloc_scratch();
     int bind_scratch(uint8_t *cnt, uint64_t *vals, int *pos);
     void rekey(const StreamReq *reqs);
