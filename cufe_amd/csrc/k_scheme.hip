@@ -60,7 +60,8 @@ __global__ __launch_bounds__(64 * FOLD_WAVES) void k_fold_few(SparseY y, const u
 }
 
 // Many sparse vectors: four consecutive coefficients a thread, 16-byte loads
-// (2,000 vectors of 14 entries: 267 -> 80 us, 98 MB written).
+// (2,000 vectors of 14 entries: 267 -> 76 us, bound by the 1.4 GB of key words
+// that they read from the caches, at 18 TB/s).
 // Grid (3 N / 1024, nvec).
 __global__ __launch_bounds__(256) void k_fold_many(SparseY y, const uint32_t *__restrict__ P,
                                                    uint32_t *__restrict__ out, BarrettConsts bc)

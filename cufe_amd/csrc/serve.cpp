@@ -175,7 +175,8 @@ int launch_batch(cufe_server *s, Slot &sl)
     // copied by DMA directly; others are first copied into the slot's pinned
     // staging.  So is c0 of up to kStageC0 bytes, and the staged c0 goes up in one
     // transfer a run: a transfer of a few KB is 7 us on the stream and as much to
-    // issue, the copy of 128 KiB 5.
+    // issue, the copy of 128 KiB 5 from the caches (24 requests of 1 to 64 rows:
+    // 1,252 -> 1,156 us a burst; from buffers not touched before 1,310 -> 1,170).
     constexpr size_t kStageC0 = (size_t)128 << 10;
     uint32_t *h_c0 = sl.h_stage + (size_t)s->cap * kPoly;
     uint32_t *d_c0 = sl.d_stage.get() + (size_t)s->cap * kPoly;

@@ -25,15 +25,15 @@
 // instead, a few threads each copying a chunk to or from the caller while the
 // others' chunks cross the link: the reference's 38.6 MB keys 2.2 -> 0.95 ms out,
 // 1.35 -> 0.9 in (a whole key generation).  Waking the threads, filling and
-// draining their chunks costs a small copy some 0.06 ms, so it gains less: out 16.8 MB 0.97 -> 0.47 ms,
-// 8.4 MB 0.49 -> 0.31, 6.3 MB 0.37 -> 0.27, 4.2 MB level, and from kStageDown bytes on
-// they take them.  In, a key generation over 4.2, 6.3, 8.4, 12.6 and 16.8 MB
-// takes 181, 228, 293, 395 and 510 us with the runtime's copy where the caches hold the
-// source, 226, 295, 380, 522 and 678 where they do not, and 245, 270, 305, 400 and
-// 465 (280, 312, 357, 434 and 537) with the threads: from kStageUp on, except
-// beside a stream's work, where the runtime's copy would wait for it.  Six
-// threads and eight give the same, more than eight are slower; chunks of 1 MiB
-// load at 30 GB/s.
+// draining their chunks costs a small copy some 0.06 ms, so it gains less: out
+// 16.8 MB 0.97 -> 0.47 ms, 8.4 MB 0.49 -> 0.31, 6.3 MB 0.37 -> 0.27, 4.2 MB level,
+// and from kStageDown bytes on they take them.  In, a key generation over 4.2,
+// 6.3, 8.4, 12.6 and 16.8 MB takes 181, 228, 293, 395 and 510 us with the runtime's
+// copy where the caches hold the source, 226, 295, 380, 522 and 678 where they do
+// not, and 245, 270, 305, 400 and 465 (280, 312, 357, 434 and 537) with the threads:
+// from kStageUp on, except beside a stream's work, where the runtime's copy
+// would wait for it.  Six threads and eight give the same, more than eight are
+// slower; chunks of 1 MiB load at 30 GB/s.
 #include <hip/hip_runtime.h>
 #include <sched.h>
 #include <stdint.h>
